@@ -1,4 +1,7 @@
-// Token sampler: temperature -> top-k -> top-p -> draw, one workgroup per row.
+// Token sampler: temperature -> top-k -> top-p -> draw. Long rows (a language
+// model's vocabulary) are split over kSplitG workgroups in four launches
+// (sample_*_kernel below); short rows, calls without a workspace and the few
+// rows the split form hands over run as one workgroup per row (sample_row).
 //
 // Semantics follow acorninfer/sampler.py:38-68 (HF warper order):
 //   x = logits / T                                   (fp32)
@@ -11,7 +14,7 @@
 // temperature == 0 means greedy (argmax, logprob 0), as Executor._sample
 // routes it (engine/executor.py:128-138).
 //
-// Design: the row is never sorted. Keys are the order-preserving uint32 image
+// One workgroup per row: the row is never sorted. Keys are the order-preserving uint32 image
 // of fp32. top-k is a 4-pass radix select (8-bit digits, MSB first) with
 // count histograms; top-p is the same descent over the softmax mass, with
 // masses accumulated as 2^-40 fixed-point integers so that the LDS atomics
@@ -109,12 +112,101 @@ __device__ uint32_t block_exclusive_scan_u32(uint32_t v, uint32_t* buf, uint32_t
   return incl - v;
 }
 
+// This thread's share of a scan of p[0, n): its maximum `bv` (first index `bi`
+// on ties) and whether it saw a NaN or an infinity. 16-byte vectors, kUnroll
+// of them in flight per thread (for one workgroup a 151936-entry bf16 row is
+// two rounds of requests); a scalar tail. Vector indices past the end re-read
+// the last vector (unconditional loads keep the wait counts static) and are
+// not visited.
+// The per-element work is what bounds a workgroup that reads a whole row: per
+// vector only its maximum is compared with the running one (the vector index
+// of the first strict improvement is kept) and the exponent fields are folded
+// into an integer max for the finiteness test. After the loop the kept vector
+// is read again and its first element equal to the maximum taken: the
+// thread's first maximum in index order, as an element-by-element scan would
+// find.
+template <typename T, int NT, int kUnroll>
+__device__ __forceinline__ void scan_max(const T* p, int64_t n, float& bv, int64_t& bi,
+                                         bool& bad) {
+  const int tid = threadIdx.x;
+  bv = -INFINITY;
+  bi = INT64_MAX;
+  bad = false;
+  auto visit = [&](float l, int64_t i) {
+    if (!(l == l) || l == INFINITY || l == -INFINITY) bad = true;
+    if (l > bv || (l == bv && i < bi)) {
+      bv = l;
+      bi = i;
+    }
+  };
+  constexpr int E = 16 / sizeof(T);                 // elements per vector
+  const bool aligned = ((uintptr_t)p % 16) == 0;
+  const int64_t nvec = aligned ? n / E : 0;
+  const u32x4v* rv = (const u32x4v*)p;
+  float vbest = -INFINITY;
+  int64_t jbest = -1;
+  uint32_t emax = 0;
+  for (int64_t j0 = tid; j0 < nvec; j0 += (int64_t)NT * kUnroll) {
+    u32x4v buf[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) buf[u] = rv[min(j0 + (int64_t)u * NT, nvec - 1)];
+    // (the empty asm keeps every load ahead of the guarded uses below;
+    // a load sunk into a guarded block is waited for on its own)
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) asm volatile("" ::"v"(buf[u]));
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int64_t j = j0 + (int64_t)u * NT;
+      if (j < nvec) {
+        float vm = word_elem<T>(buf[u], 0);
+#pragma unroll
+        for (int e = 1; e < E; ++e) vm = fmaxf(vm, word_elem<T>(buf[u], e));
+        emax = fold_exp<T>(emax, buf[u]);
+        if (vm > vbest) {
+          vbest = vm;
+          jbest = j;
+        }
+      }
+    }
+  }
+  if (exp_all_ones<T>(emax)) bad = true;
+  if (jbest >= 0) {
+    const u32x4v w = rv[jbest];
+    int ebest = E - 1;
+#pragma unroll
+    for (int e = E - 2; e >= 0; --e) ebest = word_elem<T>(w, e) == vbest ? e : ebest;
+    bv = vbest;
+    bi = jbest * E + ebest;
+  }
+  for (int64_t i = nvec * E + tid; i < n; i += NT) visit(to_f32(p[i]), i);
+}
+
+// The wave's first maximum in every lane.
+__device__ __forceinline__ void wave_first_max(float& bv, int64_t& bi) {
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    const float ov = __shfl_xor(bv, o);
+    const int64_t oi = __shfl_xor(bi, o);
+    if (ov > bv || (ov == bv && oi < bi)) {
+      bv = ov;
+      bi = oi;
+    }
+  }
+}
+
+// exp(x - M) as 2^-40 fixed point (sums of it do not depend on their order).
+__device__ __forceinline__ unsigned long long mass_fix(float x, float M) {
+  return (unsigned long long)((double)exp2f((x - M) * 1.4426950408889634f) * kFix);
+}
+
+// One row on one workgroup of kNT threads.
 template <typename T>
-__global__ __launch_bounds__(kNT) void sample_kernel(
-    const T* __restrict__ logits, int64_t V, const float* __restrict__ temperature,
-    const int32_t* __restrict__ top_k, const float* __restrict__ top_p,
-    const float* __restrict__ uniform, int64_t* __restrict__ token, float* __restrict__ logprob,
-    float* __restrict__ processed, int32_t* __restrict__ status) {
+__device__ void sample_row(
+    const int64_t r, const T* __restrict__ logits, int64_t V,
+    const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
+    const float* __restrict__ top_p, const float* __restrict__ uniform,
+    int64_t* __restrict__ token, float* __restrict__ logprob, float* __restrict__ processed,
+    int32_t* __restrict__ status) {
   __shared__ uint32_t hcnt[256];
   __shared__ unsigned long long hmass[256];
   __shared__ float sbuf[kNT];
@@ -126,7 +218,6 @@ __global__ __launch_bounds__(kNT) void sample_kernel(
   __shared__ float sh_f[4];
   __shared__ int sh_bad;
 
-  const int64_t r = blockIdx.x;
   const T* row = logits + r * V;
   const float Tm = temperature[r];
   const int tid = threadIdx.x, lane = tid % kWave, wid = tid / kWave;
@@ -134,80 +225,12 @@ __global__ __launch_bounds__(kNT) void sample_kernel(
   __syncthreads();
 
   // ---- pass 1: max (first index on ties), finiteness --------------------
-  // 16-byte vectors, kUnroll of them in flight per thread (a 151936-entry
-  // bf16 row is two rounds of requests); a scalar tail. Vector indices past
-  // the row re-read its last vector (unconditional loads keep the wait
-  // counts static) and are not visited.
-  // A single workgroup reads the whole row, so the per-element work is what
-  // bounds it: per vector only its maximum is compared with the running one
-  // (the vector index of the first strict improvement is kept) and the
-  // exponent fields are folded into an integer max for the finiteness test.
-  // After the loop the kept vector is read again and its first element equal
-  // to the maximum taken: the thread's first maximum in index order, as an
-  // element-by-element scan would find.
-  float bv = -INFINITY;
-  int64_t bi = INT64_MAX;
-  bool bad = false;
-  auto visit = [&](float l, int64_t i) {
-    if (!(l == l) || l == INFINITY || l == -INFINITY) bad = true;
-    if (l > bv || (l == bv && i < bi)) {
-      bv = l;
-      bi = i;
-    }
-  };
-  {
-    constexpr int E = 16 / sizeof(T);                 // elements per vector
-    constexpr int kUnroll = 10;
-    const bool aligned = ((uintptr_t)row % 16) == 0;
-    const int64_t nvec = aligned ? V / E : 0;
-    const u32x4v* rv = (const u32x4v*)row;
-    float vbest = -INFINITY;
-    int64_t jbest = -1;
-    uint32_t emax = 0;
-    for (int64_t j0 = tid; j0 < nvec; j0 += (int64_t)kNT * kUnroll) {
-      u32x4v buf[kUnroll];
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) buf[u] = rv[min(j0 + (int64_t)u * kNT, nvec - 1)];
-      // (the empty asm keeps every load ahead of the guarded uses below;
-      // a load sunk into a guarded block is waited for on its own)
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) asm volatile("" ::"v"(buf[u]));
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const int64_t j = j0 + (int64_t)u * kNT;
-        if (j < nvec) {
-          float vm = word_elem<T>(buf[u], 0);
-#pragma unroll
-          for (int e = 1; e < E; ++e) vm = fmaxf(vm, word_elem<T>(buf[u], e));
-          emax = fold_exp<T>(emax, buf[u]);
-          if (vm > vbest) {
-            vbest = vm;
-            jbest = j;
-          }
-        }
-      }
-    }
-    if (exp_all_ones<T>(emax)) bad = true;
-    if (jbest >= 0) {
-      const u32x4v w = rv[jbest];
-      int ebest = E - 1;
-#pragma unroll
-      for (int e = E - 2; e >= 0; --e) ebest = word_elem<T>(w, e) == vbest ? e : ebest;
-      bv = vbest;
-      bi = jbest * E + ebest;
-    }
-    for (int64_t i = nvec * E + tid; i < V; i += kNT) visit(to_f32(row[i]), i);
-  }
+  float bv;
+  int64_t bi;
+  bool bad;
+  scan_max<T, kNT, 10>(row, V, bv, bi, bad);
   if (bad) sh_bad = 1;  // benign race: every writer stores 1
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o);
-    const int64_t oi = __shfl_xor(bi, o);
-    if (ov > bv || (ov == bv && oi < bi)) {
-      bv = ov;
-      bi = oi;
-    }
-  }
+  wave_first_max(bv, bi);
   if (lane == 0) {
     red_f[wid] = bv;
     red_i[wid] = bi;
@@ -280,9 +303,7 @@ __global__ __launch_bounds__(kNT) void sample_kernel(
 
   // ---- mass of the top-k set: Z = sum exp(x - M) over key >= kkey ---------
   // (fixed-point, order independent)
-  auto wfix = [&](float x) -> unsigned long long {
-    return (unsigned long long)((double)exp2f((x - M) * 1.4426950408889634f) * kFix);
-  };
+  auto wfix = [&](float x) { return mass_fix(x, M); };
   unsigned long long zl = 0;
   for (int64_t i = tid; i < V; i += kNT) {
     const float x = to_f32(row[i]) / Tm;
@@ -461,7 +482,584 @@ __global__ __launch_bounds__(kNT) void sample_kernel(
   }
 }
 
+// ---- long rows: kSplitG workgroups per row --------------------------------
+//
+// One workgroup per row leaves all but `rows` CUs idle and walks the row about
+// ten times, an IEEE division and often an LDS atomic per element each time:
+// 444 us for 8 rows of 151936 (2.4 MB) at T 0.6, top-k 20, top-p 0.95. Here a
+// row is kSplitG chunks of consecutive elements and each launch reads a chunk
+// once:
+//   stats   chunk maxima and finiteness; clears the row's histogram
+//   hist    histogram of the row over kSplitNB bins of 1/64 in x = logit / T
+//           below the maximum: counts (top-k) or fixed-point mass (top-p);
+//           with neither, the chunk's mass. Greedy and non-finite rows end here
+//   gather  the boundary bin, from the histogram; the elements that may lie on
+//           the boundary (top-k: all down to the boundary bin; top-p: those
+//           in it) listed per chunk in vocabulary order, and the chunk's mass
+//           above it
+//   pick    one workgroup per row ranks the listed elements by counting, which
+//           gives the kept set, finds the drawn chunk from the chunks' masses
+//           and the token inside it
+// The selection is sample_row's, bit for bit: the same keys and the same
+// integer masses relative to the row's maximum. A bin is a monotone function
+// of x, so bins respect the key order. The draw adds integer masses instead of
+// fp32 ones. Rows whose boundary holds more elements than the lists (a large
+// top-k, many ties) or whose maximum overflows are left to sample_row.
+// Four launches of a few microseconds each, bound by their latency.
+constexpr int kSplitG = 32;          // workgroups (chunks) per row
+constexpr int kSplitNT = 256;        // their threads
+constexpr int kSplitNB = 2048;       // histogram bins: 32 in x, the last takes the rest
+constexpr float kSplitScale = 64.f;  // bins per unit of x
+constexpr int kSplitCapC = 64;       // listed elements per chunk (one wave)
+constexpr int kSplitCap = kNT;       // listed elements per row (one per thread of `pick`)
+// shorter rows: one workgroup reads them in less than four launches take
+constexpr int64_t kSplitMinV = 16384;
+constexpr int64_t kSplitMaxRows = 4096;  // bounds the workspace (34 KB per row)
+
+enum { kRowDrawn = 0, kRowBad = 1, kRowGreedy = 2, kRowWhole = 3 };
+enum { kModeTopK = 0, kModeTopP = 1, kModeAll = 2 };
+
+struct alignas(64) SplitRow {
+  unsigned long long hist[kSplitNB];  // counts (top-k) or masses (top-p)
+  uint32_t ckey[kSplitG * kSplitCapC];
+  uint32_t cidx[kSplitG * kSplitCapC];
+  unsigned long long hard[kSplitG];   // mass of the chunk's elements above the boundary bin
+  float cmax[kSplitG];
+  uint32_t cimax[kSplitG];
+  uint32_t cbad[kSplitG];
+  uint32_t ccnt[kSplitG];             // elements on the boundary (listed up to kSplitCapC)
+  unsigned long long zk, above;       // top-p: the row's mass, and that above the boundary bin
+  uint32_t state, pkey, tie0;         // kept: key > pkey, or key == pkey and index >= tie0
+};
+
+struct SplitArgs {
+  const void* logits;
+  int64_t V;
+  const float* temperature;
+  const int32_t* top_k;
+  const float* top_p;
+  const float* uniform;
+  int64_t* token;
+  float* logprob;
+  float* processed;
+  int32_t* status;
+  SplitRow* ws;
+};
+
+__device__ __forceinline__ int64_t split_chunk(int64_t V) {
+  return ((V + kSplitG - 1) / kSplitG + 7) & ~(int64_t)7;
+}
+__device__ __forceinline__ int split_mode(const SplitArgs& a, int64_t r) {
+  const int64_t kk = a.top_k[r];
+  if (kk > 0 && kk < a.V) return kModeTopK;
+  return a.top_p[r] < 1.0f ? kModeTopP : kModeAll;
+}
+__device__ __forceinline__ int split_bin(float x, float M) {
+  return (int)fminf((M - x) * kSplitScale, (float)(kSplitNB - 1));
+}
+__device__ __forceinline__ float key_float(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? k & 0x7fffffffu : ~k);
+}
+
+// The row's maximum (first index) and finiteness from its chunks', in every lane.
+__device__ __forceinline__ bool split_stats(const SplitRow& w, float& lmax, int64_t& imax) {
+  const int c = threadIdx.x % kSplitG;
+  lmax = w.cmax[c];
+  imax = w.cimax[c] == 0xffffffffu ? INT64_MAX : (int64_t)w.cimax[c];
+  const bool bad = __any(w.cbad[c] != 0);
+  wave_first_max(lmax, imax);
+  return bad;
+}
+
+// Elements i .. i + 7 of a row as floats (clamped to end - 1).
+template <typename T>
+__device__ __forceinline__ void load8(const T* row, int64_t i, int64_t end, bool aligned,
+                                      float (&v)[8]) {
+  if (aligned && i + 8 <= end) {
+    constexpr int E = 16 / sizeof(T);
+    u32x4v w[8 / E];
+#pragma unroll
+    for (int q = 0; q < 8 / E; ++q) w[q] = ((const u32x4v*)(row + i))[q];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = word_elem<T>(w[e / E], e % E);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = to_f32(row[min(i + e, end - 1)]);
+  }
+}
+
+// Inclusive scan over the wave.
+template <typename V>
+__device__ __forceinline__ V wave_scan(V v) {
+  const int lane = threadIdx.x % kWave;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const V u = __shfl_up(v, o);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
+// Exclusive scan over NT threads; `part` holds NT / 64 values of LDS.
+template <typename V, int NT>
+__device__ __forceinline__ V block_scan(V v, V* part, V& total) {
+  const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
+  const V incl = wave_scan(v);
+  __syncthreads();                       // part's last readers are done
+  if (lane == kWave - 1) part[wid] = incl;
+  __syncthreads();
+  V before = 0;
+  total = 0;
+#pragma unroll
+  for (int w = 0; w < NT / kWave; ++w) {
+    if (w < wid) before += part[w];
+    total += part[w];
+  }
+  return before + incl - v;
+}
+
+template <typename T>
+__global__ __launch_bounds__(kSplitNT) void sample_stats_kernel(SplitArgs a) {
+  __shared__ float red_f[kSplitNT / kWave];
+  __shared__ int64_t red_i[kSplitNT / kWave];
+  __shared__ int red_b[kSplitNT / kWave];
+  const int64_t r = blockIdx.x / kSplitG;
+  const int c = blockIdx.x % kSplitG, tid = threadIdx.x;
+  SplitRow& w = a.ws[r];
+  constexpr int kShare = kSplitNB / kSplitG;
+  if (tid < kShare) w.hist[c * kShare + tid] = 0;
+  const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
+  float bv;
+  int64_t bi;
+  bool bad;
+  scan_max<T, kSplitNT, 3>((const T*)a.logits + r * a.V + c0, c1 - c0, bv, bi, bad);
+  if (bi != INT64_MAX) bi += c0;
+  wave_first_max(bv, bi);
+  bad = __any(bad);
+  if (tid % kWave == 0) {
+    red_f[tid / kWave] = bv;
+    red_i[tid / kWave] = bi;
+    red_b[tid / kWave] = bad;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    for (int q = 1; q < kSplitNT / kWave; ++q) {
+      if (red_f[q] > bv || (red_f[q] == bv && red_i[q] < bi)) {
+        bv = red_f[q];
+        bi = red_i[q];
+      }
+      bad |= red_b[q] != 0;
+    }
+    w.cmax[c] = bv;
+    w.cimax[c] = bi == INT64_MAX ? 0xffffffffu : (uint32_t)bi;
+    w.cbad[c] = bad;
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
+  __shared__ unsigned long long lhist[kSplitNB];
+  __shared__ unsigned long long part[kSplitNT / kWave];
+  const int64_t r = blockIdx.x / kSplitG;
+  const int c = blockIdx.x % kSplitG, tid = threadIdx.x;
+  SplitRow& w = a.ws[r];
+  float lmax;
+  int64_t imax;
+  const bool bad = split_stats(w, lmax, imax);
+  const float Tm = a.temperature[r];
+  const float M = lmax / Tm;
+  if (bad || !(Tm > 0.f) || !(fabsf(M) < INFINITY)) {
+    if (c == 0 && tid == 0) {
+      if (bad) {
+        a.status[r] = 1;
+        a.token[r] = imax == INT64_MAX ? 0 : imax;
+        a.logprob[r] = NAN;
+      } else if (!(Tm > 0.f)) {
+        a.status[r] = 0;
+        a.token[r] = imax;
+        a.logprob[r] = 0.f;
+      }
+      w.state = bad ? kRowBad : !(Tm > 0.f) ? kRowGreedy : kRowWhole;
+    }
+    return;
+  }
+  const int mode = split_mode(a, r);
+  const T* row = (const T*)a.logits + r * a.V;
+  const bool aligned = ((uintptr_t)row % 16) == 0;
+  const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
+  for (int b = tid; b < kSplitNB; b += kSplitNT) lhist[b] = 0;
+  __syncthreads();
+  unsigned long long sum = 0;
+  for (int64_t i = c0 + tid * 8; i < c1; i += kSplitNT * 8) {
+    float v[8];
+    load8(row, i, c1, aligned, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if (i + e >= c1) continue;
+      const float x = v[e] / Tm;
+      if (mode == kModeTopK)
+        atomicAdd(&lhist[split_bin(x, M)], 1ull);
+      else if (mode == kModeTopP)
+        atomicAdd(&lhist[split_bin(x, M)], mass_fix(x, M));
+      else
+        sum += mass_fix(x, M);
+    }
+  }
+  if (mode == kModeAll) {
+    unsigned long long total;
+    block_scan<unsigned long long, kSplitNT>(sum, part, total);
+    if (tid == 0) w.hard[c] = total;
+    return;
+  }
+  __syncthreads();
+  for (int b = tid; b < kSplitNB; b += kSplitNT)
+    if (lhist[b]) atomicAdd(&w.hist[b], lhist[b]);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
+  __shared__ unsigned long long part[kSplitNT / kWave];
+  __shared__ uint32_t upart[kSplitNT / kWave];
+  __shared__ int sh_bin;
+  __shared__ unsigned long long sh_above;
+  const int64_t r = blockIdx.x / kSplitG;
+  const int c = blockIdx.x % kSplitG, tid = threadIdx.x;
+  SplitRow& w = a.ws[r];
+  float lmax;
+  int64_t imax;
+  const bool bad = split_stats(w, lmax, imax);
+  const float Tm = a.temperature[r];
+  const float M = lmax / Tm;
+  const int mode = split_mode(a, r);
+  if (bad || !(Tm > 0.f) || !(fabsf(M) < INFINITY) || mode == kModeAll) return;
+
+  // the first bin (from the maximum down) at which the running count reaches
+  // k, or the running mass the target
+  constexpr int kPer = kSplitNB / kSplitNT;
+  unsigned long long h[kPer], mine = 0, total;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) h[q] = w.hist[tid * kPer + q];
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) mine += h[q];
+  unsigned long long run = block_scan<unsigned long long, kSplitNT>(mine, part, total);
+  const unsigned long long goal =
+      mode == kModeTopK
+          ? (unsigned long long)a.top_k[r]
+          : max(1ull, (unsigned long long)(fmax((double)a.top_p[r], 0.0) * (double)total));
+  if (run < goal && goal <= run + mine) {
+    bool found = false;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      if (!found && goal <= run + h[q]) {
+        found = true;
+        sh_bin = tid * kPer + q;
+        sh_above = run;
+      }
+      run += h[q];
+    }
+  }
+  __syncthreads();
+  const int bin = sh_bin;
+
+  const T* row = (const T*)a.logits + r * a.V;
+  const bool aligned = ((uintptr_t)row % 16) == 0;
+  const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
+  unsigned long long hard = 0;
+  uint32_t listed = 0;
+  for (int64_t t0 = c0; t0 < c1; t0 += kSplitNT * 8) {
+    const int64_t i = t0 + tid * 8;
+    float x[8];
+    uint32_t sel = 0;
+    if (i < c1) {
+      load8(row, i, c1, aligned, x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        x[e] = x[e] / Tm;
+        if (i + e >= c1) continue;
+        const int b = split_bin(x[e], M);
+        if (b == bin || (mode == kModeTopK && b < bin))
+          sel |= 1u << e;
+        else if (b < bin)
+          hard += mass_fix(x[e], M);
+      }
+    }
+    uint32_t tile;
+    uint32_t pos =
+        listed + block_scan<uint32_t, kSplitNT>((uint32_t)__popc(sel), upart, tile);
+    listed += tile;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (sel >> e & 1) {
+        if (pos < (uint32_t)kSplitCapC) {
+          w.ckey[c * kSplitCapC + pos] = okey(x[e]);
+          w.cidx[c * kSplitCapC + pos] = (uint32_t)(i + e);
+        }
+        ++pos;
+      }
+  }
+  unsigned long long hsum;
+  block_scan<unsigned long long, kSplitNT>(hard, part, hsum);
+  if (tid == 0) {
+    w.hard[c] = hsum;
+    w.ccnt[c] = listed;
+    if (c == 0) {
+      w.zk = total;
+      w.above = sh_above;
+    }
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kNT) void sample_pick_kernel(SplitArgs a) {
+  __shared__ uint32_t skey[kSplitCap], sidx[kSplitCap];
+  __shared__ unsigned long long sw[kSplitCap];
+  __shared__ unsigned long long part[kNT / kWave];
+  __shared__ unsigned long long cm[kSplitG];          // kept mass per chunk
+  __shared__ uint32_t off[kSplitG + 1];
+  __shared__ unsigned long long sh_zk, sh_low, sh_z, sh_rem;
+  __shared__ int sh_over, sh_chunk;
+  const int64_t r = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid % kWave;
+  SplitRow& w = a.ws[r];
+  float lmax;
+  int64_t imax;
+  const bool bad = split_stats(w, lmax, imax);
+  const float Tm = a.temperature[r];
+  const float M = lmax / Tm;
+  if (bad || !(Tm > 0.f)) return;                     // written by `hist`
+  const int mode = split_mode(a, r);
+  const int64_t kk = a.top_k[r];
+  const float pp = a.top_p[r];
+  const int64_t chunk = split_chunk(a.V);
+  const bool whole = !(fabsf(M) < INFINITY);
+
+  if (tid < kWave) {                                  // wave 0: the lists' offsets
+    const uint32_t n = lane < kSplitG && mode != kModeAll && !whole ? w.ccnt[lane] : 0u;
+    const bool over = __any(n > (uint32_t)kSplitCapC);
+    const uint32_t incl = wave_scan(n);
+    if (lane < kSplitG) {
+      off[lane + 1] = incl;
+      cm[lane] = mode == kModeTopK ? 0 : w.hard[lane];
+    }
+    if (lane == 0) {
+      off[0] = 0;
+      sh_zk = 0;
+      sh_low = ~0ull;
+    }
+    if (lane == kSplitG - 1) sh_over = over || incl > (uint32_t)kSplitCap;
+  }
+  __syncthreads();
+  if (whole || sh_over) {                             // (uniform over the workgroup)
+    if (tid == 0) w.state = kRowWhole;
+    sample_row<T>(r, (const T*)a.logits, a.V, a.temperature, a.top_k, a.top_p, a.uniform,
+                  a.token, a.logprob, a.processed, a.status);
+    return;
+  }
+  const int n = (int)off[kSplitG];
+  for (int s = tid; s < kSplitG * kSplitCapC; s += kNT) {
+    const int c = s / kSplitCapC, j = s % kSplitCapC;
+    if (j < (int)(off[c + 1] - off[c])) {
+      skey[off[c] + j] = w.ckey[s];
+      sidx[off[c] + j] = w.cidx[s];
+    }
+  }
+  __syncthreads();
+  uint32_t key = 0, idx = 0;
+  unsigned long long m = 0;
+  if (tid < n) {
+    key = skey[tid];
+    idx = sidx[tid];
+    m = mass_fix(key_float(key), M);
+    sw[tid] = m;
+  }
+  __syncthreads();
+  // rank by counting: elements above mine, their mass, ties and those after me
+  uint32_t higher = 0, ties = 0, after = 0;
+  unsigned long long above = 0;
+  if ((tid & ~(kWave - 1)) < n) {
+    for (int j = 0; j < n; ++j) {
+      const uint32_t kj = skey[j];
+      const unsigned long long mj = sw[j];
+      if (kj > key) {
+        ++higher;
+        above += mj;
+      }
+      if (kj == key) {
+        ++ties;
+        after += j > tid;
+      }
+    }
+  }
+  bool keep = tid < n && (mode != kModeTopK || (int64_t)higher < kk);
+  if (mode == kModeTopK && keep) atomicAdd(&sh_zk, m);
+  __syncthreads();
+  if (pp < 1.0f && mode != kModeAll) {
+    const unsigned long long zk = mode == kModeTopK ? sh_zk : w.zk;
+    if (mode == kModeTopP) above += w.above;
+    const unsigned long long target =
+        max(1ull, (unsigned long long)(fmax((double)pp, 0.0) * (double)zk));
+    // a group of equal values is kept while the mass above it is below the
+    // target; of the last one, as many as reach it, from the highest index down
+    keep = keep && above < target;
+    if (keep && m > 0) {
+      const double need = ceil(((double)target - (double)above) / (double)m);
+      keep = (double)after < fmax(1.0, fmin(need, (double)ties));
+    }
+  }
+  if (keep) {
+    atomicAdd(&cm[idx / (uint32_t)chunk], m);
+    atomicMin(&sh_low, ((unsigned long long)key << 32) | idx);
+  }
+  if (tid < n) sw[tid] = keep ? m : 0;
+  __syncthreads();
+  const uint32_t pkey = mode == kModeAll ? 0u : (uint32_t)(sh_low >> 32);
+  const uint32_t tie0 = mode == kModeAll ? 0u : (uint32_t)sh_low;
+  if (tid < kWave) {                                  // wave 0: the drawn chunk
+    const unsigned long long mc = lane < kSplitG ? cm[lane] : 0;
+    const unsigned long long incl = wave_scan(mc);
+    const unsigned long long Z = __shfl(incl, kWave - 1);
+    const unsigned long long t = min(
+        (unsigned long long)(fmax((double)a.uniform[r], 0.0) * (double)Z), Z - 1);
+    const int c = __ffsll((unsigned long long)__ballot(incl > t)) - 1;
+    if (lane == c) {
+      sh_chunk = c;
+      sh_rem = t - (incl - mc);
+    }
+    if (lane == 0) {
+      sh_z = Z;
+      w.state = kRowDrawn;
+      w.pkey = pkey;
+      w.tie0 = tie0;
+    }
+  }
+  __syncthreads();
+  const int c = sh_chunk;
+  const unsigned long long rem = sh_rem;
+  auto draw = [&](int64_t i, float x) {
+    a.token[r] = i;
+    a.logprob[r] = (x - M) - logf((float)((double)sh_z / kFix));
+    a.status[r] = 0;
+  };
+  if (mode == kModeTopK) {                            // inside the chunk's list
+    if (tid >= kWave) return;
+    const int j = (int)off[c] + lane;
+    const unsigned long long mj = j < (int)off[c + 1] ? sw[j] : 0;
+    const int pick = __ffsll((unsigned long long)__ballot(wave_scan(mj) > rem)) - 1;
+    if (lane == pick) draw(sidx[j], key_float(skey[j]));
+    return;
+  }
+  const T* row = (const T*)a.logits + r * a.V;
+  const bool aligned = ((uintptr_t)row % 16) == 0;
+  const int64_t c0 = min(c * chunk, a.V), c1 = min(c0 + chunk, a.V);
+  unsigned long long base = 0;
+  for (int64_t t0 = c0; t0 < c1 && base <= rem; t0 += kNT * 8) {
+    const int64_t i = t0 + tid * 8;
+    float x[8];
+    unsigned long long me[8], mine = 0, total;
+    if (i < c1) load8(row, i, c1, aligned, x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      me[e] = 0;
+      if (i + e < c1) {
+        x[e] = x[e] / Tm;
+        const uint32_t k = okey(x[e]);
+        if (k > pkey || (k == pkey && (uint64_t)(i + e) >= tie0)) me[e] = mass_fix(x[e], M);
+      }
+      mine += me[e];
+    }
+    unsigned long long run = base + block_scan<unsigned long long, kNT>(mine, part, total);
+    if (run <= rem && rem < run + mine) {
+      bool found = false;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        run += me[e];
+        if (!found && rem < run) {
+          found = true;
+          draw(i + e, x[e]);
+        }
+      }
+    }
+    base += total;
+  }
+}
+
+// The processed logits of the rows the split form drew (and of greedy ones).
+template <typename T>
+__global__ __launch_bounds__(kSplitNT) void sample_processed_kernel(SplitArgs a) {
+  const int64_t r = blockIdx.x / kSplitG;
+  const int c = blockIdx.x % kSplitG;
+  const SplitRow& w = a.ws[r];
+  const uint32_t state = w.state;
+  if (state != kRowDrawn && state != kRowGreedy) return;
+  const float Tm = a.temperature[r];
+  const uint32_t pkey = w.pkey, tie0 = w.tie0;
+  const T* row = (const T*)a.logits + r * a.V;
+  const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
+  for (int64_t i = c0 + threadIdx.x; i < c1; i += kSplitNT) {
+    const float l = to_f32(row[i]);
+    const float x = l / Tm;
+    const uint32_t k = okey(x);
+    a.processed[r * a.V + i] =
+        state == kRowGreedy ? l
+                            : (k > pkey || (k == pkey && (uint64_t)i >= tie0)) ? x : -INFINITY;
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kNT) void sample_kernel(
+    const T* __restrict__ logits, int64_t V, const float* __restrict__ temperature,
+    const int32_t* __restrict__ top_k, const float* __restrict__ top_p,
+    const float* __restrict__ uniform, int64_t* __restrict__ token, float* __restrict__ logprob,
+    float* __restrict__ processed, int32_t* __restrict__ status) {
+  sample_row<T>(blockIdx.x, logits, V, temperature, top_k, top_p, uniform, token, logprob,
+                processed, status);
+}
+
+template <typename T>
+void launch_split(const SplitArgs& a, int64_t rows, hipStream_t st) {
+  const dim3 grid((unsigned)(rows * kSplitG));
+  sample_stats_kernel<T><<<grid, kSplitNT, 0, st>>>(a);
+  sample_hist_kernel<T><<<grid, kSplitNT, 0, st>>>(a);
+  sample_gather_kernel<T><<<grid, kSplitNT, 0, st>>>(a);
+  sample_pick_kernel<T><<<(unsigned)rows, kNT, 0, st>>>(a);
+  if (a.processed) sample_processed_kernel<T><<<grid, kSplitNT, 0, st>>>(a);
+}
+
 }  // namespace
+
+extern "C" int acorn_sample_workspace(int64_t rows, int64_t vocab, int64_t* bytes) {
+  if (rows < 0 || vocab <= 0 || !bytes) return ACORN_ERR_VALUE;
+  *bytes = vocab >= kSplitMinV && vocab <= ((int64_t)1 << 31) && rows <= kSplitMaxRows
+               ? rows * (int64_t)sizeof(SplitRow)
+               : 0;
+  return ACORN_OK;
+}
+
+extern "C" int acorn_sample_split(const void* logits, int64_t rows, int64_t vocab, int dtype,
+                                  const float* temperature, const int32_t* top_k,
+                                  const float* top_p, const float* uniform, int64_t* token,
+                                  float* logprob, float* processed, int32_t* status, void* ws,
+                                  int64_t ws_bytes, void* stream) {
+  int64_t need = 0;
+  if (rows < 0 || vocab <= 0 || acorn_sample_workspace(rows, vocab, &need) != ACORN_OK)
+    return ACORN_ERR_SHAPE;
+  if (!ws || need == 0 || ws_bytes < need)
+    return acorn_sample(logits, rows, vocab, dtype, temperature, top_k, top_p, uniform, token,
+                        logprob, processed, status, stream);
+  if (!logits || !temperature || !top_k || !top_p || !uniform || !token || !logprob || !status ||
+      (uintptr_t)ws % alignof(SplitRow))
+    return ACORN_ERR_VALUE;
+  const SplitArgs a{logits, vocab,   temperature, top_k,     top_p,  uniform,
+                    token,  logprob, processed,   status, (SplitRow*)ws};
+  hipStream_t st = (hipStream_t)stream;
+  switch (dtype) {
+    case ACORN_F32: launch_split<float>(a, rows, st); break;
+    case ACORN_F16: launch_split<_Float16>(a, rows, st); break;
+    case ACORN_BF16: launch_split<__bf16>(a, rows, st); break;
+    default: return ACORN_ERR_DTYPE;
+  }
+  ACORN_LAUNCH_CHECK();
+  return ACORN_OK;
+}
 
 extern "C" int acorn_sample(const void* logits, int64_t rows, int64_t vocab, int dtype,
                             const float* temperature, const int32_t* top_k, const float* top_p,

@@ -43,6 +43,7 @@ from acorninfer_amd._lib import (BF16, WFMT_BF16, WFMT_BF16B, WFMT_W4, WFMT_W4B,
 from acorninfer_amd.config import Qwen3Config
 from acorninfer_amd.ops.paged_attention import prefill_supported
 from acorninfer_amd.quant import quantize as Q
+from acorninfer_amd.sampler import sample_workspace
 
 MI355X_CUS = 256
 FORMATS = {"bf16": WFMT_BF16, "w8a16": WFMT_W8, "w4a16": WFMT_W4}
@@ -657,10 +658,12 @@ class Qwen3DecodeModel:
                             part=buf.ws_lm, stream=st)
         # next token: greedy rows (temperature 0) take the argmax, the others
         # temperature -> top-k -> top-p -> inverse-CDF draw of their uniform
-        check(L.acorn_sample(ptr(buf.logits), B, cfg.vocab_size, dtype_code(buf.logits),
-                             ptr(buf.temperature), ptr(buf.top_k), ptr(buf.top_p),
-                             ptr(buf.uniform), ptr(buf.next_ids), ptr(buf.logprob), None,
-                             ptr(buf.status), st), "sample")
+        check(L.acorn_sample_split(ptr(buf.logits), B, cfg.vocab_size, dtype_code(buf.logits),
+                                   ptr(buf.temperature), ptr(buf.top_k), ptr(buf.top_p),
+                                   ptr(buf.uniform), ptr(buf.next_ids), ptr(buf.logprob), None,
+                                   ptr(buf.status), ptr(buf.ws_sample),
+                                   0 if buf.ws_sample is None else buf.ws_sample.numel(), st),
+              "sample")
         return None
 
     def prefill_swiglu(self, rows: int) -> bool:
@@ -1230,7 +1233,8 @@ class StepBuffers:
         self.ws_ml = z(2 * B * nq * S, dtype=f32) if S > 1 else None
         if self.prefill:
             # step(head_rows=...) computes the few logits it needs on its own
-            self.ws_lm = self.logits = None
+            self.ws_lm = self.logits = self.ws_sample = None
         else:
+            self.ws_sample = sample_workspace(B, cfg.vocab_size, dev)
             self.ws_lm = z(ks_lm, B, cfg.vocab_size, dtype=f32) if ks_lm > 1 else None
             self.logits = z(B, cfg.vocab_size, dtype=dt)

@@ -3,7 +3,7 @@
 Drop-in for acorninfer/sampler.py: `SamplingParams` (:18-22) and
 `Sampler(params, generator)` with `.process(logits)` (:38-55) and
 `.sample(logits) -> (token, logprob)` (:57-68), same argument checks and
-errors. The work is csrc/sampler.hip (acorn_sample): the row is never
+errors. The work is csrc/sampler.hip (acorn_sample_split): the row is never
 sorted; top-k and top-p are radix selects over the fp32 order keys (top-p on
 fixed-point softmax mass, so results are deterministic), ties at the top-p
 boundary resolved in the stable ascending order HF sorts in.
@@ -16,6 +16,7 @@ graph-capturable batched form for the decode step: it never synchronises.
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 
 import torch
@@ -28,6 +29,14 @@ class SamplingParams:
     temperature: float = 1.0
     top_p: float = 1.0
     top_k: int = 0  # 0 = disabled
+
+
+def sample_workspace(rows: int, vocab: int, device) -> torch.Tensor | None:
+    """The workspace acorn_sample_split takes for (rows, vocab), or None where
+    it uses none."""
+    n = ctypes.c_int64(0)
+    check(lib().acorn_sample_workspace(rows, vocab, ctypes.byref(n)), "sample_workspace")
+    return torch.empty(n.value, dtype=torch.uint8, device=device) if n.value else None
 
 
 def sample_batch(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
@@ -58,9 +67,11 @@ def sample_batch(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.T
     if processed is not None:
         assert processed.shape == (B, V) and processed.dtype == torch.float32
         assert processed.device == dev and processed.is_contiguous()
-    rc = lib().acorn_sample(ptr(lg), B, V, dtype_code(lg), ptr(temperature), ptr(top_k),
-                            ptr(top_p), ptr(uniform), ptr(token), ptr(logprob), ptr(processed),
-                            ptr(status), stream_ptr(dev))
+    ws = sample_workspace(B, V, dev)
+    rc = lib().acorn_sample_split(ptr(lg), B, V, dtype_code(lg), ptr(temperature), ptr(top_k),
+                                  ptr(top_p), ptr(uniform), ptr(token), ptr(logprob),
+                                  ptr(processed), ptr(status), ptr(ws),
+                                  0 if ws is None else ws.numel(), stream_ptr(dev))
     check(rc, "sample")
     return token, logprob, status
 

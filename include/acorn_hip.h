@@ -409,6 +409,22 @@ int acorn_sample(const void* logits, int64_t rows, int64_t vocab, int dtype,
                  const float* uniform, int64_t* token, float* logprob, float* processed,
                  int32_t* status, void* stream);
 
+/*
+ * acorn_sample with a caller-held workspace, so that long rows (a vocabulary)
+ * can be read by many workgroups: the same selection, the draw from integer
+ * instead of fp32 sums (the same token but where the uniform falls within their
+ * rounding of a boundary). ws is 64-byte aligned device memory of at least the
+ * bytes acorn_sample_workspace reports for (rows, vocab); its contents need not
+ * be set, and calls that overlap need workspaces of their own. Where it reports
+ * 0 (short rows), or with ws NULL or too small, the call is acorn_sample.
+ */
+int acorn_sample_split(const void* logits, int64_t rows, int64_t vocab, int dtype,
+                       const float* temperature, const int32_t* top_k, const float* top_p,
+                       const float* uniform, int64_t* token, float* logprob, float* processed,
+                       int32_t* status, void* ws, int64_t ws_bytes, void* stream);
+/* *bytes = workspace of acorn_sample_split (0: none is used). No GPU access. */
+int acorn_sample_workspace(int64_t rows, int64_t vocab, int64_t* bytes);
+
 #ifdef __cplusplus
 }
 #endif

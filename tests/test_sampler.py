@@ -166,3 +166,66 @@ def test_greedy_is_first_maximum(dtype, V):
     want = torch.argmax(logits.float(), dim=1)
     assert tok.cpu().tolist() == want.tolist()
     assert lp.cpu().eq(0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [16384, 16385, 16640 + 9, 151936])
+def test_split_rows_equal_one_workgroup_rows(dtype, V):
+    """The split form (a workspace given) against the one-workgroup form
+    (acorn_sample) on the same rows: the kept set and its values bit for bit,
+    the token the one whose interval of the 64-bit cumulative distribution holds
+    the uniform, the logprob within fp32 rounding. V: the shortest split
+    row, odd lengths (rows off 16-byte alignment, a short last chunk), a
+    vocabulary. Rows: peaked, flat, all equal (every element on the boundary:
+    handed to the one-workgroup form), few distinct values (ties across
+    chunks), a tie group of the maximum, zeros of both signs, a maximum in the
+    last element, an infinity. Options: each of top-k and top-p alone,
+    together, neither, a top-k past the lists, greedy, a tiny top-p."""
+    from acorninfer_amd._lib import check, dtype_code, lib, ptr, stream_ptr
+    from acorninfer_amd.sampler import sample_batch, sample_workspace
+    g = torch.Generator().manual_seed(V)
+    x = torch.randn(8, V, generator=g) * 3
+    x[0, ::997] += 9
+    x[2] = 1.5
+    x[3] = torch.randint(0, 40, (V,), generator=g).float() / 8
+    x[4, ::V // 40] = 15.0
+    x[5] = -x[5].abs()
+    x[5, ::777] = 0.0
+    x[5, 5::777] = -0.0
+    x[6, V - 1] = 30.0
+    x[7, V // 2] = float("inf")
+    options = [(0.7, 20, 0.95), (1.0, 0, 0.9), (0.6, 50, 1.0), (1.0, 0, 1.0), (0.9, 5000, 0.8),
+               (0.0, 0, 1.0), (1.0, 1, 1.0), (1.2, 0, 1e-6), (0.8, V, 0.5)]
+    rows = x.repeat_interleave(len(options), 0).to(dtype).cuda()
+    opts = options * x.shape[0]
+    B = rows.shape[0]
+    t = torch.tensor([o[0] for o in opts], device="cuda")
+    k = torch.tensor([o[1] for o in opts], dtype=torch.int32, device="cuda")
+    p = torch.tensor([o[2] for o in opts], device="cuda")
+    u = torch.rand(B, generator=g).cuda()
+    assert sample_workspace(B, V, "cuda") is not None
+    got_p, want_p = (torch.full((B, V), 7.0, device="cuda") for _ in range(2))
+    tok, lp, st = sample_batch(rows, t, k, p, u, processed=got_p)
+    wtok, wlp, wst = torch.empty_like(tok), torch.empty_like(lp), torch.empty_like(st)
+    check(lib().acorn_sample(ptr(rows), B, V, dtype_code(rows), ptr(t), ptr(k), ptr(p), ptr(u),
+                             ptr(wtok), ptr(wlp), ptr(want_p), ptr(wst), stream_ptr()), "sample")
+    assert torch.equal(st, wst) and int(st.sum()) == len(options)
+    assert torch.equal(got_p, want_p)
+    drawn = (wst == 0) & (t > 0)
+    assert torch.equal(tok[~drawn], wtok[~drawn])
+    # the masses are exp2f of x - max (at most 28 in magnitude where they count)
+    # times log2 e in fp32: within 28 * 2^-24 + 2 ulp, i.e. 2e-6, of exact
+    prob = torch.softmax(want_p[drawn].double(), 1)
+    cum = prob.cumsum(1).gather(1, tok[drawn, None])[:, 0]
+    lo = cum - prob.gather(1, tok[drawn, None])[:, 0]
+    assert (prob.gather(1, tok[drawn, None]) > 0).all()
+    assert ((lo - 4e-6 <= u[drawn]) & (u[drawn] <= cum + 4e-6)).all()
+    # sums of at most 151936 fp32 terms against exact integer sums
+    same = tok == wtok
+    assert same.float().mean() > 0.9
+    torch.testing.assert_close(lp[same], wlp[same], rtol=1e-5, atol=1e-5, equal_nan=True)
+    # without the processed row (no fifth launch), and twice
+    for _ in range(2):
+        tok2, lp2, _ = sample_batch(rows, t, k, p, u)
+        assert torch.equal(tok2, tok) and torch.equal(lp2.view(torch.int32), lp.view(torch.int32))
