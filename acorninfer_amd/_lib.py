@@ -52,6 +52,10 @@ _SIGNATURES = {
                                       _i64, _i64, _i64, _i64, _f32, _i32, _vp],
     "acorn_paged_prefill_attention": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64,
                                       _i64, _i64, _i64, _i64, _i64, _i64, _f32, _i32, _vp],
+    "acorn_paged_prefill_attention_ws": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64,
+                                         _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32, _i32,
+                                         _vp, _i64, _vp],
+    "acorn_paged_prefill_workspace": [_i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp],
     "acorn_paged_attention_qkv": [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                   _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _f32,
                                   _vp, _vp, _f32, _vp, _vp, _i32, _i32, _vp],

@@ -521,6 +521,24 @@ __device__ __forceinline__ uint32_t pack_sum(float lo, float hi, float& sum) {
   }
 }
 
+// pack_sum with the two rounded values added by one dot product with (1, 1).
+template <typename T>
+__device__ __forceinline__ uint32_t pack_dot(float lo, float hi, float& sum) {
+  if constexpr (std::is_same<T, __bf16>::value) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    const uint32_t u = pack_bf16x2(lo, hi);
+    sum = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, u),
+                                          __builtin_bit_cast(bf16x2_t, 0x3F803F80u), sum, false);
+    return u;
+  } else {
+    typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+    const uint32_t u = pack2<T>(lo, hi);
+    sum = __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, u),
+                                 __builtin_bit_cast(f16x2_t, 0x3C003C00u), sum, false);
+    return u;
+  }
+}
+
 // Byte offset of the per-wave K slabs in the MFMA kernel's dynamic LDS:
 // after the wave partials [NWV][REP][D], their (m, l) and the split's pps
 // block ids, rounded up to 16 bytes.
@@ -1264,6 +1282,27 @@ int dispatch_d(int64_t D, int64_t rep, const void* q, const void* kp, const void
   return ACORN_ERR_UNSUPPORTED;
 }
 
+// One sequence of a prefill launch: its first q row, that row's position and
+// its rows. With no seq_nq every sequence is a window of max_nq rows at row
+// n max_nq and seq_pos0 holds its length, the window included. Rows past q's R
+// rows (or past max_nq) are not served, so bad metadata cannot reach past q / out.
+struct PrefillSeq {
+  int row0, pos0, nq;
+};
+__device__ __forceinline__ PrefillSeq prefill_seq(const int32_t* row0, const int32_t* pos0,
+                                                  const int32_t* nq, int n, int R, int max_nq) {
+  PrefillSeq s;
+  if (nq == nullptr) {
+    s = {n * max_nq, pos0[n] - max_nq, max_nq};
+    if (s.pos0 + max_nq <= 0) s.nq = 0;
+  } else {
+    s = {row0[n], pos0[n], nq[n]};
+    if (s.row0 < 0 || s.pos0 < 0) s.nq = 0;
+  }
+  s.nq = min(min(s.nq, max_nq), R - s.row0);
+  return s;
+}
+
 // ---------------------------------------------------------------------------
 // Prefill attention: query-tiled flash attention over the paged cache with a
 // causal mask, for a chunked prefill whose new rows' K/V are already in the
@@ -1296,13 +1335,22 @@ int dispatch_d(int64_t D, int64_t rep, const void* q, const void* kp, const void
 // A workgroup reads its keys once for REP x QG x 32 query rows: O(L^2 / 32)
 // K / V bytes per prompt of L tokens and kv head, against O(L^2) for one
 // decode row per token.
-template <typename T, int D, int REP, int QG, int KC>
+//
+// Few query rows over long contexts (a late chunk of a chunked prefill, a
+// follow-up turn, a verify window) give tiles x KV x N workgroups that leave
+// CUs idle while each walks its whole prefix alone: three sequences of 40..300
+// rows over 2000..8000 tokens took 155 us. With SPLIT the keys of a tile are
+// divided into runs of `cps` chunks, one workgroup each; a tile of more than
+// one run leaves (acc, m, l) per run in fp32 for paged_prefill_combine_kernel,
+// and a run in which a query sees no key adds nothing (m stays -inf).
+// QW: 16-query blocks per wave; 1 for windows of at most 16 QG rows.
+template <typename T, int D, int REP, int QG, int KC, int QW, bool SPLIT>
 __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
     const T* __restrict__ q, const T* __restrict__ k_pages, const T* __restrict__ v_pages,
     const int32_t* __restrict__ tables, const int32_t* __restrict__ seq_row0,
     const int32_t* __restrict__ seq_pos0, const int32_t* __restrict__ seq_nq, T* __restrict__ out,
-    int R, int H, int KV, int P, int num_blocks, int table_stride, float scale_log2) {
-  constexpr int QW = 2;                          // 16-query blocks per wave
+    int R, int H, int KV, int P, int num_blocks, int table_stride, float scale_log2, int max_nq,
+    int S, int cps, float* __restrict__ ws) {
   constexpr int NT = REP * QG * kWave;           // threads
   constexpr int KB = D / 32, DPL = D / 16;
   constexpr int KPITCH = 2 * D + 32;             // bytes per staged K row (padded)
@@ -1320,16 +1368,21 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
   const int r = lane >> 4, c = lane & 15;
   const int hq = wid % REP, sub = wid / REP;
   const int h = kvh * REP + hq;
-  const int pos0 = seq_pos0[n];
-  const int row0 = seq_row0[n];
-  // rows past q's R rows are not served (so bad metadata cannot reach past q / out)
-  const int nq = row0 < 0 || pos0 < 0 ? 0 : min(seq_nq[n], R - row0);
-  const int wg_j0 = (gridDim.x - 1 - blockIdx.x) * WQ;          // longest tiles first
+  const PrefillSeq sq = prefill_seq(seq_row0, seq_pos0, seq_nq, n, R, max_nq);
+  const int pos0 = sq.pos0, row0 = sq.row0, nq = sq.nq;
+  const int tile = SPLIT ? (gridDim.x - 1 - blockIdx.x) / S : gridDim.x - 1 - blockIdx.x;
+  const int wg_j0 = tile * WQ;                                  // longest tiles first
   if (wg_j0 >= nq) return;                                       // uniform over the workgroup
   const int j0 = wg_j0 + sub * QW * 16;                          // this wave's first query row
   const int nvalid = max(0, min(QW * 16, nq - j0));              // 0: the wave only stages
   const int L = pos0 + min(wg_j0 + WQ, nq);                      // keys of the workgroup's last query
-  const int nchunks = (L + KC - 1) / KC;
+  // this workgroup's chunks [cb, nchunks) of the tile's `total`
+  const int total = (L + KC - 1) / KC;
+  const int sp = SPLIT ? (gridDim.x - 1 - blockIdx.x) % S : 0;
+  const int cb = SPLIT ? sp * cps : 0;
+  const int nchunks = SPLIT ? min(cb + cps, total) : total;
+  // (uniform over the workgroup; no keys at all: a window longer than its sequence)
+  if (cb >= nchunks) return;
   const int32_t* trow = tables + (size_t)n * table_stride;
   const int pshift = __builtin_ctz(P);
   const int tok_stride = KV * D;
@@ -1379,12 +1432,12 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
     }
   };
 
-  float m[QW], l[QW];
+  float m[QW], l[QW], nm[QW];                    // nm: -m (0 while m is -inf)
   f32x4_t acc[QW][DPL];
 #pragma unroll
   for (int qw = 0; qw < QW; ++qw) {
     m[qw] = -INFINITY;
-    l[qw] = 0.f;
+    l[qw] = nm[qw] = 0.f;
 #pragma unroll
     for (int jj = 0; jj < DPL; ++jj) acc[qw][jj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   }
@@ -1467,17 +1520,18 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
         mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         const float mn = fmaxf(m[qw], mx);
-        const float alpha = __builtin_amdgcn_exp2f(m[qw] - mn);
+        // (a query that has seen no key yet keeps -inf: alpha 0, p = exp2(-inf))
+        nm[qw] = SPLIT && mn == -INFINITY ? 0.f : -mn;
+        const float alpha = __builtin_amdgcn_exp2f(m[qw] + nm[qw]);
         m[qw] = mn;
         l[qw] *= alpha;
 #pragma unroll
         for (int jj = 0; jj < DPL; ++jj) acc[qw][jj] *= alpha;
       }
-      const float nm = -m[qw];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        pb[qw][i] = pack_sum<T>(__builtin_amdgcn_exp2f(__builtin_fmaf(sv[2 * i], scale_log2, nm)),
-                                __builtin_amdgcn_exp2f(__builtin_fmaf(sv[2 * i + 1], scale_log2, nm)),
+        pb[qw][i] = pack_dot<T>(__builtin_amdgcn_exp2f(__builtin_fmaf(sv[2 * i], scale_log2, nm[qw])),
+                                __builtin_amdgcn_exp2f(__builtin_fmaf(sv[2 * i + 1], scale_log2, nm[qw])),
                                 l[qw]);
     }
     typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
@@ -1495,15 +1549,15 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
 
   // prologue: chunk 0 staged, chunk 1's loads and page ids in flight
 #pragma unroll
-  for (int i = 0; i < PH; ++i) pg[i] = page_of(0, i);
-  load_chunk(0, pg);
+  for (int i = 0; i < PH; ++i) pg[i] = page_of(cb, i);
+  load_chunk(cb, pg);
 #pragma unroll
-  for (int i = 0; i < PH; ++i) pg_next[i] = page_of(min(1, nchunks - 1), i);
+  for (int i = 0; i < PH; ++i) pg_next[i] = page_of(min(cb + 1, nchunks - 1), i);
   store_chunk(0);
-  load_chunk(min(1, nchunks - 1), pg_next);
+  load_chunk(min(cb + 1, nchunks - 1), pg_next);
   __syncthreads();
-  for (int ci = 0; ci < nchunks; ++ci) {
-    const int b = ci & 1;
+  for (int ci = cb; ci < nchunks; ++ci) {
+    const int b = (ci - cb) & 1;
     // page ids two chunks ahead
 #pragma unroll
     for (int i = 0; i < PH; ++i) pg[i] = page_of(min(ci + 2, nchunks - 1), i);
@@ -1520,6 +1574,24 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
   }
   if (nvalid == 0) return;
   if (pend) pv();
+  if (SPLIT && total > cps) {                    // one run of several: its fp32 partial
+    const size_t slots = (size_t)gridDim.z * max_nq * H;
+    float2* ml = (float2*)(ws + (size_t)S * slots * D);
+#pragma unroll
+    for (int qw = 0; qw < QW; ++qw) {
+      float lt = l[qw];
+      lt += __shfl_xor(lt, 16);
+      lt += __shfl_xor(lt, 32);
+      if (16 * qw + c < nvalid) {
+        const size_t slot = (size_t)sp * slots + ((size_t)n * max_nq + j0 + 16 * qw + c) * H + h;
+#pragma unroll
+        for (int jj = 0; jj < DPL; ++jj)
+          *(f32x4_t*)(ws + slot * D + 16 * jj + 4 * r) = acc[qw][jj];
+        if (r == 0) ml[slot] = make_float2(m[qw], lt);
+      }
+    }
+    return;
+  }
   // lane (r, c) of block qw holds dims 16 jj + 4 r + i of query column 16 qw + c
 #pragma unroll
   for (int qw = 0; qw < QW; ++qw) {
@@ -1541,33 +1613,147 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
 
 constexpr int kPrefillChunk = 64;   // keys staged per barrier (32: 3% slower at 8192 tokens)
 
-template <typename T, int D, int REP>
-int launch_prefill(const void* q, const void* kp, const void* vp, const int32_t* tables,
-                   const int32_t* row0, const int32_t* pos0, const int32_t* nq, void* out,
-                   int64_t N, int64_t R, int64_t max_nq, int64_t H, int64_t KV, int64_t P,
-                   int64_t num_blocks, int64_t table_stride, float scale, hipStream_t st) {
-  // four waves per workgroup (eight for 8 q heads per kv head), 32 query rows each
+// Merge of a split tile's partials: one group of D / 4 lanes per (row, head),
+// four dims per lane; tiles of one run were written by the kernel itself.
+constexpr int kPrefillCombineNT = 256;
+template <typename T, int D>
+__global__ __launch_bounds__(kPrefillCombineNT) void paged_prefill_combine_kernel(
+    const float* __restrict__ ws, const int32_t* __restrict__ seq_row0,
+    const int32_t* __restrict__ seq_pos0, const int32_t* __restrict__ seq_nq, T* __restrict__ out,
+    int R, int H, int max_nq, int S, int cps, int WQ) {
+  constexpr int LPP = D / 4;
+  const int n = blockIdx.y;
+  const int pair = (int)(blockIdx.x * (kPrefillCombineNT / LPP)) + threadIdx.x / LPP;
+  const int j = pair / H, h = pair % H, d0 = 4 * (threadIdx.x % LPP);
+  const PrefillSeq sq = prefill_seq(seq_row0, seq_pos0, seq_nq, n, R, max_nq);
+  if (j >= sq.nq) return;
+  const int L = sq.pos0 + min(j / WQ * WQ + WQ, sq.nq);
+  const int total = (L + kPrefillChunk - 1) / kPrefillChunk;
+  if (total <= cps) return;
+  const int ns = (total + cps - 1) / cps;        // <= S
+  const size_t slots = (size_t)gridDim.y * max_nq * H;
+  const size_t slot = ((size_t)n * max_nq + j) * H + h;
+  const float2* ml = (const float2*)(ws + (size_t)S * slots * D) + slot;
+  const float* src = ws + slot * D + d0;
+  float M = -INFINITY;
+  for (int s = 0; s < ns; ++s) M = fmaxf(M, ml[s * slots].x);
+  f32x4_t a = {0.f, 0.f, 0.f, 0.f};
+  float lsum = 0.f;
+  constexpr int U = 4;                           // runs requested together
+  for (int s0 = 0; s0 < ns; s0 += U) {
+    f32x4_t x[U];
+    float2 mls[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t s = (size_t)min(s0 + u, ns - 1);
+      x[u] = *(const f32x4_t*)(src + s * slots * D);
+      mls[u] = ml[s * slots];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s0 + u >= ns) continue;
+      const float w = M == -INFINITY ? 0.f : exp2f(mls[u].x - M);
+      lsum += w * mls[u].y;
+      a += w * x[u];
+    }
+  }
+  const float inv = 1.0f / lsum;
+  const u32x2_t w = {pack2<T>(a[0] * inv, a[1] * inv), pack2<T>(a[2] * inv, a[3] * inv)};
+  *(u32x2_t*)(out + ((size_t)(sq.row0 + j) * H + h) * D + d0) = w;
+}
+
+// The key split of a prefill launch: S runs of cps chunks per query tile (S ==
+// 1: none) and the 16-query blocks per wave.
+struct PrefillPlan {
+  int qw = 2, S = 1, cps = 1;
+  int64_t ws_bytes = 0;
+};
+// The tiles alone (R rows in all, a partly filled tile per sequence) leave
+// CUs idle: split towards two workgroups per CU, the most that fit their LDS,
+// three where sequences may differ in length (a short one's runs end early). A
+// run costs its rows' fp32 partials, written and read: small next to a window's
+// keys, about five chunks' time for a full tile, so runs keep kWindowMinRun
+// chunks, kPrefillMinRun, or kPrefillBusyRun once half the CUs have a tile.
+// Measured, one split / this rule (us): 8 windows of 5 rows over 1024..8192
+// tokens 162 / 48, 3 prompts' 40..300 rows over 2000..8000 tokens 153 / 64,
+// 100 rows over 8000 219 / 48, 512 over 8000 232 / 112, 1000 over 8000
+// 250 / 197; 1000 rows with no prefix 39.5 unsplit, 43.7 in two runs.
+constexpr int64_t kWindowMinRun = 4, kPrefillMinRun = 6, kPrefillBusyRun = 16;
+constexpr int64_t kPrefillMaxRuns = 64;
+PrefillPlan prefill_plan(int64_t N, int64_t R, int64_t max_nq, int64_t H, int64_t KV, int64_t D,
+                         int64_t P, int64_t table_stride) {
+  PrefillPlan p;
+  const int64_t rep = H / KV;
+  const int64_t qg = rep >= 4 ? 1 : 4 / rep;
+  if (max_nq <= 16 * qg) p.qw = 1;
+  const int64_t wq = 16 * p.qw * qg;
+  const int64_t tiles = std::min(N * ((max_nq + wq - 1) / wq), (R + wq - 1) / wq + N / 2);
+  const int64_t base = std::max<int64_t>(1, tiles * KV);
+  const int64_t chunks = (table_stride * P + kPrefillChunk - 1) / kPrefillChunk;
+  const int64_t min_run = p.qw == 1 ? kWindowMinRun
+                          : base >= kCUs / 2 ? kPrefillBusyRun
+                                             : kPrefillMinRun;
+  const int64_t target = p.qw == 2 && N > 1 ? 3 * kCUs : 2 * kCUs;
+  const int64_t S = std::min(std::min((target + base / 2) / base, (chunks + min_run - 1) / min_run),
+                             kPrefillMaxRuns);
+  if (S <= 1) return p;
+  p.cps = (int)((chunks + S - 1) / S);
+  p.S = (int)((chunks + p.cps - 1) / p.cps);
+  if (p.S > 1) p.ws_bytes = p.S * N * max_nq * H * (D + 2) * 4;
+  return p;
+}
+
+struct PrefillArgs {
+  const void *q, *kp, *vp;
+  const int32_t *tables, *row0, *pos0, *nq;
+  void* out;
+  int64_t N, R, max_nq, H, KV, P, num_blocks, table_stride;
+  float scale;
+  PrefillPlan plan;
+  float* ws;
+  hipStream_t st;
+};
+
+template <typename T, int D, int REP, int QW, bool SPLIT>
+int launch_prefill(const PrefillArgs& a) {
+  // four waves per workgroup (eight for 8 q heads per kv head), 16 QW query rows each
   constexpr int QG = REP >= 4 ? 1 : 4 / REP;
-  const int64_t tiles = (max_nq + 32 * QG - 1) / (32 * QG);
-  paged_prefill_kernel<T, D, REP, QG, kPrefillChunk>
-      <<<dim3((unsigned)tiles, (unsigned)KV, (unsigned)N), dim3(REP * QG * kWave), 0, st>>>(
-          (const T*)q, (const T*)kp, (const T*)vp, tables, row0, pos0, nq, (T*)out, (int)R,
-          (int)H, (int)KV, (int)P, (int)num_blocks, (int)table_stride, scale * kLog2e);
+  constexpr int WQ = 16 * QW * QG;
+  const int64_t tiles = (a.max_nq + WQ - 1) / WQ;
+  const int S = SPLIT ? a.plan.S : 1;
+  paged_prefill_kernel<T, D, REP, QG, kPrefillChunk, QW, SPLIT>
+      <<<dim3((unsigned)(tiles * S), (unsigned)a.KV, (unsigned)a.N), dim3(REP * QG * kWave), 0,
+         a.st>>>((const T*)a.q, (const T*)a.kp, (const T*)a.vp, a.tables, a.row0, a.pos0, a.nq,
+                 (T*)a.out, (int)a.R, (int)a.H, (int)a.KV, (int)a.P, (int)a.num_blocks,
+                 (int)a.table_stride, a.scale * kLog2e, (int)a.max_nq, S, a.plan.cps, a.ws);
   ACORN_LAUNCH_CHECK();
+  if (SPLIT) {
+    constexpr int pairs = kPrefillCombineNT / (D / 4);
+    paged_prefill_combine_kernel<T, D>
+        <<<dim3((unsigned)((a.max_nq * a.H + pairs - 1) / pairs), (unsigned)a.N),
+           dim3(kPrefillCombineNT), 0, a.st>>>(a.ws, a.row0, a.pos0, a.nq, (T*)a.out, (int)a.R,
+                                               (int)a.H, (int)a.max_nq, S, a.plan.cps, WQ);
+    ACORN_LAUNCH_CHECK();
+  }
   return ACORN_OK;
 }
 
+template <typename T, int D, int REP>
+int prefill_form(const PrefillArgs& a) {
+  if (a.plan.S > 1)
+    return a.plan.qw == 1 ? launch_prefill<T, D, REP, 1, true>(a)
+                          : launch_prefill<T, D, REP, 2, true>(a);
+  return a.plan.qw == 1 ? launch_prefill<T, D, REP, 1, false>(a)
+                        : launch_prefill<T, D, REP, 2, false>(a);
+}
+
 template <typename T, int D>
-int prefill_rep(int64_t rep, const void* q, const void* kp, const void* vp,
-                const int32_t* tables, const int32_t* row0, const int32_t* pos0,
-                const int32_t* nq, void* out, int64_t N, int64_t R, int64_t max_nq, int64_t H,
-                int64_t KV, int64_t P, int64_t num_blocks, int64_t ts, float scale,
-                hipStream_t st) {
-  switch (rep) {
-    case 1: return launch_prefill<T, D, 1>(q, kp, vp, tables, row0, pos0, nq, out, N, R, max_nq, H, KV, P, num_blocks, ts, scale, st);
-    case 2: return launch_prefill<T, D, 2>(q, kp, vp, tables, row0, pos0, nq, out, N, R, max_nq, H, KV, P, num_blocks, ts, scale, st);
-    case 4: return launch_prefill<T, D, 4>(q, kp, vp, tables, row0, pos0, nq, out, N, R, max_nq, H, KV, P, num_blocks, ts, scale, st);
-    case 8: return launch_prefill<T, D, 8>(q, kp, vp, tables, row0, pos0, nq, out, N, R, max_nq, H, KV, P, num_blocks, ts, scale, st);
+int prefill_rep(const PrefillArgs& a) {
+  switch (a.H / a.KV) {
+    case 1: return prefill_form<T, D, 1>(a);
+    case 2: return prefill_form<T, D, 2>(a);
+    case 4: return prefill_form<T, D, 4>(a);
+    case 8: return prefill_form<T, D, 8>(a);
   }
   return ACORN_ERR_UNSUPPORTED;
 }
@@ -1598,6 +1784,53 @@ extern "C" int acorn_paged_attention(const void* q, const void* k_pages, const v
   return ACORN_ERR_DTYPE;
 }
 
+static int prefill_shape(int64_t N, int64_t R, int64_t max_nq, int64_t H, int64_t KV, int64_t D,
+                         int64_t P, int64_t num_blocks, int64_t table_stride) {
+  if (N < 0 || R < 0 || max_nq < 0 || H <= 0 || KV <= 0 || D <= 0 || P <= 0 ||
+      num_blocks <= 0 || table_stride < 1)
+    return ACORN_ERR_SHAPE;
+  if ((P & (P - 1)) != 0 || P % 16 != 0 || H % KV != 0) return ACORN_ERR_SHAPE;
+  if (KV > 65535 || N > 65535 || R > 0x7fffffff || max_nq > 0x7fffffff) return ACORN_ERR_SHAPE;
+  return ACORN_OK;
+}
+
+extern "C" int acorn_paged_prefill_workspace(int64_t N, int64_t R, int64_t max_nq, int64_t H, int64_t KV,
+                                             int64_t D, int64_t P, int64_t table_stride,
+                                             int64_t* bytes) {
+  const int rc = prefill_shape(N, R, max_nq, H, KV, D, P, 1, table_stride);
+  if (rc != ACORN_OK) return rc;
+  if (!bytes) return ACORN_ERR_VALUE;
+  *bytes = N == 0 || R == 0 || max_nq == 0
+               ? 0
+               : prefill_plan(N, R, max_nq, H, KV, D, P, table_stride).ws_bytes;
+  return ACORN_OK;
+}
+
+extern "C" int acorn_paged_prefill_attention_ws(
+    const void* q, const void* k_pages, const void* v_pages, const int32_t* tables,
+    const int32_t* seq_row0, const int32_t* seq_pos0, const int32_t* seq_nq, void* out, int64_t N,
+    int64_t R, int64_t max_nq, int64_t H, int64_t KV, int64_t D, int64_t P, int64_t num_blocks,
+    int64_t table_stride, float scale, int dtype, void* ws, int64_t ws_bytes, void* stream) {
+  const int rc = prefill_shape(N, R, max_nq, H, KV, D, P, num_blocks, table_stride);
+  if (rc != ACORN_OK) return rc;
+  if (N == 0 || R == 0 || max_nq == 0) return ACORN_OK;
+  if (!q || !k_pages || !v_pages || !tables || !seq_pos0 || !out || !seq_row0 != !seq_nq)
+    return ACORN_ERR_VALUE;
+  if (!seq_nq && R != N * max_nq) return ACORN_ERR_SHAPE;
+  if ((uintptr_t)ws % 16) return ACORN_ERR_VALUE;
+  PrefillArgs a{q,  k_pages, v_pages, tables, seq_row0, seq_pos0,     seq_nq, out,
+                N,  R,       max_nq,  H,      KV,       P,            num_blocks, table_stride,
+                scale, prefill_plan(N, R, max_nq, H, KV, D, P, table_stride), (float*)ws,
+                (hipStream_t)stream};
+  if (!ws || ws_bytes < a.plan.ws_bytes) a.plan.S = 1;   // nothing is split
+  if (D != 64 && D != 128) return ACORN_ERR_UNSUPPORTED;
+  switch (dtype) {
+    case ACORN_F16: return D == 64 ? prefill_rep<_Float16, 64>(a) : prefill_rep<_Float16, 128>(a);
+    case ACORN_BF16: return D == 64 ? prefill_rep<__bf16, 64>(a) : prefill_rep<__bf16, 128>(a);
+  }
+  return ACORN_ERR_UNSUPPORTED;
+}
+
 extern "C" int acorn_paged_prefill_attention(const void* q, const void* k_pages,
                                              const void* v_pages, const int32_t* tables,
                                              const int32_t* seq_row0, const int32_t* seq_pos0,
@@ -1606,26 +1839,13 @@ extern "C" int acorn_paged_prefill_attention(const void* q, const void* k_pages,
                                              int64_t D, int64_t P, int64_t num_blocks,
                                              int64_t table_stride, float scale, int dtype,
                                              void* stream) {
-  if (N < 0 || R < 0 || max_nq < 0 || H <= 0 || KV <= 0 || D <= 0 || P <= 0 ||
-      num_blocks <= 0 || table_stride < 1)
-    return ACORN_ERR_SHAPE;
-  if ((P & (P - 1)) != 0 || P % 16 != 0 || H % KV != 0) return ACORN_ERR_SHAPE;
-  if (KV > 65535 || N > 65535 || R > 0x7fffffff || max_nq > 0x7fffffff) return ACORN_ERR_SHAPE;
-  if (N == 0 || R == 0 || max_nq == 0) return ACORN_OK;
-  if (!q || !k_pages || !v_pages || !tables || !seq_row0 || !seq_pos0 || !seq_nq || !out)
-    return ACORN_ERR_VALUE;
-  const int64_t rep = H / KV;
-  hipStream_t st = (hipStream_t)stream;
-  if (D != 64 && D != 128) return ACORN_ERR_UNSUPPORTED;
-  switch (dtype) {
-    case ACORN_F16:
-      return D == 64 ? prefill_rep<_Float16, 64>(rep, q, k_pages, v_pages, tables, seq_row0, seq_pos0, seq_nq, out, N, R, max_nq, H, KV, P, num_blocks, table_stride, scale, st)
-                     : prefill_rep<_Float16, 128>(rep, q, k_pages, v_pages, tables, seq_row0, seq_pos0, seq_nq, out, N, R, max_nq, H, KV, P, num_blocks, table_stride, scale, st);
-    case ACORN_BF16:
-      return D == 64 ? prefill_rep<__bf16, 64>(rep, q, k_pages, v_pages, tables, seq_row0, seq_pos0, seq_nq, out, N, R, max_nq, H, KV, P, num_blocks, table_stride, scale, st)
-                     : prefill_rep<__bf16, 128>(rep, q, k_pages, v_pages, tables, seq_row0, seq_pos0, seq_nq, out, N, R, max_nq, H, KV, P, num_blocks, table_stride, scale, st);
+  if (N > 0 && R > 0 && max_nq > 0 && (!seq_row0 || !seq_nq)) {
+    const int rc = prefill_shape(N, R, max_nq, H, KV, D, P, num_blocks, table_stride);
+    return rc != ACORN_OK ? rc : ACORN_ERR_VALUE;
   }
-  return ACORN_ERR_UNSUPPORTED;
+  return acorn_paged_prefill_attention_ws(q, k_pages, v_pages, tables, seq_row0, seq_pos0, seq_nq,
+                                          out, N, R, max_nq, H, KV, D, P, num_blocks,
+                                          table_stride, scale, dtype, nullptr, 0, stream);
 }
 
 // ---------------------------------------------------------------------------

@@ -41,7 +41,7 @@ from acorninfer_amd._lib import (BF16, WFMT_BF16, WFMT_BF16B, WFMT_W4, WFMT_W4B,
                                  check,
                                  dtype_code, lib, ptr, stream_ptr)
 from acorninfer_amd.config import Qwen3Config
-from acorninfer_amd.ops.paged_attention import prefill_supported
+from acorninfer_amd.ops.paged_attention import prefill_supported, prefill_workspace
 from acorninfer_amd.quant import quantize as Q
 from acorninfer_amd.sampler import sample_workspace
 
@@ -541,6 +541,11 @@ class Qwen3DecodeModel:
             L.acorn_paged_attention_qkv_supported(nq, nkv, D, page_size, buf.max_pages,
                                                   buf.num_splits, dt, wdt))
 
+        # (one workspace for the layers' prefill attention, which run in order)
+        ws_attn = None if segments is None else prefill_workspace(
+            segments.count, B, segments.max_nq, nq, nkv, D, page_size, segments.tables.shape[1],
+            self.device)
+
         def k1(first: bool, y, part, ks: int, w) -> None:
             """K1 after a projection: the residual add + RMSNorm from its
             output in the activation dtype (y), or from its fp32 partials; the
@@ -594,10 +599,11 @@ class Qwen3DecodeModel:
                     "qkv_epilogue")
                 if segments is not None:
                     sg = segments
-                    check(L.acorn_paged_prefill_attention(
+                    check(L.acorn_paged_prefill_attention_ws(
                         ptr(buf.q), kp, vp, ptr(sg.tables), ptr(sg.row0), ptr(sg.pos0),
                         ptr(sg.nq), ptr(buf.attn), sg.count, B, sg.max_nq, nq, nkv, D,
-                        page_size, num_blocks, sg.tables.shape[1], float(self.scale), dt, st),
+                        page_size, num_blocks, sg.tables.shape[1], float(self.scale), dt,
+                        ptr(ws_attn), 0 if ws_attn is None else ws_attn.numel(), st),
                         "prefill attention")
                 else:
                     # K3

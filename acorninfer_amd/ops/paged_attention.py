@@ -12,6 +12,8 @@ use it.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from acorninfer_amd._lib import check, dtype_code, lib, ptr, require_gpu, stream_ptr
@@ -82,6 +84,16 @@ def prefill_supported(dtype: torch.dtype, head_dim: int, page_size: int, num_hea
             and num_heads % kv_heads == 0 and num_heads // kv_heads in (1, 2, 4, 8))
 
 
+def prefill_workspace(N: int, R: int, max_nq: int, H: int, KV: int, D: int, P: int,
+                      table_width: int, device) -> torch.Tensor | None:
+    """The workspace a prefill launch of these sizes splits its keys over, or
+    None where it does not."""
+    n = ctypes.c_int64(0)
+    check(lib().acorn_paged_prefill_workspace(N, R, max_nq, H, KV, D, P, table_width,
+                                              ctypes.byref(n)), "paged_prefill_workspace")
+    return torch.empty(n.value, dtype=torch.uint8, device=device) if n.value else None
+
+
 def paged_prefill_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
                             tables: torch.Tensor, seq_row0: torch.Tensor,
                             seq_pos0: torch.Tensor, seq_nq: torch.Tensor, max_nq: int, *,
@@ -110,10 +122,13 @@ def paged_prefill_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: tor
     if out is None:
         out = torch.empty_like(q2)
     _check_out(out, (R, H, D), q)
-    rc = lib().acorn_paged_prefill_attention(
+    W = max(1, tables.shape[1])
+    ws = prefill_workspace(N, R, int(max_nq), H, KV, D, P, W, q.device)
+    rc = lib().acorn_paged_prefill_attention_ws(
         ptr(q2), ptr(k_pages), ptr(v_pages), ptr(tables), ptr(seq_row0), ptr(seq_pos0),
-        ptr(seq_nq), ptr(out), N, R, int(max_nq), H, KV, D, P, NB, max(1, tables.shape[1]),
-        float(D ** -0.5), dtype_code(q2), stream_ptr(q.device))
+        ptr(seq_nq), ptr(out), N, R, int(max_nq), H, KV, D, P, NB, W,
+        float(D ** -0.5), dtype_code(q2), ptr(ws), 0 if ws is None else ws.numel(),
+        stream_ptr(q.device))
     check(rc, "paged_prefill_attention")
     return out
 

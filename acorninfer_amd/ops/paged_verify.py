@@ -7,20 +7,23 @@ seq_lens[b] - (m - 1 - j) tokens (its history plus the window's first j + 1
 tokens); seq_lens counts the whole window, and the window's k/v are already in
 the pages (`PagedKVCache.scatter_verify`).
 
-On this build the rows are K3 rows (csrc/paged_attention.hip through
-`acorn_paged_attention`): the window is flattened to B*m query rows, row
-(b, j) carries sequence b's block table and its own visible length, and the
-same split/combine kernels as decode run over them. Nothing about K3 changes:
-decode is the m = 1 case. Like the reference this path is eager (a verify
-step is not graph-captured there); the per-row tables and lengths are built
-on the device each call.
+A window is a short prefill whose prefix is in the cache: it runs on the
+query-tiled prefill kernel (`acorn_paged_prefill_attention_ws`), which reads a
+sequence's K/V once for the whole window and divides a long context over
+several workgroups. As one K3 row per window token, the form below, eight
+windows of five over 1024..8192 tokens took 110 us, each row reading the
+context for itself; shapes the prefill kernel is not built for (fp32, head
+sizes other than 64 / 128, pages under 16 tokens) and one-token windows, which
+are decode, keep it: the window is flattened to B*m query rows and the
+split/combine kernels of decode run over them.
 """
 from __future__ import annotations
 
 import torch
 
-from acorninfer_amd._lib import require_gpu
-from acorninfer_amd.ops.paged_attention import paged_decode_attention
+from acorninfer_amd._lib import check, dtype_code, lib, ptr, require_gpu, stream_ptr
+from acorninfer_amd.ops.paged_attention import (paged_decode_attention, prefill_supported,
+                                                prefill_workspace)
 
 __all__ = ["paged_verify_attention"]
 
@@ -45,6 +48,20 @@ def paged_verify_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torc
     assert k_pages.is_contiguous() and v_pages.is_contiguous()
     assert tables.is_contiguous() and seq_lens.is_contiguous()
     assert tables.dtype == torch.int32 and seq_lens.dtype == torch.int32
+    if M > 1 and B > 0 and prefill_supported(q.dtype, D, P, H, KV):
+        assert k_pages.dtype == q.dtype == v_pages.dtype
+        assert k_pages.shape[3] == D
+        assert tables.shape[1] >= 1, "tables must hold at least one page per sequence"
+        q2 = q.contiguous()
+        out = torch.empty_like(q2)
+        W = tables.shape[1]
+        ws = prefill_workspace(B, B * M, M, H, KV, D, P, W, q.device)
+        rc = lib().acorn_paged_prefill_attention_ws(
+            ptr(q2), ptr(k_pages), ptr(v_pages), ptr(tables), None, ptr(seq_lens), None, ptr(out),
+            B, B * M, M, H, KV, D, P, NB, W, float(D ** -0.5), dtype_code(q2), ptr(ws),
+            0 if ws is None else ws.numel(), stream_ptr(q.device))
+        check(rc, "paged_verify_attention")
+        return out
     # row (b, j): sequence b's table, length seq_lens[b] - (m - 1 - j)
     row_tables = tables.repeat_interleave(M, dim=0)
     back = torch.arange(M - 1, -1, -1, device=seq_lens.device, dtype=torch.int32)

@@ -230,6 +230,28 @@ int acorn_paged_prefill_attention(const void* q, const void* k_pages, const void
                                   float scale, int dtype, void* stream);
 
 /*
+ * acorn_paged_prefill_attention with a caller-held workspace (16-byte aligned,
+ * at least the bytes acorn_paged_prefill_workspace reports; its contents need
+ * not be set, overlapping calls need their own): where the query tiles alone
+ * would leave CUs idle, a tile's keys are divided over several workgroups,
+ * whose fp32 partials a second launch merges. Where it reports 0, or with ws
+ * NULL or too small, nothing is split. seq_row0 and seq_nq both NULL: every
+ * sequence is a window of max_nq rows at row n * max_nq (R == N * max_nq), and
+ * seq_pos0[n] is its length, the window included (the verify attention of
+ * acorninfer/ops/paged_verify.py:96-123; >= max_nq).
+ */
+int acorn_paged_prefill_attention_ws(const void* q, const void* k_pages, const void* v_pages,
+                                     const int32_t* tables, const int32_t* seq_row0,
+                                     const int32_t* seq_pos0, const int32_t* seq_nq, void* out,
+                                     int64_t N, int64_t R, int64_t max_nq, int64_t H, int64_t KV,
+                                     int64_t D, int64_t P, int64_t num_blocks,
+                                     int64_t table_stride, float scale, int dtype, void* ws,
+                                     int64_t ws_bytes, void* stream);
+/* *bytes = workspace of acorn_paged_prefill_attention_ws (0: none). No GPU access. */
+int acorn_paged_prefill_workspace(int64_t N, int64_t R, int64_t max_nq, int64_t H, int64_t KV,
+                                  int64_t D, int64_t P, int64_t table_stride, int64_t* bytes);
+
+/*
  * 1 when acorn_paged_attention_qkv supports the shape: bf16 or fp16
  * activations with norm weights of the same dtype, D in {64, 128}, H/KV in
  * {1, 2, 4, 8}, pages of a power-of-two multiple of 16 tokens, and splits

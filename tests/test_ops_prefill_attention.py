@@ -195,3 +195,80 @@ def test_prefill_attention_contract():
         paged_prefill_attention(q.cuda(), kp[:, :8].contiguous().cuda(),
                                 vp[:, :8].contiguous().cuda(), tb.cuda(),
                                 *[m.cuda() for m in meta], 4)
+
+
+# (H, KV, D, P, [(pos0, nq), ...]) whose keys are divided into runs: run
+# boundaries (multiples of 64 cps keys) inside a tile's rows, so that some of its
+# queries see no key of the last run; sequences of one, two and more runs in one
+# launch; windows of at most 16 rows per group; every GQA ratio and head size
+SPLIT_CASES = [
+    (32, 8, 128, 16, [(370, 40), (760, 3)]),
+    (32, 8, 128, 16, [(250, 12), (500, 12), (3, 5)]),
+    (16, 8, 128, 16, [(370, 30), (700, 60)]),
+    (8, 8, 64, 32, [(380, 130), (900, 1)]),
+    (8, 8, 128, 16, [(1020, 5)]),
+    (64, 8, 64, 16, [(1500, 33), (0, 33)]),
+    (8, 2, 128, 16, [(2500, 16)]),
+    (4, 4, 64, 16, [(255, 2), (256, 1), (640, 7)]),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", range(len(SPLIT_CASES)))
+def test_split_keys_match_oracle_and_unsplit(case, dtype):
+    """The split form against the oracle and against the unsplit launch (the
+    entry without a workspace): both round fp32 sums of the same terms once, so
+    they differ by one rounding step of an output at most. Repeated and replayed
+    runs are bitwise equal; a workspace that is too small is not used."""
+    from acorninfer_amd._lib import check, dtype_code, lib, ptr, stream_ptr
+    from acorninfer_amd.ops.paged_attention import paged_prefill_attention, prefill_workspace
+    H, KV, D, P, segs = SPLIT_CASES[case]
+    q, kp, vp, tb, meta = _make(H, KV, D, P, segs, dtype, seed=90 + case)
+    N, R, W, max_nq = len(segs), q.shape[0], tb.shape[1], int(meta[2].max())
+    ws = prefill_workspace(N, R, max_nq, H, KV, D, P, W, "cuda")
+    assert ws is not None, "the case is meant to split"
+    ws.fill_(0xFF)                                   # NaN: stale contents must not matter
+    dev = [t.cuda() for t in (q, kp, vp, tb, *meta)]
+
+    def run(out, work, size):
+        check(lib().acorn_paged_prefill_attention_ws(
+            *(ptr(t) for t in dev), ptr(out), N, R, max_nq, H, KV, D, P, kp.shape[0], W,
+            float(D ** -0.5), dtype_code(q), ptr(work), size, stream_ptr()), "prefill")
+        return out
+
+    got = run(torch.full_like(dev[0], 7.0), ws, ws.numel())
+    flat = run(torch.full_like(dev[0], 7.0), None, 0)
+    assert torch.equal(flat, run(torch.full_like(dev[0], 7.0), ws, ws.numel() - 1))
+    covered = torch.zeros(R, dtype=torch.bool)
+    for i, w in _oracle(q, kp, vp, tb, meta).items():
+        a, n = int(meta[0][i]), int(meta[2][i])
+        torch.testing.assert_close(got[a:a + n].cpu(), w, **TOL_BF16)
+        covered[a:a + n] = True
+    assert bool((got.cpu()[~covered] == 7.0).all()), "rows outside every sequence were written"
+    eps = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)     # one step of a rounded output,
+    torch.testing.assert_close(got.float(), flat.float(), rtol=eps, atol=2e-3)  # P's near zero
+    out = torch.zeros_like(dev[0])                   # (uncovered rows stay as they are)
+
+    def op():
+        paged_prefill_attention(*dev, max_nq, out=out)
+    op()
+    assert torch.equal(out.cpu()[covered], got.cpu()[covered])
+    assert graph_replays_match(op, lambda: out)
+
+
+@pytest.mark.parametrize("max_nq", [1, 5, 16, 17, 100, 2000])
+@pytest.mark.parametrize("width", [1, 40, 512, 20000])
+def test_workspace_grows_no_further_than_its_split(max_nq, width):
+    """The planned workspace (no GPU): whole runs of (D + 2) floats per row and
+    head, at most 64 of them, and none where the tiles fill the CUs."""
+    import ctypes
+    from acorninfer_amd._lib import check, lib
+    n = ctypes.c_int64(-1)
+    for N, H, KV, D in ((1, 32, 8, 128), (9, 16, 8, 64), (300, 8, 8, 128)):
+        check(lib().acorn_paged_prefill_workspace(N, N * max_nq, max_nq, H, KV, D, 16, width,
+                                                  ctypes.byref(n)), "workspace")
+        run = N * max_nq * H * (D + 2) * 4
+        assert n.value % run == 0 and (n.value == 0 or 2 <= n.value // run <= 64)
+        if N == 300:
+            assert n.value == 0
