@@ -492,11 +492,13 @@ __device__ void sample_row(
 //   stats   chunk maxima and finiteness; clears the row's histogram
 //   hist    histogram of the row over kSplitNB bins of 1/64 in x = logit / T
 //           below the maximum: counts (top-k) or fixed-point mass (top-p);
-//           with neither, the chunk's mass. Greedy and non-finite rows end here
+//           with neither, the chunk's mass. Top-k also lists the chunk's own
+//           first k elements, in vocabulary order. Greedy and non-finite rows
+//           end here
 //   gather  the boundary bin, from the histogram; the elements that may lie on
-//           the boundary (top-k: all down to the boundary bin; top-p: those
-//           in it) listed per chunk in vocabulary order, and the chunk's mass
-//           above it
+//           the boundary (top-p: those in it; top-k, only where some chunk's
+//           first k overflowed its list: all down to it) listed per chunk, and
+//           the chunk's mass above it
 //   pick    one workgroup per row ranks the listed elements by counting, which
 //           gives the kept set, finds the drawn chunk from the chunks' masses
 //           and the token inside it
@@ -507,7 +509,7 @@ __device__ void sample_row(
 // top-k, many ties) or whose maximum overflows are left to sample_row.
 // Four launches of a few microseconds each, bound by their latency.
 constexpr int kSplitG = 32;          // workgroups (chunks) per row
-constexpr int kSplitNT = 256;        // their threads
+constexpr int kSplitNT = 1024;       // their threads
 constexpr int kSplitNB = 2048;       // histogram bins: 32 in x, the last takes the rest
 constexpr float kSplitScale = 64.f;  // bins per unit of x
 constexpr int kSplitCapC = 64;       // listed elements per chunk (one wave)
@@ -527,7 +529,8 @@ struct alignas(64) SplitRow {
   float cmax[kSplitG];
   uint32_t cimax[kSplitG];
   uint32_t cbad[kSplitG];
-  uint32_t ccnt[kSplitG];             // elements on the boundary (listed up to kSplitCapC)
+  uint32_t lcnt[kSplitG];             // top-k: listed by `hist` (up to kSplitCapC), and ...
+  uint32_t ccnt[kSplitG];             // ... by `gather`
   unsigned long long zk, above;       // top-p: the row's mass, and that above the boundary bin
   uint32_t state, pkey, tie0;         // kept: key > pkey, or key == pkey and index >= tie0
 };
@@ -588,6 +591,65 @@ __device__ __forceinline__ void load8(const T* row, int64_t i, int64_t end, bool
   }
 }
 
+// Elements [c0, c1) of a row in groups of eight, kOct of a thread's groups
+// requested together. Rows whose groups are whole and 16-byte aligned (V % 8 ==
+// 0) are read as vectors, clamped to the last one so that every load is
+// unconditional; others element by element.
+constexpr int kOct = 1;
+template <typename T, int NT>
+struct Octets {
+  static constexpr int E = 16 / sizeof(T), Q = 8 / E;
+  const T* row;
+  int64_t c0, c1, n;                    // the range and its groups
+  bool fast;
+  u32x4v w[kOct][Q];
+  __device__ Octets(const T* row_, int64_t V, int64_t c0_, int64_t c1_)
+      : row(row_), c0(c0_), c1(c1_), n((c1_ - c0_ + 7) / 8),
+        fast(((uintptr_t)row_ % 16) == 0 && V % 8 == 0) {}
+  // request groups j0, j0 + stride, ... (kOct of them)
+  __device__ __forceinline__ void load(int64_t j0, int64_t stride) {
+    if (!fast || n == 0) return;
+#pragma unroll
+    for (int u = 0; u < kOct; ++u)
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+        w[u][q] = ((const u32x4v*)(row + c0 + min(j0 + u * stride, n - 1) * 8))[q];
+#pragma unroll
+    for (int u = 0; u < kOct; ++u)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) asm volatile("" ::"v"(w[u][q]));
+  }
+  // f(index, value) of the groups j0, j0 + stride, ... < end; the first kOct
+  // have been requested by load(j0, stride)
+  template <typename F>
+  __device__ __forceinline__ void each(int64_t j0, int64_t stride, int64_t end, F f) {
+    for (int64_t j = j0; j < end; j += kOct * stride) {
+      if (j != j0) load(j, stride);
+#pragma unroll
+      for (int u = 0; u < kOct; ++u) {
+        const int64_t ju = j + u * stride;
+        if (ju >= end) continue;
+        const int64_t i = c0 + ju * 8;
+        float v[8];
+        if (fast) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = word_elem<T>(w[u][e / E], e % E);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = to_f32(row[min(i + e, c1 - 1)]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (i + e < c1) f(i + e, v[e]);
+      }
+    }
+  }
+  template <typename F>
+  __device__ __forceinline__ void each(int64_t j0, int64_t stride, F f) {
+    each(j0, stride, n, f);
+  }
+};
+
 // Inclusive scan over the wave.
 template <typename V>
 __device__ __forceinline__ V wave_scan(V v) {
@@ -631,7 +693,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_stats_kernel(SplitArgs a) {
   float bv;
   int64_t bi;
   bool bad;
-  scan_max<T, kSplitNT, 3>((const T*)a.logits + r * a.V + c0, c1 - c0, bv, bi, bad);
+  scan_max<T, kSplitNT, 1>((const T*)a.logits + r * a.V + c0, c1 - c0, bv, bi, bad);
   if (bi != INT64_MAX) bi += c0;
   wave_first_max(bv, bi);
   bad = __any(bad);
@@ -659,13 +721,22 @@ template <typename T>
 __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
   __shared__ unsigned long long lhist[kSplitNB];
   __shared__ unsigned long long part[kSplitNT / kWave];
+  __shared__ uint32_t upart[kSplitNT / kWave];
+  __shared__ int sh_bin;
   const int64_t r = blockIdx.x / kSplitG;
   const int c = blockIdx.x % kSplitG, tid = threadIdx.x;
   SplitRow& w = a.ws[r];
+  const float Tm = a.temperature[r];
+  if (!(Tm > 0.f) && c != 0) return;
+  const T* row = (const T*)a.logits + r * a.V;
+  const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
+  Octets<T, kSplitNT> o(row, a.V, c0, c1);
+  // consecutive elements per thread: thread order is vocabulary order
+  const int64_t seg = (o.n + kSplitNT - 1) / kSplitNT, end = min((tid + 1) * seg, o.n);
+  o.load(tid * seg, 1);                  // in flight with the chunk maxima
   float lmax;
   int64_t imax;
   const bool bad = split_stats(w, lmax, imax);
-  const float Tm = a.temperature[r];
   const float M = lmax / Tm;
   if (bad || !(Tm > 0.f) || !(fabsf(M) < INFINITY)) {
     if (c == 0 && tid == 0) {
@@ -683,27 +754,18 @@ __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
     return;
   }
   const int mode = split_mode(a, r);
-  const T* row = (const T*)a.logits + r * a.V;
-  const bool aligned = ((uintptr_t)row % 16) == 0;
-  const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
   for (int b = tid; b < kSplitNB; b += kSplitNT) lhist[b] = 0;
   __syncthreads();
   unsigned long long sum = 0;
-  for (int64_t i = c0 + tid * 8; i < c1; i += kSplitNT * 8) {
-    float v[8];
-    load8(row, i, c1, aligned, v);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      if (i + e >= c1) continue;
-      const float x = v[e] / Tm;
-      if (mode == kModeTopK)
-        atomicAdd(&lhist[split_bin(x, M)], 1ull);
-      else if (mode == kModeTopP)
-        atomicAdd(&lhist[split_bin(x, M)], mass_fix(x, M));
-      else
-        sum += mass_fix(x, M);
-    }
-  }
+  o.each(tid * seg, 1, end, [&](int64_t, float l) {
+    const float x = l / Tm;
+    if (mode == kModeTopK)
+      atomicAdd(&lhist[split_bin(x, M)], 1ull);
+    else if (mode == kModeTopP)
+      atomicAdd(&lhist[split_bin(x, M)], mass_fix(x, M));
+    else
+      sum += mass_fix(x, M);
+  });
   if (mode == kModeAll) {
     unsigned long long total;
     block_scan<unsigned long long, kSplitNT>(sum, part, total);
@@ -711,8 +773,69 @@ __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
     return;
   }
   __syncthreads();
-  for (int b = tid; b < kSplitNB; b += kSplitNT)
-    if (lhist[b]) atomicAdd(&w.hist[b], lhist[b]);
+  constexpr int kPer = kSplitNB / kSplitNT;
+  if (mode == kModeTopP) {
+    for (int q = tid; q < kSplitNB; q += kSplitNT)
+      if (lhist[q]) atomicAdd(&w.hist[q], lhist[q]);
+    return;
+  }
+  // top-k: what lies past the chunk's own k-th element cannot be among the
+  // row's first k: neither those bins nor those elements are passed on
+  unsigned long long mine = 0, total;
+  for (int q = 0; q < kPer; ++q) mine += lhist[tid * kPer + q];
+  unsigned long long run = block_scan<unsigned long long, kSplitNT>(mine, part, total);
+  const unsigned long long kk = (unsigned long long)a.top_k[r];
+  if (tid == 0 && total < kk) sh_bin = kSplitNB - 1;
+  for (int q = 0; q < kPer; ++q) {
+    const unsigned long long h = lhist[tid * kPer + q];
+    if (h && run < kk) {
+      atomicAdd(&w.hist[tid * kPer + q], h);
+      if (run + h >= kk) sh_bin = tid * kPer + q;
+    }
+    run += h;
+  }
+  __syncthreads();
+  const int bin = sh_bin;
+  uint32_t mine_n = 0, listed;
+  if (seg > kOct) o.load(tid * seg, 1);
+  o.each(tid * seg, 1, end, [&](int64_t, float l) { mine_n += split_bin(l / Tm, M) <= bin; });
+  uint32_t pos = block_scan<uint32_t, kSplitNT>(mine_n, upart, listed);
+  if (mine_n && pos < (uint32_t)kSplitCapC) {
+    if (seg > kOct) o.load(tid * seg, 1);
+    o.each(tid * seg, 1, end, [&](int64_t i, float l) {
+      const float x = l / Tm;
+      if (split_bin(x, M) <= bin) {
+        if (pos < (uint32_t)kSplitCapC) {
+          w.ckey[c * kSplitCapC + pos] = okey(x);
+          w.cidx[c * kSplitCapC + pos] = (uint32_t)i;
+        }
+        ++pos;
+      }
+    });
+  }
+  if (tid == 0) w.lcnt[c] = listed;
+}
+
+// The first bin (from the maximum down) at which the running count or mass
+// reaches `goal`, in sh_bin, and that above it in sh_above; NT threads hold
+// the histogram's bins in order, PER each.
+template <int NT, int PER>
+__device__ __forceinline__ void split_boundary(const unsigned long long (&h)[PER],
+                                               unsigned long long run, unsigned long long mine,
+                                               unsigned long long goal, int* sh_bin,
+                                               unsigned long long* sh_above) {
+  if (run < goal && goal <= run + mine) {
+    bool found = false;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      if (!found && goal <= run + h[q]) {
+        found = true;
+        *sh_bin = threadIdx.x * PER + q;
+        *sh_above = run;
+      }
+      run += h[q];
+    }
+  }
 }
 
 template <typename T>
@@ -724,77 +847,65 @@ __global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
   const int64_t r = blockIdx.x / kSplitG;
   const int c = blockIdx.x % kSplitG, tid = threadIdx.x;
   SplitRow& w = a.ws[r];
-  float lmax;
-  int64_t imax;
-  const bool bad = split_stats(w, lmax, imax);
   const float Tm = a.temperature[r];
-  const float M = lmax / Tm;
   const int mode = split_mode(a, r);
-  if (bad || !(Tm > 0.f) || !(fabsf(M) < INFINITY) || mode == kModeAll) return;
-
-  // the first bin (from the maximum down) at which the running count reaches
-  // k, or the running mass the target
+  if (!(Tm > 0.f) || mode == kModeAll) return;
+  if (mode == kModeTopK && !__any(w.lcnt[tid % kSplitG] > (uint32_t)kSplitCapC)) return;
+  // the chunk, the histogram and the chunk maxima in one round trip. A thread
+  // holds consecutive elements, so that thread order is vocabulary order
+  const T* row = (const T*)a.logits + r * a.V;
+  const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
+  Octets<T, kSplitNT> o(row, a.V, c0, c1);
+  const int64_t seg = (o.n + kSplitNT - 1) / kSplitNT;
+  o.load(tid * seg, 1);
   constexpr int kPer = kSplitNB / kSplitNT;
   unsigned long long h[kPer], mine = 0, total;
 #pragma unroll
   for (int q = 0; q < kPer; ++q) h[q] = w.hist[tid * kPer + q];
 #pragma unroll
+  for (int q = 0; q < kPer; ++q) asm volatile("" ::"v"(h[q]));
+  float lmax;
+  int64_t imax;
+  const bool bad = split_stats(w, lmax, imax);
+  const float M = lmax / Tm;
+  if (bad || !(fabsf(M) < INFINITY)) return;
+
+#pragma unroll
   for (int q = 0; q < kPer; ++q) mine += h[q];
-  unsigned long long run = block_scan<unsigned long long, kSplitNT>(mine, part, total);
+  const unsigned long long run = block_scan<unsigned long long, kSplitNT>(mine, part, total);
   const unsigned long long goal =
       mode == kModeTopK
           ? (unsigned long long)a.top_k[r]
           : max(1ull, (unsigned long long)(fmax((double)a.top_p[r], 0.0) * (double)total));
-  if (run < goal && goal <= run + mine) {
-    bool found = false;
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-      if (!found && goal <= run + h[q]) {
-        found = true;
-        sh_bin = tid * kPer + q;
-        sh_above = run;
-      }
-      run += h[q];
-    }
-  }
+  split_boundary<kSplitNT, kPer>(h, run, mine, goal, &sh_bin, &sh_above);
   __syncthreads();
   const int bin = sh_bin;
 
-  const T* row = (const T*)a.logits + r * a.V;
-  const bool aligned = ((uintptr_t)row % 16) == 0;
-  const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
   unsigned long long hard = 0;
-  uint32_t listed = 0;
-  for (int64_t t0 = c0; t0 < c1; t0 += kSplitNT * 8) {
-    const int64_t i = t0 + tid * 8;
-    float x[8];
-    uint32_t sel = 0;
-    if (i < c1) {
-      load8(row, i, c1, aligned, x);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        x[e] = x[e] / Tm;
-        if (i + e >= c1) continue;
-        const int b = split_bin(x[e], M);
-        if (b == bin || (mode == kModeTopK && b < bin))
-          sel |= 1u << e;
-        else if (b < bin)
-          hard += mass_fix(x[e], M);
-      }
-    }
-    uint32_t tile;
-    uint32_t pos =
-        listed + block_scan<uint32_t, kSplitNT>((uint32_t)__popc(sel), upart, tile);
-    listed += tile;
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-      if (sel >> e & 1) {
+  uint32_t mine_n = 0, listed;
+  const int64_t end = min((tid + 1) * seg, o.n);
+  o.each(tid * seg, 1, end, [&](int64_t, float l) {
+    const float x = l / Tm;
+    const int b = split_bin(x, M);
+    if (b == bin || (mode == kModeTopK && b < bin))
+      ++mine_n;
+    else if (b < bin)
+      hard += mass_fix(x, M);
+  });
+  uint32_t pos = block_scan<uint32_t, kSplitNT>(mine_n, upart, listed);
+  if (mine_n && pos < (uint32_t)kSplitCapC) {    // (few threads: the chunk is read again)
+    o.load(tid * seg, 1);
+    o.each(tid * seg, 1, end, [&](int64_t i, float l) {
+      const float x = l / Tm;
+      const int b = split_bin(x, M);
+      if (b == bin || (mode == kModeTopK && b < bin)) {
         if (pos < (uint32_t)kSplitCapC) {
-          w.ckey[c * kSplitCapC + pos] = okey(x[e]);
-          w.cidx[c * kSplitCapC + pos] = (uint32_t)(i + e);
+          w.ckey[c * kSplitCapC + pos] = okey(x);
+          w.cidx[c * kSplitCapC + pos] = (uint32_t)i;
         }
         ++pos;
       }
+    });
   }
   unsigned long long hsum;
   block_scan<unsigned long long, kSplitNT>(hard, part, hsum);
@@ -814,31 +925,78 @@ __global__ __launch_bounds__(kNT) void sample_pick_kernel(SplitArgs a) {
   __shared__ unsigned long long sw[kSplitCap];
   __shared__ unsigned long long part[kNT / kWave];
   __shared__ unsigned long long cm[kSplitG];          // kept mass per chunk
-  __shared__ uint32_t off[kSplitG + 1];
-  __shared__ unsigned long long sh_zk, sh_low, sh_z, sh_rem;
-  __shared__ int sh_over, sh_chunk;
+  __shared__ uint32_t cnt[kSplitG], off[kSplitG + 1];
+  __shared__ unsigned long long sh_zk, sh_low, sh_z, sh_rem, sh_above;
+  __shared__ int sh_over, sh_chunk, sh_bin;
   const int64_t r = blockIdx.x;
   const int tid = threadIdx.x, lane = tid % kWave;
   SplitRow& w = a.ws[r];
+  const float Tm = a.temperature[r];
+  if (!(Tm > 0.f)) return;                            // written by `hist`
+  // every slot of the lists (the unused ones hold anything), the counts and
+  // the chunk maxima in one round trip
+  constexpr int kSlots = kSplitG * kSplitCapC / kNT;
+  uint32_t lk[kSlots], li[kSlots];
+#pragma unroll
+  for (int u = 0; u < kSlots; ++u) {
+    lk[u] = w.ckey[u * kNT + tid];
+    li[u] = w.cidx[u * kNT + tid];
+  }
+  constexpr int kPer = kSplitNB / kNT;
+  unsigned long long h[kPer];                         // (top-k: the boundary bin again)
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) h[q] = w.hist[tid * kPer + q];
+  const uint32_t llist = w.lcnt[lane % kSplitG];
+  const uint32_t clist = w.ccnt[lane % kSplitG];
+  const unsigned long long lhard = w.hard[lane % kSplitG];
+#pragma unroll
+  for (int u = 0; u < kSlots; ++u) asm volatile("" ::"v"(lk[u]), "v"(li[u]));
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) asm volatile("" ::"v"(h[q]));
+  asm volatile("" ::"v"(llist), "v"(clist), "v"(lhard));
   float lmax;
   int64_t imax;
   const bool bad = split_stats(w, lmax, imax);
-  const float Tm = a.temperature[r];
   const float M = lmax / Tm;
-  if (bad || !(Tm > 0.f)) return;                     // written by `hist`
+  if (bad) return;                                    // written by `hist`
   const int mode = split_mode(a, r);
   const int64_t kk = a.top_k[r];
   const float pp = a.top_p[r];
   const int64_t chunk = split_chunk(a.V);
   const bool whole = !(fabsf(M) < INFINITY);
 
+  // the lists' lengths: top-k, those of `hist` unless one overflowed
+  const bool again = mode == kModeTopK && __any(llist > (uint32_t)kSplitCapC);
+  const uint32_t lcnt = mode == kModeTopK && !again ? llist : clist;
+  const bool over = mode != kModeAll && __any(lcnt > (uint32_t)kSplitCapC);
+  int bin = kSplitNB;                                 // elements past it are not on the boundary
+  if (mode == kModeTopK && !whole) {
+    unsigned long long mine = 0, total;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) mine += h[q];
+    const unsigned long long run = block_scan<unsigned long long, kNT>(mine, part, total);
+    split_boundary<kNT, kPer>(h, run, mine, (unsigned long long)kk, &sh_bin, &sh_above);
+    __syncthreads();
+    bin = sh_bin;
+  }
+  // compacted in slot order, which is vocabulary order: a wave holds one
+  // chunk's list (kSplitCapC slots) per round
+  static_assert(kSplitCapC == kWave && kSlots * kNT == kSplitG * kSplitCapC, "a wave per list");
+  uint64_t sel[kSlots];
+#pragma unroll
+  for (int u = 0; u < kSlots; ++u) {
+    const int c = u * (kNT / kWave) + tid / kWave;
+    sel[u] = __ballot(mode != kModeAll && !whole && (uint32_t)lane < __shfl(lcnt, c) &&
+                      split_bin(key_float(lk[u]), M) <= bin);
+    if (lane == 0) cnt[c] = (uint32_t)__popcll(sel[u]);
+  }
+  __syncthreads();
   if (tid < kWave) {                                  // wave 0: the lists' offsets
-    const uint32_t n = lane < kSplitG && mode != kModeAll && !whole ? w.ccnt[lane] : 0u;
-    const bool over = __any(n > (uint32_t)kSplitCapC);
+    const uint32_t n = lane < kSplitG ? cnt[lane] : 0u;
     const uint32_t incl = wave_scan(n);
     if (lane < kSplitG) {
       off[lane + 1] = incl;
-      cm[lane] = mode == kModeTopK ? 0 : w.hard[lane];
+      cm[lane] = mode == kModeTopK ? 0 : lhard;
     }
     if (lane == 0) {
       off[0] = 0;
@@ -855,11 +1013,13 @@ __global__ __launch_bounds__(kNT) void sample_pick_kernel(SplitArgs a) {
     return;
   }
   const int n = (int)off[kSplitG];
-  for (int s = tid; s < kSplitG * kSplitCapC; s += kNT) {
-    const int c = s / kSplitCapC, j = s % kSplitCapC;
-    if (j < (int)(off[c + 1] - off[c])) {
-      skey[off[c] + j] = w.ckey[s];
-      sidx[off[c] + j] = w.cidx[s];
+#pragma unroll
+  for (int u = 0; u < kSlots; ++u) {
+    const int c = u * (kNT / kWave) + tid / kWave;
+    if (sel[u] >> lane & 1) {
+      const uint32_t at = off[c] + __popcll(sel[u] & (((uint64_t)1 << lane) - 1));
+      skey[at] = lk[u];
+      sidx[at] = li[u];
     }
   }
   __syncthreads();

@@ -181,7 +181,8 @@ def test_split_rows_equal_one_workgroup_rows(dtype, V):
     handed to the one-workgroup form), few distinct values (ties across
     chunks), a tie group of the maximum, zeros of both signs, a maximum in the
     last element, an infinity. Options: each of top-k and top-p alone,
-    together, neither, a top-k past the lists, greedy, a tiny top-p."""
+    together, neither, a top-k past the lists (of the row, of a chunk), greedy, a
+    tiny top-p."""
     from acorninfer_amd._lib import check, dtype_code, lib, ptr, stream_ptr
     from acorninfer_amd.sampler import sample_batch, sample_workspace
     g = torch.Generator().manual_seed(V)
@@ -196,7 +197,7 @@ def test_split_rows_equal_one_workgroup_rows(dtype, V):
     x[6, V - 1] = 30.0
     x[7, V // 2] = float("inf")
     options = [(0.7, 20, 0.95), (1.0, 0, 0.9), (0.6, 50, 1.0), (1.0, 0, 1.0), (0.9, 5000, 0.8),
-               (0.0, 0, 1.0), (1.0, 1, 1.0), (1.2, 0, 1e-6), (0.8, V, 0.5)]
+               (0.0, 0, 1.0), (1.0, 1, 1.0), (1.2, 0, 1e-6), (0.8, V, 0.5), (1.1, 100, 0.9)]
     rows = x.repeat_interleave(len(options), 0).to(dtype).cuda()
     opts = options * x.shape[0]
     B = rows.shape[0]
