@@ -509,6 +509,186 @@ __global__ __launch_bounds__(NW * 64, 1) void dense_dl_kernel(const __bf16* __re
   }
 }
 
+// The direct-to-LDS form on int8 weights in the W8B layout (bytes q + 128; a
+// 1 KB block is 16 rows x 64 k, one pair of stages of a 16-row block). The
+// bytes go to LDS as they are, half the bf16 form's weight traffic, and become
+// exact bf16 integers when a wave reads them as operands; the fp16 row scale
+// multiplies the finished fp32 sums. At prefill sizes int8 ran on the 128 x 128
+// tiled kernel at 0.5-0.6 PFLOP/s (M = 3000: gate|up 1250 us); the alternative,
+// a bf16 copy of the weights first, moves 5 bytes per weight more than this.
+// Everything not said here is dense_dl_kernel's.
+//  * lane 16 r + c of an A block holds row c's bytes of k 16 r .. 16 r + 15, so
+//    stage half h multiplies k 16 r + 8 h .. + 7: the x operand of half h is
+//    row piece 2 r + h (of 8 k) instead of 4 h + r;
+//  * a pair's blocks are read whole (one 16-byte read per block and lane): in
+//    stage 2 d + 1, behind the barrier that follows pair d + 1, block i is
+//    refilled for both halves of the next pair after its own last use;
+//  * 8 bytes become an operand in 14 VALU instructions (xor, signed byte
+//    conversions, packs) beside the 4 MFMAs it feeds.
+template <typename OUT, bool SWIGLU>
+__global__ __launch_bounds__(512, 1) void dense_dl8_kernel(const __bf16* __restrict__ x,
+                                                           const uint8_t* __restrict__ w,
+                                                           const _Float16* __restrict__ scale,
+                                                           OUT* __restrict__ out, int M, int N,
+                                                           int K, int tiles_n, int tiles_m,
+                                                           int steps) {
+  constexpr int T = kLdsTile, NW = 8;
+  constexpr int NB = 8, MB = 32 / NW;          // wave tile 128 x 16 MB
+  constexpr int LPX = 32 / NW, LPA = 16 / NW;  // 1 KB loads per wave per pair: x, weights
+  constexpr int XPAIR = 2 * kDlOpBytes;        // x: 256 rows x 128 B
+  constexpr int WPAIR = kDlOpBytes;            // weights: 16 blocks of 1 KB
+  __shared__ __align__(1024) uint8_t lds[2][WPAIR + XPAIR];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane >> 4, c = lane & 15;
+  const int G = tiles_n * tiles_m;
+  int t = blockIdx.x;
+  if (G % 8 == 0) t = (t % 8) * (G / 8) + t / 8;
+  constexpr int GN = 4;
+  const int group = t / (GN * tiles_m);
+  const int first_n = group * GN;
+  const int gsize = min(tiles_n - first_n, GN);
+  const int in_group = t - group * GN * tiles_m;
+  const int tn = first_n + in_group % gsize;
+  const int tm = in_group / gsize;
+  const int n0 = tn * T, m0 = tm * T;
+  const int wn = (wid & 1) * 128, wm = (wid >> 1) * 16 * MB;
+  const int kbase = blockIdx.y * steps * kDlBK;
+  out += (size_t)blockIdx.y * M * N;
+
+  const uint8_t* wsrc[LPA];
+  const uint8_t* xsrc[LPX];
+#pragma unroll
+  for (int j = 0; j < LPA; ++j)
+    wsrc[j] = w + ((size_t)min(n0 / 16 + LPA * wid + j, N / 16 - 1) * (K / 64) + kbase / 64) * 1024 +
+              16 * lane;
+#pragma unroll
+  for (int j = 0; j < LPX; ++j) {
+    const int row = 8 * (LPX * wid + j) + (lane >> 3);
+    const int piece = (lane & 7) ^ ((row >> 1) & 7);
+    xsrc[j] = (const uint8_t*)(x + (size_t)min(m0 + row, M - 1) * K + kbase + 8 * piece);
+  }
+  const uint32_t aoff = (uint32_t)(wn / 16 * 1024 + 16 * lane);
+  const uint32_t boff0 = (uint32_t)(WPAIR + (wm + c) * 128 + 16 * ((2 * r) ^ (c >> 1)));
+  const uint32_t boff1 = (uint32_t)(WPAIR + (wm + c) * 128 + 16 * ((2 * r + 1) ^ (c >> 1)));
+
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)(&lds[0][0]);
+  auto dma = [&](const uint8_t* src, uint32_t dst) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                 :: "v"(src), "s"(dst) : "memory", "m0");
+#pragma clang diagnostic pop
+  };
+  const int pairs = steps / 2;
+  auto issue_one = [&](int d, int i) {         // load i of pair d: weights, then x
+    const size_t dd = (size_t)min(d, pairs - 1);
+    const uint32_t base = lds0 + (uint32_t)((d & 1) * (WPAIR + XPAIR));
+    if (i < LPA)
+      dma(wsrc[i] + dd * 1024, base + (uint32_t)((LPA * wid + i) * 1024));
+    else
+      dma(xsrc[i - LPA] + dd * 128, base + (uint32_t)(WPAIR + (LPX * wid + i - LPA) * 1024));
+  };
+  auto opA = [&](int d, int i) {
+    return *(const u32x4*)(&lds[d & 1][aoff + 1024 * i]);
+  };
+  auto opB = [&](int s, int j) {
+    return *(const u32x4*)(&lds[(s >> 1) & 1][((s & 1) ? boff1 : boff0) + 2048 * j]);
+  };
+
+  f32x4 acc[NB][MB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < MB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 a[NB], b0[MB], b1[MB];                 // a: both halves of the pair's bytes
+  auto stage = [&](int s, const u32x4 (&bc)[MB], u32x4 (&bn)[MB], int dq) {
+#pragma unroll
+    for (int j = 0; j < MB; ++j) bn[j] = opB(s + 1, j);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int h = s & 1;
+      const u32x4 av = unpack_w8s(a[i][2 * h], a[i][2 * h + 1]);
+#pragma unroll
+      for (int j = 0; j < MB; ++j) acc[i][j] = mfma(av, bc[j], acc[i][j]);
+      if (h) a[i] = opA((s + 1) >> 1, i);
+      if (dq >= 0 && i < LPA + LPX) issue_one(dq, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+#define ACORN_DL_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (((n) >> 4) << 14) | (7 << 4) | (15 << 8))
+  constexpr int LPS = LPA + LPX;
+#pragma unroll
+  for (int i = 0; i < LPS; ++i) issue_one(0, i);
+#pragma unroll
+  for (int i = 0; i < LPS; ++i) issue_one(1, i);
+  ACORN_DL_VMCNT(LPS);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NB; ++i) a[i] = opA(0, i);
+#pragma unroll
+  for (int j = 0; j < MB; ++j) b0[j] = opB(0, j);
+  for (int d = 0; d < pairs; ++d) {
+    stage(2 * d, b0, b1, -1);
+    ACORN_DL_VMCNT(0);
+    __syncthreads();
+    stage(2 * d + 1, b1, b0, d + 2);
+  }
+#undef ACORN_DL_VMCNT
+  __builtin_amdgcn_s_waitcnt(0);      // no LDS write of this wave outlives it
+
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int n = min(n0 + wn + 16 * i + 4 * r, N - 4);
+    const h16x4 sc = *(const h16x4*)(scale + n);
+#pragma unroll
+    for (int j = 0; j < MB; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][j][e] *= (float)sc[e];
+  }
+  if constexpr (SWIGLU) {
+#pragma unroll
+    for (int j = 0; j < MB; ++j) {
+      const int m = m0 + wm + 16 * j + c;
+      if (m >= M) continue;
+#pragma unroll
+      for (int q = 0; q < NB / 2; ++q) {
+        const int nb = n0 + wn + 32 * q;
+        if (nb >= N) continue;
+        const f32x4 g = acc[2 * q][j], u = acc[2 * q + 1][j];
+        u32x2 v;
+        v[0] = pack_bf16x2(swiglu_bf16(g[0], u[0]), swiglu_bf16(g[1], u[1]));
+        v[1] = pack_bf16x2(swiglu_bf16(g[2], u[2]), swiglu_bf16(g[3], u[3]));
+        *(u32x2*)(out + (size_t)m * (N / 2) + nb / 2 + 4 * r) = v;
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < MB; ++j) {
+    const int m = m0 + wm + 16 * j + c;
+    if (m >= M) continue;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const int n = n0 + wn + 16 * i + 4 * r;
+      if (n >= N) continue;
+      OUT* o = out + (size_t)m * N + n;
+      if constexpr (sizeof(OUT) == 4) {
+        *(f32x4*)o = acc[i][j];
+      } else {
+        u32x2 v;
+        v[0] = pack_bf16x2(acc[i][j][0], acc[i][j][1]);
+        v[1] = pack_bf16x2(acc[i][j][2], acc[i][j][3]);
+        *(u32x2*)o = v;
+      }
+    }
+  }
+}
+
 template <typename OUT, int NW, bool SWIGLU, bool BLK>
 int launch_dl(const void* x, const void* w, void* out, int64_t M, int64_t N, int64_t K, int ks,
               hipStream_t st) {
@@ -604,6 +784,32 @@ int dense_gemm_swiglu_launch(const void* x, const void* w, void* act, int64_t M,
   if (!dense_gemm_swiglu_supported(N, K, wn, bm, depth, blocked)) return ACORN_ERR_UNSUPPORTED;
   return blocked ? launch_dl<__bf16, 8, true, true>(x, w, act, M, N, K, 1, st)
                  : launch_dl<__bf16, 8, true, false>(x, w, act, M, N, K, 1, st);
+}
+
+bool dense_gemm8_supported(int64_t N, int64_t K, int ks, bool swiglu) {
+  return N % (swiglu ? 32 : 16) == 0 && K % 64 == 0 && ks >= 1 && ks <= 64 &&
+         (K / kDlBK) % (2 * ks) == 0 && !(swiglu && ks != 1);
+}
+
+int dense_gemm8_launch(const void* x, const void* w, const void* scale, void* out_bf16,
+                       float* out_f32, int64_t M, int64_t N, int64_t K, int ks, bool swiglu,
+                       hipStream_t st) {
+  if (!dense_gemm8_supported(N, K, ks, swiglu)) return ACORN_ERR_UNSUPPORTED;
+  if (!out_f32 && ks != 1) return ACORN_ERR_VALUE;
+  const int64_t tiles_n = (N + kLdsTile - 1) / kLdsTile, tiles_m = (M + kLdsTile - 1) / kLdsTile;
+  if (tiles_n * tiles_m > 0x7fffffff) return ACORN_ERR_SHAPE;
+  const dim3 grid((unsigned)(tiles_n * tiles_m), (unsigned)ks), block(512);
+  const int tn = (int)tiles_n, tm = (int)tiles_m, steps = (int)(K / kDlBK / ks);
+  const __bf16* xp = (const __bf16*)x;
+  const uint8_t* wp = (const uint8_t*)w;
+  const _Float16* sp = (const _Float16*)scale;
+  if (out_f32)
+    dense_dl8_kernel<float, false><<<grid, block, 0, st>>>(xp, wp, sp, out_f32, (int)M, (int)N, (int)K, tn, tm, steps);
+  else if (swiglu)
+    dense_dl8_kernel<__bf16, true><<<grid, block, 0, st>>>(xp, wp, sp, (__bf16*)out_bf16, (int)M, (int)N, (int)K, tn, tm, steps);
+  else
+    dense_dl8_kernel<__bf16, false><<<grid, block, 0, st>>>(xp, wp, sp, (__bf16*)out_bf16, (int)M, (int)N, (int)K, tn, tm, steps);
+  return ACORN_OK;
 }
 
 }  // namespace acorn

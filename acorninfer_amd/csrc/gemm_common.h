@@ -90,6 +90,19 @@ __device__ __forceinline__ float fma_half(const uint32_t (&d)[NDW], int h, float
   return __builtin_fmaf((float)s, v, acc);
 }
 
+// Eight W8B bytes (q + 128) as a bf16 MFMA operand of the integers q, exact:
+// signed byte conversions (14 VALU instructions).
+__device__ __forceinline__ u32x4 unpack_w8s(uint32_t w0, uint32_t w1) {
+  u32x4 v;
+  const uint32_t w[2] = {w0 ^ 0x80808080u, w1 ^ 0x80808080u};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    v[2 * i] = pack_bf16x2((float)(int8_t)(w[i] & 0xffu), (float)(int8_t)((w[i] >> 8) & 0xffu));
+    v[2 * i + 1] = pack_bf16x2((float)(int8_t)((w[i] >> 16) & 0xffu), (float)(int8_t)(w[i] >> 24));
+  }
+  return v;
+}
+
 // SwiGLU epilogue of the fused gate|up projection: g, u rounded to bf16,
 // act = round(round(silu(g)) * u), silu(g) = g / (1 + exp(-g)) in fp32
 // (models/qwen3.py:392-396, each torch bf16 op rounded).
@@ -369,5 +382,11 @@ int dense_gemm_swiglu_launch(const void* x, const void* w, void* act, int64_t M,
 int dense_gemm_launch(const void* x, const void* w, void* out_bf16, float* out_f32, int64_t M,
                       int64_t N, int64_t K, int wn, int bm, int depth, int ks, bool blocked,
                       hipStream_t st);
+// The same 256 x 256 direct-to-LDS form on W8B weights (fp16 row scales applied
+// to the fp32 sums); swiglu as above (one split).
+bool dense_gemm8_supported(int64_t N, int64_t K, int ks, bool swiglu);
+int dense_gemm8_launch(const void* x, const void* w, const void* scale, void* out_bf16,
+                       float* out_f32, int64_t M, int64_t N, int64_t K, int ks, bool swiglu,
+                       hipStream_t st);
 
 }  // namespace acorn

@@ -755,7 +755,8 @@ struct Tiling {
                                  //     per wave, nw = waves, tpw = groups in flight),
                                  // 5 = W8B decode kernel (tpw = its pipeline depth),
                                  // 6 = BF16B decode kernel (tpw = its pipeline depth),
-                                 // 7 = W8B mid-M kernel (as 4, tpw = steps in flight)
+                                 // 7 = W8B mid-M kernel (as 4, tpw = steps in flight),
+                                 // 8 = large-M kernel on W8B weights (as 3)
   W4bPlan w4b;
   DirectPlan w8b;
   DirectPlan bf16b;
@@ -800,6 +801,21 @@ size_t lds_bytes(int wfmt, int mt, int R, int rt, int nw, int KR, int upw) {
 // weight bytes.
 int make_tile_plan(int64_t M, int64_t N, int64_t K, int wfmt, int req_bm, int req_bn,
                    int req_ks, Tiling* t) {
+  // bf16 with nothing requested, but small weights at few rows: 128-row weight
+  // tiles (whole-line loads, half the x re-reads of 64) and one round of
+  // workgroups in powers of two. 64 rows, qkv / o / gate|up / down of an 8B
+  // layer, 64-row tiles towards two workgroups per CU 34 / 25 / 70 / 40 us, this
+  // rule 21 / 19 / 44 / 30; 160 rows 41 / 31 / 100 / 55 and 38 / 27 / 97 / 54.
+  // The weights of a 0.6B layer at 17 and 64 rows are 5-20% faster in 64-row tiles.
+  if ((wfmt == ACORN_WFMT_BF16 || wfmt == ACORN_WFMT_BF16B) && !req_bm && !req_bn && !req_ks &&
+      M > 16 && N % 128 == 0 && K % 64 == 0 && (M > 64 || N * K >= ((int64_t)8 << 20))) {
+    int64_t bm = M <= 32 ? 32 : M <= 128 ? 64 : 128;
+    if (bm == 64 && N / 128 * ((M + 63) / 64) > kCUs) bm = 128;
+    const int64_t tiles = N / 128 * ((M + bm - 1) / bm);
+    int ks = 1;
+    while (tiles * ks * 2 <= kCUs && ks < 8 && K % (128 * ks) == 0) ks *= 2;
+    return make_tile_plan(M, N, K, wfmt, (int)bm, 128, ks, t);
+  }
   const int bn = (req_bn == 64 || req_bn == 128) ? req_bn : M <= 64 ? 64 : 128;
   if (N % bn) return ACORN_ERR_UNSUPPORTED;
   const int bk = kTileKN / bn;
@@ -869,6 +885,100 @@ constexpr int64_t kDenseLdsM = 512;
 // W4B above 16 rows on request (rt == kMidRT): the mid-M int4 kernel
 constexpr int kMidRT = -3;
 
+// K splits that stay within one round of the CUs: the mid-M kernels' 256 x 64
+// tiles, and the large-M W8B kernel's 256 x 256 ones.
+int mid_splits(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = N / 256 * ((M + 63) / 64);
+  int ks = 1;
+  while (tiles * ks * 2 <= kCUs && ks < 8 && K % (512 * ks) == 0) ks *= 2;
+  return ks;
+}
+int dense8_splits(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = (N + 255) / 256 * ((M + 255) / 256);
+  int ks = 1;
+  while (tiles * 2 * ks <= kCUs && ks < 16 && dense_gemm8_supported(N, K, 2 * ks, false)) ks *= 2;
+  return ks;
+}
+// W8B from 256 rows: the large-M kernel or the mid-M one. Both run in whole
+// rounds of the 256 CUs, 37 us per 4096 k for a round of 256 x 64 tiles and 111
+// for one of 256 x 256, plus the split planes at 5 TB/s, written and read; the
+// smaller tile wins where the larger leaves a good part of a round empty (by
+// 10%: in one split the larger can write its consumer's bf16 input). This
+// predicts the measured times within 10%: 1000 rows, mid / large, qkv 74 / 77
+// us, o 40 / 56, gate|up 236 / 225, down 112 / 109; gate|up at 700 rows 186 /
+// 218, at 2000 477 / 361.
+bool dense8_faster(int64_t M, int64_t N, int64_t K) {
+  if (M < 256) return false;
+  if (N % 256 || K % 512) return true;      // no mid-M form
+  auto us = [&](int64_t tiles, int ks, double round) {
+    return (double)((tiles * ks + kCUs - 1) / kCUs) / ks * round * (double)K / 4096.0 +
+           (ks > 1 ? 8.0 * ks * (double)M * (double)N / 5e6 : 0.0);
+  };
+  return us((N + 255) / 256 * ((M + 255) / 256), dense8_splits(M, N, K), 111.0) <
+         1.1 * us(N / 256 * ((M + 63) / 64), mid_splits(M, N, K), 37.0);
+}
+
+// The tiling of a block-layout launch with nothing requested, from a sweep of
+// every tiling over the projections of an 8B and a 0.6B layer; false leaves the
+// choice to the kernel's own planner (shapes the sizes below do not divide).
+//
+// Up to 16 rows one split wins everywhere: K slices inside a workgroup (22, 44)
+// give a projection of few row tiles its waves without the fp32 partials and
+// the second launch that adds them, and let the RMSNorms fold into o and down
+// (one split only). From about 1000 row tiles the waves are there without
+// slices. us at 8 rows, splitting K to 768 waves / this rule (8B): int4 qkv
+// 7.9 / 6.1, o 8.5 / 5.3, gate|up 13.2 / 13.0, down 11.1 / 10.2; int8 9.1 / 7.1,
+// 9.3 / 5.8, 19.5 / 19.1, 13.5 / 12.1; bf16 11.8 / 11.2, 9.9 / 7.5, 33.8 / 32.4,
+// 21.1 / 18.3. (int4 and int8 down at 16 rows are 6-10% slower than split, and
+// gain more than that back as the folded norm.)
+// Above, int4 up to 24 rows stages x once (11.0 against 11.6 us for qkv); the
+// rest runs on the mid-M kernels with 256-row workgroups and as many splits as
+// stay within one round of the CUs: int4 at 64 rows, tiled / mid-M, 21 / 15, 20
+// / 13, 42 / 31, 29 / 23 us, at 1000 rows 92 / 79, 60 / 42, 348 / 241, 182 / 120.
+// Launches of few workgroups (a 0.6B down) stay on the tiled kernel at few rows.
+bool default_request(int64_t M, int64_t N, int64_t K, int wfmt, bool swiglu, int* d) {
+  const int64_t nt = N / 16;
+  const int ku = wfmt == ACORN_WFMT_W4B ? 128 : wfmt == ACORN_WFMT_W8B ? 64 : 32;
+  for (int i = 0; i < 5; ++i) d[i] = 0;
+  if (M <= 16) {
+    const bool many = nt >= 1024;
+    const int rt = nt >= 384 && nt % 2 == 0 ? 2 : 1;
+    if (swiglu && rt != 2) return false;
+    if (wfmt == ACORN_WFMT_W4B) {
+      const int kw = many ? 2 : 4;
+      const int64_t st = K / 128 / (2 * kw);          // stages of two groups per slice
+      const int depth = M <= 8 && rt == 1 && st % 4 == 0 ? 4 : st % 2 == 0 ? 2 : 1;
+      if (K % (256 * kw)) return false;
+      d[0] = rt; d[1] = 2; d[2] = 11 * kw; d[3] = 1; d[4] = depth;
+    } else if (wfmt == ACORN_WFMT_W8B) {
+      const int kw = many ? 1 : 4;
+      const int64_t st = K / 64 / kw;
+      if (K % (64 * kw * 4)) return false;
+      d[0] = rt; d[1] = 1; d[2] = many ? 1 : 44; d[3] = 1; d[4] = rt == 1 && st % 8 == 0 ? 8 : 4;
+    } else {
+      const int kw = many ? 1 : 4;
+      if (K % (64 * kw * 4)) return false;
+      d[0] = rt; d[1] = 2; d[2] = many ? 1 : 44; d[3] = 1; d[4] = K % (64 * kw * 8) ? 4 : 8;
+      if (many && swiglu) { d[1] = 4; d[4] = 4; }
+      if (many && !swiglu) { d[0] = M <= 8 ? 1 : 2; d[1] = M <= 8 ? 2 : 1; }
+    }
+    // few waves, and K left to split: the kernel's own planner
+    const int kw = d[2] < 10 ? 1 : d[2] % 10;
+    return swiglu || nt / d[0] * kw >= 3 * kCUs || K / ku == (int64_t)kw * d[1] * d[4];
+  }
+  if (swiglu || (wfmt != ACORN_WFMT_W4B && wfmt != ACORN_WFMT_W8B) || N % 64) return false;
+  const bool w4 = wfmt == ACORN_WFMT_W4B;
+  if (w4 && M <= 24 && K % 1024 == 0) {
+    d[0] = 4; d[1] = 1; d[2] = 4; d[3] = 8; d[4] = 2;
+    return true;
+  }
+  if (N % 256 || K % 512) return false;
+  const int ks = mid_splits(M, N, K);
+  if (N / 256 * ((M + 63) / 64) * ks < kCUs / 4 && M <= (w4 ? 32 : 64)) return false;
+  d[0] = kMidRT; d[1] = 2; d[2] = 8; d[3] = ks; d[4] = 2;
+  return true;
+}
+
 int make_plan(int64_t M, int64_t N, int64_t K, int wfmt, const int* cfg, Tiling* t,
               bool swiglu = false) {
   if (M <= 0 || N <= 0 || K <= 0) return ACORN_ERR_SHAPE;
@@ -880,6 +990,41 @@ int make_plan(int64_t M, int64_t N, int64_t K, int wfmt, const int* cfg, Tiling*
   t->kind = 0;
   const bool no_request = !cfg || (cfg[0] == 0 && cfg[1] == 0 && cfg[2] == 0 && cfg[3] <= 1 &&
                                    cfg[4] == 0);
+  const bool req8 = cfg && cfg[0] == kDenseRT;
+  if (wfmt == ACORN_WFMT_W8B &&
+      (req8 || (no_request && (swiglu ? M >= kDenseLdsM : N % 128 == 0 && dense8_faster(M, N, K))))) {
+    const int64_t tiles = (N + 255) / 256 * ((M + 255) / 256);
+    const int ks = req8 && cfg[3] > 0 ? cfg[3] : swiglu ? 1 : dense8_splits(M, N, K);
+    const bool form = !req8 || ((cfg[1] == 0 || cfg[1] == 256) && (cfg[2] == 0 || cfg[2] == 128) &&
+                               (cfg[4] == 0 || cfg[4] == 4));
+    if (form && dense_gemm8_supported(N, K, ks, swiglu)) {
+      t->kind = 8;
+      t->rt = kDenseRT;
+      t->upw = 256;
+      t->nw = 128;
+      t->ksplit = ks;
+      t->tpw = 4;
+      t->mt = 1;
+      t->R = 256;
+      t->nk = (int)(K / 64);
+      t->ntiles = (int)((N + 255) / 256);
+      t->mblocks = (int)((M + 255) / 256);
+      t->groups = 1;
+      t->lds = 0;
+      return tiles > 0x7fffffff ? ACORN_ERR_SHAPE : ACORN_OK;
+    }
+    if (req8) return ACORN_ERR_UNSUPPORTED;
+  }
+  if ((!cfg || (!cfg[0] && !cfg[1] && !cfg[2] && !cfg[3] && !cfg[4])) &&
+      (wfmt == ACORN_WFMT_W4B || wfmt == ACORN_WFMT_W8B ||
+       (wfmt == ACORN_WFMT_BF16B && M <= 16))) {
+    int d[5];
+    if (default_request(M, N, K, wfmt, swiglu, d) &&
+        make_plan(M, N, K, wfmt, d, t, swiglu) == ACORN_OK)
+      return ACORN_OK;
+    t->swiglu = swiglu;
+    t->kind = 0;
+  }
   // the SwiGLU epilogue is built into the direct-to-LDS form only (from
   // kDenseLdsM rows, or on request)
   const bool blocked = wfmt == ACORN_WFMT_BF16B;
@@ -1276,6 +1421,10 @@ int gemm_entry(const void* x, const void* w, const void* scale, const void* zero
     rc = t.swiglu ? dense_gemm_swiglu_launch(x, w, out_bf16, M, N, K, t.nw, t.upw, t.tpw, blk, st)
                   : dense_gemm_launch(x, w, direct ? out_bf16 : nullptr, direct ? nullptr : part,
                                       M, N, K, t.nw, t.upw, t.tpw, t.ksplit, blk, st);
+  } else if (t.kind == 8) {
+    const bool direct = out_bf16 && t.ksplit == 1;
+    rc = dense_gemm8_launch(x, w, scale, direct ? out_bf16 : nullptr, direct ? nullptr : part, M,
+                            N, K, t.ksplit, t.swiglu != 0, st);
   } else if (t.kind == 2) {
     rc = w4b_launch(t.w4b, x, w, scale, zero, t.ksplit == 1 ? out_bf16 : nullptr, part, M, N, K,
                     ni, ro, st);

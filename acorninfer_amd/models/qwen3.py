@@ -679,7 +679,8 @@ class Qwen3DecodeModel:
         interleave."""
         gu = self.layers[0].gate_up
         return gu.il16 and rows >= PREFILL_SWIGLU_M and (
-            gu.fmt in (WFMT_BF16, WFMT_BF16B) or (gu.fmt == WFMT_W4B and rows >= DEQUANT_M_MIN))
+            gu.fmt in (WFMT_BF16, WFMT_BF16B, WFMT_W8B) or
+            (gu.fmt == WFMT_W4B and rows >= DEQUANT_M_MIN))
 
     def fused_swiglu_possible(self, batch: int) -> bool:
         """The gate|up launch can carry the SwiGLU epilogue (decode sizes,

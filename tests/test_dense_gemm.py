@@ -205,3 +205,97 @@ def test_planner_refuses_blocked_weights_on_the_staged_form():
     with pytest.raises(NotImplementedError):
         plan(4096, 4096, 4096, WFMT_BF16B, Tiling(DENSE_RT, 256, 64, 1, 2))
     assert plan(4096, 4096, 4096, WFMT_BF16B)[0] == Tiling(DENSE_RT, 256, 128, 1, 4)
+
+
+# (M, N, K): ragged rows and weight tiles (N a multiple of 16 only), the fewest
+# k, one more than a tile, several splits
+W8_SHAPES = [(256, 256, 128), (257, 272, 256), (700, 1040, 512), (513, 4096, 1024),
+             (1025, 768, 384)]
+
+
+def _w8b(N, K, seed):
+    from acorninfer_amd.models.qwen3 import WFMT_W8, QLinear
+    g = torch.Generator().manual_seed(seed)
+    q = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8)
+    q[0, :] = -127                                     # the range's ends in whole rows
+    q[1, :] = 127
+    scale = (0.001 + 0.01 * torch.rand(N, generator=g)).half()
+    return QLinear(WFMT_W8, q.cuda(), N, K, scale.cuda()).blocked(), q, scale
+
+
+def _launch8(lin, x, tiling, fp32):
+    t, _ = lin.plan(x.shape[0], tiling)
+    M = x.shape[0]
+    st = torch.cuda.current_stream().cuda_stream
+    part = torch.full((t.ksplit, M, lin.N), float("nan"), device="cuda")
+    out = None if fp32 else torch.empty(M, lin.N, dtype=torch.bfloat16, device="cuda")
+    lin.launch(x, M, t, out=out, part=part, stream=st)
+    return part if fp32 else out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", W8_SHAPES)
+def test_w8b_large_m_matches_float64(shape):
+    """int8 weights on the large-M kernel: the integers enter the MFMAs exactly,
+    so fp32 sums differ from float64 by accumulation drift only; the bf16 output
+    is the fp32 output rounded once; a split's planes add up to the whole."""
+    from acorninfer_amd.ops.quant_gemm import Tiling
+    M, N, K = shape
+    lin, q, scale = _w8b(N, K, 7 * M + N)
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    want = x.double() @ (q.cuda().double() * scale.cuda().double()[:, None]).t()
+    rms = want.square().mean().sqrt()
+    one = _launch8(lin, x, Tiling(DENSE_RT, 0, 0, 1, 0), True)
+    # K terms of relative size up to 127 * 4 / (73 * 1): each add rounds at 2^-24 of the sum
+    assert ((one[0].double() - want).abs().max() / rms) < K * 2.0 ** -24 * 8
+    out = _launch8(lin, x, Tiling(DENSE_RT, 0, 0, 1, 0), False)
+    assert torch.equal(out, one[0].bfloat16())
+    for ks in (2, 4, 8):
+        if (K // 32) % (2 * ks):
+            continue
+        planes = _launch8(lin, x, Tiling(DENSE_RT, 0, 0, ks, 0), True)
+        assert planes.shape[0] == ks and bool(planes.isfinite().all())
+        assert ((planes.double().sum(0) - want).abs().max() / rms) < K * 2.0 ** -24 * 8
+    if N % 128:                                        # no form by default, as before
+        with pytest.raises(NotImplementedError):
+            lin.plan(M)
+        return
+    # the planner's own choice at this size
+    auto = _launch8(lin, x, None, False)
+    assert ((auto.double() - want).norm() / want.norm()) < 4e-3       # one bf16 rounding
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(512, 512, 256), (600, 1056, 512)])
+def test_w8b_large_m_swiglu_is_silu_mul_of_the_output(M, N, K):
+    from acorninfer_amd._lib import BF16, check, lib, ptr, stream_ptr
+    from acorninfer_amd.ops.quant_gemm import Tiling
+    lin, _, _ = _w8b(N, K, N)
+    lin.il16 = True                                    # rows read as gate / up blocks of 16
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(3)).bfloat16().cuda()
+    act = torch.empty(M, N // 2, dtype=torch.bfloat16, device="cuda")
+    t, _ = lin.swiglu_plan(M)
+    assert t.rt == DENSE_RT and t.ksplit == 1
+    lin.launch_swiglu(x, M, t, act, stream_ptr())
+    plane = _launch8(lin, x, Tiling(DENSE_RT, 0, 0, 1, 0), True)
+    want = torch.empty_like(act)
+    check(lib().acorn_silu_mul(ptr(plane), 1, None, ptr(want), M, N // 2, 1, BF16, stream_ptr()),
+          "silu_mul")
+    assert torch.equal(act, want)
+
+
+@pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 4096), (24576, 4096), (4096, 12288),
+                                 (1024, 3072), (4096, 1024), (1040, 512)])
+def test_default_tilings_of_the_block_layouts_are_launchable(N, K):
+    """The library's choice with nothing requested, asked for again in full, is
+    accepted as it is, for every size from one row to a long prompt (no GPU)."""
+    from acorninfer_amd._lib import WFMT_BF16B, WFMT_W4B, WFMT_W8B
+    from acorninfer_amd.ops.quant_gemm import plan
+    for fmt in (WFMT_W4B, WFMT_W8B, WFMT_BF16B):
+        for M in (1, 2, 8, 9, 16, 17, 24, 25, 64, 65, 200, 255, 256, 511, 512, 1000, 8192):
+            if N % 128 and 16 < M and not (fmt == WFMT_BF16B and M >= 256):
+                continue                               # no tiled form: refused
+            t, tiles = plan(M, N, K, fmt)
+            assert tiles >= 1 and t.ksplit >= 1
+            assert plan(M, N, K, fmt, t)[0] == t, (fmt, M, t)
