@@ -357,6 +357,10 @@ struct DirectPlan {
 int w8b_make_plan(int64_t M, int64_t N, int64_t K, const int* cfg, bool swiglu, DirectPlan* p);
 // out (bf16 [M,N], or act [M,N/2] for swiglu) when given and ksplit == 1;
 // otherwise fp32 partials part[ksplit, M, N] (each already scaled).
+// natural int8 rows at decode sizes (the plan: one split, K slices)
+bool w8n_make_plan(int64_t M, int64_t N, int64_t K, DirectPlan* p);
+int w8n_launch(const DirectPlan& p, const void* x, const void* w, const void* scale, void* out,
+               float* part, int64_t M, int64_t N, int64_t K, hipStream_t st);
 int w8b_launch(const DirectPlan& p, const void* x, const void* w, const void* scale, void* out,
                float* part, int64_t M, int64_t N, int64_t K, const NormIn* ni,
                const ResidOut* ro, hipStream_t st);

@@ -756,7 +756,9 @@ struct Tiling {
                                  // 5 = W8B decode kernel (tpw = its pipeline depth),
                                  // 6 = BF16B decode kernel (tpw = its pipeline depth),
                                  // 7 = W8B mid-M kernel (as 4, tpw = steps in flight),
-                                 // 8 = large-M kernel on W8B weights (as 3)
+                                 // 8 = large-M kernel on W8B weights (as 3),
+                                 // 9 = W8 direct kernel on natural rows (rt == kNatRT,
+                                 //     upw = row tiles per wave, nw = wave layout)
   W4bPlan w4b;
   DirectPlan w8b;
   DirectPlan bf16b;
@@ -884,6 +886,9 @@ constexpr int64_t kDenseMinM = 256;
 constexpr int64_t kDenseLdsM = 512;
 // W4B above 16 rows on request (rt == kMidRT): the mid-M int4 kernel
 constexpr int kMidRT = -3;
+// natural W8 rows up to 16 x rows: the direct kernel, by default (one split;
+// the streaming kernel below it splits K to 4 workgroups per CU)
+constexpr int kNatRT = -5;
 
 // K splits that stay within one round of the CUs: the mid-M kernels' 256 x 64
 // tiles, and the large-M W8B kernel's 256 x 256 ones.
@@ -990,6 +995,25 @@ int make_plan(int64_t M, int64_t N, int64_t K, int wfmt, const int* cfg, Tiling*
   t->kind = 0;
   const bool no_request = !cfg || (cfg[0] == 0 && cfg[1] == 0 && cfg[2] == 0 && cfg[3] <= 1 &&
                                    cfg[4] == 0);
+  if (wfmt == ACORN_WFMT_W8 && !swiglu && M <= 16 &&
+      (!cfg || cfg[0] == kNatRT ||
+       (!cfg[0] && !cfg[1] && !cfg[2] && !cfg[3] && !cfg[4])) &&
+      w8n_make_plan(M, N, K, &t->w8b)) {
+    t->kind = 9;
+    t->rt = kNatRT;
+    t->upw = t->w8b.rt;
+    t->nw = t->w8b.nw_field;
+    t->ksplit = 1;
+    t->tpw = t->w8b.depth;
+    t->mt = 1;
+    t->R = (int)M;
+    t->nk = 0;
+    t->ntiles = (int)(N / 16);
+    t->mblocks = 1;
+    t->groups = t->w8b.groups;
+    t->lds = 0;
+    return ACORN_OK;
+  }
   const bool req8 = cfg && cfg[0] == kDenseRT;
   if (wfmt == ACORN_WFMT_W8B &&
       (req8 || (no_request && (swiglu ? M >= kDenseLdsM : N % 128 == 0 && dense8_faster(M, N, K))))) {
@@ -1433,6 +1457,8 @@ int gemm_entry(const void* x, const void* w, const void* scale, const void* zero
     rc = w4m_launch(t.w4m, x, w, scale, t.ksplit == 1 ? out_bf16 : nullptr, part, M, N, K, st);
   } else if (t.kind == 7) {
     rc = w8m_launch(t.w8m, x, w, scale, t.ksplit == 1 ? out_bf16 : nullptr, part, M, N, K, st);
+  } else if (t.kind == 9) {
+    rc = w8n_launch(t.w8b, x, w, scale, out_bf16, part, M, N, K, st);
   } else if (t.kind == 5) {
     rc = w8b_launch(t.w8b, x, w, scale, t.ksplit == 1 ? out_bf16 : nullptr, part, M, N, K, ni,
                     ro, st);

@@ -22,6 +22,14 @@
 //    their results through LDS in fixed order at the end.
 //  * Split-K (ksplit > 1) writes scaled fp32 partials [ksplit, M, N], summed
 //    in split order by the consumer (bitwise deterministic).
+//  * NAT: the same kernel on the reference's rows (int8 [N, K]), for callers of
+//    the operator: a wave's load covers 16 rows x 64 bytes, the same lanes' same
+//    bytes, and a stage holds an even number of blocks, so that the two halves
+//    of a 128-byte line are requested together (default cache policy: the second
+//    half comes from the first one's line). The bytes are signed as they lie, so
+//    no bias is removed. Without the streaming kernel's x staging, split planes
+//    and reduction launch: the seven projections of an 8B layer at 8 rows 130 us
+//    there, @NAT@ here.
 //  * MODE 1 / 2: the RMSNorm folded in as in bf16_decode.hip (results scaled
 //    by the rows' 1 / rms, after the per-channel scale; the residual epilogue
 //    with the weighted rows and the sums of squares).
@@ -64,13 +72,20 @@ __device__ __forceinline__ u32x4 unpack_w8(uint32_t a, uint32_t b) {
   return r;
 }
 
+// 8 signed bytes -> bf16 in slot order
+__device__ __forceinline__ u32x4 unpack_i8(uint32_t a, uint32_t b) {
+  return unpack_w8s(a ^ 0x80808080u, b ^ 0x80808080u);
+}
+
 // Grid: x = tile groups of RG * RT 16-row tiles, y = ksplit; block RG * KW
 // waves. Row group r of workgroup b owns tiles (b RG + r) RT .. + RT - 1; its
 // KW waves split the split's K range. Lane (lr, lg) holds x row min(lr, M - 1)
 // (rows past M feed only columns that are never stored).
 // HX (M <= 8, UPW even): the paired-x form (gemm_common.h, rot8).
-template <int RT, int UPW, int DEPTH, int RG, int KW, bool SWIGLU, int MODE, bool HX = false>
+template <int RT, int UPW, int DEPTH, int RG, int KW, bool SWIGLU, int MODE, bool HX = false,
+          bool NAT = false>
 __global__ __launch_bounds__(RG * KW * kWave) void w8b_direct_kernel(W8dArgs a) {
+  static_assert(!NAT || UPW % 2 == 0, "whole lines of a natural row");
   static_assert(!HX || UPW % 2 == 0, "x in block pairs");
   constexpr int NW = RG * KW;
   constexpr bool NORM = MODE == 1;
@@ -85,7 +100,8 @@ __global__ __launch_bounds__(RG * KW * kWave) void w8b_direct_kernel(W8dArgs a) 
   const int BW = a.kr / (64 * KW);                // blocks of this wave
   const int kw0 = blockIdx.y * a.kr + kq * BW * 64;
   const int ns = BW / UPW;                        // stages, a multiple of DEPTH
-  const uint8_t* wb = a.w + ((size_t)tt * KB + kw0 / 64) * 1024 + lane * 16;
+  const uint8_t* wb = NAT ? a.w + ((size_t)tt * 16 + lr) * a.K + kw0 + 16 * lg
+                          : a.w + ((size_t)tt * KB + kw0 / 64) * 1024 + lane * 16;
   const __bf16* xb = HX ? a.x + (size_t)min(lr & 7, a.M - 1) * a.K + kw0 + 16 * lg + 64 * (lr >> 3)
                         : a.x + (size_t)min(lr, a.M - 1) * a.K + kw0 + 16 * lg;
   auto load = [&](int s, W8Stage<RT, UPW, HX>& r) {
@@ -98,7 +114,8 @@ __global__ __launch_bounds__(RG * KW * kWave) void w8b_direct_kernel(W8dArgs a) 
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
       for (int u = 0; u < UPW; ++u)
-        r.w[rt][u] = load_nt((const u32x4*)(wb + ((size_t)rt * KB + s * UPW + u) * 1024));
+        r.w[rt][u] = NAT ? *(const u32x4*)(wb + (size_t)rt * 16 * a.K + (s * UPW + u) * 64)
+                         : load_nt((const u32x4*)(wb + ((size_t)rt * KB + s * UPW + u) * 1024));
   };
 
   NormRegs nr;
@@ -124,13 +141,17 @@ __global__ __launch_bounds__(RG * KW * kWave) void w8b_direct_kernel(W8dArgs a) 
       u32x4 xu[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) xu[j] = HX && (u & 1) ? rot8(r.x[u / 2][j]) : r.x[HX ? u / 2 : u][j];
+      if constexpr (!NAT) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) xacc = mfma(neg128, xu[j], xacc);
+        for (int j = 0; j < 2; ++j) xacc = mfma(neg128, xu[j], xacc);
+      }
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          acc[rt] = mfma(unpack_w8(r.w[rt][u][2 * j], r.w[rt][u][2 * j + 1]), xu[j], acc[rt]);
+          acc[rt] = mfma(NAT ? unpack_i8(r.w[rt][u][2 * j], r.w[rt][u][2 * j + 1])
+                             : unpack_w8(r.w[rt][u][2 * j], r.w[rt][u][2 * j + 1]),
+                         xu[j], acc[rt]);
       // one block at a time: keeps the unpacked operands of later blocks from
       // being hoisted past the register ring's budget
       __builtin_amdgcn_sched_barrier(0);
@@ -302,6 +323,18 @@ int by_upw(const DirectPlan& p, const W8dArgs& a, hipStream_t st) {
     case 2: return by_depth<RT, 2>(p, a, st);
   }
   return ACORN_ERR_UNSUPPORTED;
+}
+
+// The natural-layout form: one row tile (few row tiles) or two per wave, two
+// blocks per stage, four stages in flight where K allows, four K slices.
+template <int RT, int DEPTH, int KW>
+int launch_nat(const DirectPlan& p, const W8dArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)p.groups), block(KW * kWave);
+  if (p.hx)
+    w8b_direct_kernel<RT, 2, DEPTH, 1, KW, false, 0, true, true><<<grid, block, 0, st>>>(a);
+  else
+    w8b_direct_kernel<RT, 2, DEPTH, 1, KW, false, 0, false, true><<<grid, block, 0, st>>>(a);
+  return ACORN_OK;
 }
 
 int divisor_at_least(int64_t n, int64_t v) {
@@ -608,6 +641,49 @@ int w8b_launch(const DirectPlan& p, const void* x, const void* w, const void* sc
     case 1: rc = by_upw<1>(p, a, st); break;
     case 2: rc = by_upw<2>(p, a, st); break;
     case 4: rc = by_upw<4>(p, a, st); break;
+  }
+  if (rc) return rc;
+  ACORN_LAUNCH_CHECK();
+  return ACORN_OK;
+}
+
+// The natural layout at decode sizes: N in 16s, rows of whole 128-byte lines per
+// K slice, 16-byte aligned operands (checked at the launch).
+bool w8n_make_plan(int64_t M, int64_t N, int64_t K, DirectPlan* p) {
+  if (M < 1 || M > 16 || N % 16) return false;
+  const int64_t nt = N / 16;
+  const int rt = nt % 2 == 0 && nt >= 512 ? 2 : 1;
+  const int kw = nt >= 512 ? 4 : 8;
+  int depth = 4;
+  while (depth > 1 && (K % (128 * kw * depth) ||
+                       depth * stage_dwords(rt, 2, M <= 8) > kRingDwords))
+    depth /= 2;
+  if (K % (128 * kw * depth) || nt / rt > 0x7fffffff) return false;
+  *p = DirectPlan{};
+  p->rt = rt;
+  p->upw = 2;
+  p->rg = 1;
+  p->kw = kw;
+  p->nw_field = 11 * kw;
+  p->ksplit = 1;
+  p->depth = depth;
+  p->groups = (int)(nt / rt);
+  p->hx = M <= 8;
+  return true;
+}
+
+int w8n_launch(const DirectPlan& p, const void* x, const void* w, const void* scale, void* out,
+               float* part, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+  const W8dArgs a{(const __bf16*)x, (const uint8_t*)w, (const _Float16*)scale, (__bf16*)out,
+                  part, (int)M, (int)N, (int)K, (int)K, NormIn{}, ResidOut{}};
+  int rc = ACORN_ERR_UNSUPPORTED;
+  switch (p.rt * 100 + p.kw * 10 + p.depth) {
+    case 181: rc = launch_nat<1, 1, 8>(p, a, st); break;
+    case 182: rc = launch_nat<1, 2, 8>(p, a, st); break;
+    case 184: rc = launch_nat<1, 4, 8>(p, a, st); break;
+    case 241: rc = launch_nat<2, 1, 4>(p, a, st); break;
+    case 242: rc = launch_nat<2, 2, 4>(p, a, st); break;
+    case 244: rc = launch_nat<2, 4, 4>(p, a, st); break;
   }
   if (rc) return rc;
   ACORN_LAUNCH_CHECK();
