@@ -603,18 +603,29 @@ __global__ __launch_bounds__(512, 1) void dense_dl8_kernel(const __bf16* __restr
 #pragma unroll
     for (int j = 0; j < MB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   u32x4 a[NB], b0[MB], b1[MB];                 // a: both halves of the pair's bytes
+  // row i's operand is converted during row i - 1's MFMAs (row 0's during the
+  // previous stage's last row, its bytes being refilled first in a pair's second
+  // stage), four VALU instructions to an MFMA
+  u32x4 av = {0u, 0u, 0u, 0u};
   auto stage = [&](int s, const u32x4 (&bc)[MB], u32x4 (&bn)[MB], int dq) {
+    const int h = s & 1;
 #pragma unroll
     for (int j = 0; j < MB; ++j) bn[j] = opB(s + 1, j);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-      const int h = s & 1;
-      const u32x4 av = unpack_w8s(a[i][2 * h], a[i][2 * h + 1]);
+      if (h) a[i] = opA((s + 1) >> 1, i);
+      const int ni = (i + 1) % NB, nh = i + 1 < NB ? h : h ^ 1;
+      const u32x4 nv = unpack_w8s(a[ni][2 * nh], a[ni][2 * nh + 1]);
 #pragma unroll
       for (int j = 0; j < MB; ++j) acc[i][j] = mfma(av, bc[j], acc[i][j]);
-      if (h) a[i] = opA((s + 1) >> 1, i);
+      av = nv;
       if (dq >= 0 && i < LPA + LPX) issue_one(dq, i);
+#pragma unroll
+      for (int j = 0; j < MB; ++j) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);   // MFMA
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);   // VALU
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
@@ -630,6 +641,7 @@ __global__ __launch_bounds__(512, 1) void dense_dl8_kernel(const __bf16* __restr
   for (int i = 0; i < NB; ++i) a[i] = opA(0, i);
 #pragma unroll
   for (int j = 0; j < MB; ++j) b0[j] = opB(0, j);
+  av = unpack_w8s(a[0][0], a[0][1]);
   for (int d = 0; d < pairs; ++d) {
     stage(2 * d, b0, b1, -1);
     ACORN_DL_VMCNT(0);

@@ -729,15 +729,43 @@ size_t tile_lds_bytes(int wfmt, int bm, int bn, int64_t kper) {
   return b;
 }
 
-// Split-K reduction (fixed order) with the output cast.
-template <typename T>
-__global__ void splitk_reduce_kernel(const float* __restrict__ part, int nsplit, size_t count,
-                                     T* __restrict__ out) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Split-K reduction (fixed order) with the output cast: V consecutive outputs
+// per thread, eight splits requested at a time (indices past the last re-read
+// it; their values are not added).
+constexpr int kReduceBatch = 8;
+template <typename T, int V>
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ part,
+                                                            int nsplit, size_t count,
+                                                            T* __restrict__ out) {
+  typedef float fV __attribute__((ext_vector_type(V)));
+  typedef T tV __attribute__((ext_vector_type(V)));
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * V;
   if (i >= count) return;
-  float acc = part[i];
-  for (int s = 1; s < nsplit; ++s) acc += part[(size_t)s * count + i];
-  out[i] = (T)acc;
+  fV acc;
+  for (int s0 = 0; s0 < nsplit; s0 += kReduceBatch) {
+    fV v[kReduceBatch];
+#pragma unroll
+    for (int u = 0; u < kReduceBatch; ++u)
+      v[u] = *(const fV*)(part + (size_t)min(s0 + u, nsplit - 1) * count + i);
+#pragma unroll
+    for (int u = 0; u < kReduceBatch; ++u)
+      if (s0 + u < nsplit) acc = s0 + u == 0 ? v[u] : acc + v[u];
+  }
+  *(tV*)(out + i) = __builtin_convertvector(acc, tV);
+}
+
+template <typename T>
+void splitk_reduce(const float* part, int nsplit, size_t count, T* out, hipStream_t st) {
+  // four outputs per thread from a size that still fills the chip (the bf16
+  // projections of 999 rows 431 -> 426 us); below, one per thread (the int4 ones
+  // of 64 rows 159 us, 176 with four)
+  const bool four = count >= ((size_t)3 << 20) && count % 4 == 0 && (uintptr_t)part % 16 == 0 && (uintptr_t)out % 16 == 0;
+  const size_t threads = four ? count / 4 : count;
+  const unsigned grid = (unsigned)((threads + 255) / 256);
+  if (four)
+    splitk_reduce_kernel<T, 4><<<grid, 256, 0, st>>>(part, nsplit, count, out);
+  else
+    splitk_reduce_kernel<T, 1><<<grid, 256, 0, st>>>(part, nsplit, count, out);
 }
 
 // ----------------------------------------------------------------- planning --
@@ -756,7 +784,8 @@ struct Tiling {
                                  // 5 = W8B decode kernel (tpw = its pipeline depth),
                                  // 6 = BF16B decode kernel (tpw = its pipeline depth),
                                  // 7 = W8B mid-M kernel (as 4, tpw = steps in flight),
-                                 // 8 = large-M kernel on W8B weights (as 3),
+                                 // 8 = large-M kernel on W8B weights (as 3; tpw = its
+                                 //     256-row tiles, the rows past them on kind 7),
                                  // 9 = W8 direct kernel on natural rows (rt == kNatRT,
                                  //     upw = row tiles per wave, nw = wave layout)
   W4bPlan w4b;
@@ -904,23 +933,39 @@ int dense8_splits(int64_t M, int64_t N, int64_t K) {
   while (tiles * 2 * ks <= kCUs && ks < 16 && dense_gemm8_supported(N, K, 2 * ks, false)) ks *= 2;
   return ks;
 }
-// W8B from 256 rows: the large-M kernel or the mid-M one. Both run in whole
-// rounds of the 256 CUs, 37 us per 4096 k for a round of 256 x 64 tiles and 111
-// for one of 256 x 256, plus the split planes at 5 TB/s, written and read; the
-// smaller tile wins where the larger leaves a good part of a round empty (by
-// 10%: in one split the larger can write its consumer's bf16 input). This
-// predicts the measured times within 10%: 1000 rows, mid / large, qkv 74 / 77
-// us, o 40 / 56, gate|up 236 / 225, down 112 / 109; gate|up at 700 rows 186 /
-// 218, at 2000 477 / 361.
-bool dense8_faster(int64_t M, int64_t N, int64_t K) {
-  if (M < 256) return false;
+// W8B from 256 rows: the large-M kernel, the mid-M one, or the large one on the
+// first 256-row tiles and the mid-M one on the rest. Both run in whole rounds
+// of the 256 CUs, 37 us per 4096 k for a round of 256 x 64 tiles and 111 for one
+// of 256 x 256, plus the split planes at 5 TB/s, written and read; the smaller
+// tile wins where the larger leaves a good part of a round empty (by 10%: in
+// one split the larger can write its consumer's bf16 input), and finishes what
+// the larger has left after its full rounds. This predicts the measured times
+// within 10%: 1000 rows, mid / large, qkv 74 / 77 us, o 40 / 56, gate|up 236 /
+// 225, down 112 / 109; gate|up at 700 rows 186 / 218, at 2000 477 / 361; at 4502
+// rows o 213 / 222 and @SPLIT8@ for 4096 of them on the large one.
+// False: the mid-M kernel. Else *ks splits, *first row tiles on the large one.
+bool dense8_choice(int64_t M, int64_t N, int64_t K, int* ks, int* first) {
+  const int mtiles = (int)((M + 255) / 256);
+  *ks = dense8_splits(M, N, K);
+  *first = mtiles;
   if (N % 256 || K % 512) return true;      // no mid-M form
-  auto us = [&](int64_t tiles, int ks, double round) {
-    return (double)((tiles * ks + kCUs - 1) / kCUs) / ks * round * (double)K / 4096.0 +
-           (ks > 1 ? 8.0 * ks * (double)M * (double)N / 5e6 : 0.0);
+  auto us = [&](int64_t tiles, int splits, double round) {
+    return (double)((tiles * splits + kCUs - 1) / kCUs) / splits * round * (double)K / 4096.0 +
+           (splits > 1 ? 8.0 * splits * (double)M * (double)N / 5e6 : 0.0);
   };
-  return us((N + 255) / 256 * ((M + 255) / 256), dense8_splits(M, N, K), 111.0) <
-         1.1 * us(N / 256 * ((M + 63) / 64), mid_splits(M, N, K), 37.0);
+  const double large = us(N / 256 * mtiles, *ks, 111.0);
+  const double mid = 1.1 * us(N / 256 * ((M + 63) / 64), mid_splits(M, N, K), 37.0);
+  double best = std::min(large, mid);
+  for (int f = 1; f < mtiles; ++f) {
+    const double both = us(N / 256 * f, 1, 111.0) +
+                        us(N / 256 * ((M - 256 * (int64_t)f + 63) / 64), 1, 37.0) + 4.0;
+    if (both < 0.95 * best) {
+      best = both;
+      *first = f;
+    }
+  }
+  if (*first < mtiles) *ks = 1;
+  return *first < mtiles || large < mid;
 }
 
 // The tiling of a block-layout launch with nothing requested, from a sweep of
@@ -1016,26 +1061,37 @@ int make_plan(int64_t M, int64_t N, int64_t K, int wfmt, const int* cfg, Tiling*
   }
   const bool req8 = cfg && cfg[0] == kDenseRT;
   if (wfmt == ACORN_WFMT_W8B &&
-      (req8 || (no_request && (swiglu ? M >= kDenseLdsM : N % 128 == 0 && dense8_faster(M, N, K))))) {
-    const int64_t tiles = (N + 255) / 256 * ((M + 255) / 256);
-    const int ks = req8 && cfg[3] > 0 ? cfg[3] : swiglu ? 1 : dense8_splits(M, N, K);
+      (req8 || (no_request && (swiglu ? M >= kDenseLdsM : N % 128 == 0 && M >= kDenseMinM)))) {
+    const int mtiles = (int)((M + 255) / 256);
+    int ks = req8 && cfg[3] > 0 ? cfg[3] : 1, first = mtiles;
+    if (req8 && cfg[4] > 0) first = std::min(cfg[4], mtiles);
     const bool form = !req8 || ((cfg[1] == 0 || cfg[1] == 256) && (cfg[2] == 0 || cfg[2] == 128) &&
-                               (cfg[4] == 0 || cfg[4] == 4));
-    if (form && dense_gemm8_supported(N, K, ks, swiglu)) {
+                                (first == mtiles || (ks == 1 && !swiglu && N % 256 == 0 &&
+                                                     K % 512 == 0)));
+    bool large = true;
+    if (!swiglu && !(req8 && cfg[3] > 0)) ks = dense8_splits(M, N, K);
+    if (!req8 && !swiglu) large = dense8_choice(M, N, K, &ks, &first);
+    if (large && form && dense_gemm8_supported(N, K, ks, swiglu)) {
+      const int64_t ntiles = (N + 255) / 256;
       t->kind = 8;
       t->rt = kDenseRT;
       t->upw = 256;
       t->nw = 128;
       t->ksplit = ks;
-      t->tpw = 4;
+      t->tpw = first;
       t->mt = 1;
       t->R = 256;
       t->nk = (int)(K / 64);
-      t->ntiles = (int)((N + 255) / 256);
-      t->mblocks = (int)((M + 255) / 256);
+      t->ntiles = (int)ntiles;
+      t->mblocks = mtiles;
       t->groups = 1;
       t->lds = 0;
-      return tiles > 0x7fffffff ? ACORN_ERR_SHAPE : ACORN_OK;
+      if (first < mtiles) {
+        const int mid[5] = {kMidRT, 2, 8, 1, 2};
+        const int rc = w8m_make_plan(M - 256 * (int64_t)first, N, K, mid, &t->w8m);
+        if (rc) return rc;
+      }
+      return ntiles * mtiles > 0x7fffffff ? ACORN_ERR_SHAPE : ACORN_OK;
     }
     if (req8) return ACORN_ERR_UNSUPPORTED;
   }
@@ -1447,8 +1503,13 @@ int gemm_entry(const void* x, const void* w, const void* scale, const void* zero
                                       M, N, K, t.nw, t.upw, t.tpw, t.ksplit, blk, st);
   } else if (t.kind == 8) {
     const bool direct = out_bf16 && t.ksplit == 1;
-    rc = dense_gemm8_launch(x, w, scale, direct ? out_bf16 : nullptr, direct ? nullptr : part, M,
+    const int64_t m0 = std::min<int64_t>(M, 256 * (int64_t)t.tpw);
+    rc = dense_gemm8_launch(x, w, scale, direct ? out_bf16 : nullptr, direct ? nullptr : part, m0,
                             N, K, t.ksplit, t.swiglu != 0, st);
+    if (!rc && m0 < M)                     // (one split) the rows past the large tiles
+      rc = w8m_launch(t.w8m, (const __bf16*)x + m0 * K, w, scale,
+                      direct ? (__bf16*)out_bf16 + m0 * N : nullptr,
+                      direct ? nullptr : part + m0 * N, M - m0, N, K, st);
   } else if (t.kind == 2) {
     rc = w4b_launch(t.w4b, x, w, scale, zero, t.ksplit == 1 ? out_bf16 : nullptr, part, M, N, K,
                     ni, ro, st);
@@ -1485,8 +1546,7 @@ int gemm_entry(const void* x, const void* w, const void* scale, const void* zero
   ACORN_LAUNCH_CHECK();
   if (out_bf16 && t.ksplit > 1) {
     const int64_t count = M * N;
-    splitk_reduce_kernel<__bf16><<<(unsigned)((count + 255) / 256), 256, 0, st>>>(
-        part, t.ksplit, (size_t)count, (__bf16*)out_bf16);
+    splitk_reduce<__bf16>(part, t.ksplit, (size_t)count, (__bf16*)out_bf16, st);
     ACORN_LAUNCH_CHECK();
   }
   return ACORN_OK;
@@ -1577,12 +1637,11 @@ extern "C" int acorn_splitk_reduce(const float* part, int64_t nsplit, int64_t co
   if (nsplit < 1 || count < 0) return ACORN_ERR_SHAPE;
   if (count == 0) return ACORN_OK;
   if (!part || !out) return ACORN_ERR_VALUE;
-  dim3 grid((unsigned)((count + 255) / 256)), block(256);
   hipStream_t st = (hipStream_t)stream;
   switch (dtype) {
-    case ACORN_F32: splitk_reduce_kernel<float><<<grid, block, 0, st>>>(part, (int)nsplit, (size_t)count, (float*)out); break;
-    case ACORN_F16: splitk_reduce_kernel<_Float16><<<grid, block, 0, st>>>(part, (int)nsplit, (size_t)count, (_Float16*)out); break;
-    case ACORN_BF16: splitk_reduce_kernel<__bf16><<<grid, block, 0, st>>>(part, (int)nsplit, (size_t)count, (__bf16*)out); break;
+    case ACORN_F32: splitk_reduce<float>(part, (int)nsplit, (size_t)count, (float*)out, st); break;
+    case ACORN_F16: splitk_reduce<_Float16>(part, (int)nsplit, (size_t)count, (_Float16*)out, st); break;
+    case ACORN_BF16: splitk_reduce<__bf16>(part, (int)nsplit, (size_t)count, (__bf16*)out, st); break;
     default: return ACORN_ERR_DTYPE;
   }
   ACORN_LAUNCH_CHECK();

@@ -101,7 +101,11 @@ class Tiling(NamedTuple):
     steps (2 / 4). 256 (256 x 256 tiles): nw 64 with tpw 2 stages both
     operands through registers; nw 128 with tpw 4 loads them straight into
     LDS through a 4-stage ring (the default). Reported as (-2, BM, nw,
-    ksplit, tpw).
+    ksplit, tpw). On W8B (M >= 256): (-2, 256, 128, ksplit, tpw), tpw the number
+    of 256-row tiles of x on the large-M kernel; the rows past them (one split)
+    run on the mid-M kernel.
+    Natural W8 rows (M <= 16, the default there): (-5, row tiles per wave, wave
+    layout, 1, stages in flight), the direct kernel on the reference's layout.
     """
     rt: int = 0
     upw: int = 0

@@ -210,7 +210,7 @@ def test_planner_refuses_blocked_weights_on_the_staged_form():
 # (M, N, K): ragged rows and weight tiles (N a multiple of 16 only), the fewest
 # k, one more than a tile, several splits
 W8_SHAPES = [(256, 256, 128), (257, 272, 256), (700, 1040, 512), (513, 4096, 1024),
-             (1025, 768, 384)]
+             (1025, 768, 384), (257, 512, 512), (900, 256, 1024)]
 
 
 def _w8b(N, K, seed):
@@ -261,6 +261,13 @@ def test_w8b_large_m_matches_float64(shape):
         with pytest.raises(NotImplementedError):
             lin.plan(M)
         return
+    # the first rows on this kernel, the rest on the mid-M kernel
+    if N % 256 == 0 and K % 512 == 0 and M > 256:
+        tail = _launch8(lin, x, Tiling(DENSE_RT, 0, 0, 1, 1), False)
+        assert torch.equal(tail[:256], out[:256])
+        assert ((tail.double() - want).norm() / want.norm()) < 4e-3
+        planes = _launch8(lin, x, Tiling(DENSE_RT, 0, 0, 1, 1), True)
+        assert torch.equal(planes[0].bfloat16(), tail)
     # the planner's own choice at this size
     auto = _launch8(lin, x, None, False)
     assert ((auto.double() - want).norm() / want.norm()) < 4e-3       # one bf16 rounding
