@@ -29,7 +29,7 @@
 //    half comes from the first one's line). The bytes are signed as they lie, so
 //    no bias is removed. Without the streaming kernel's x staging, split planes
 //    and reduction launch: the seven projections of an 8B layer at 8 rows 130 us
-//    there, @NAT@ here.
+//    there, 72 here.
 //  * MODE 1 / 2: the RMSNorm folded in as in bf16_decode.hip (results scaled
 //    by the rows' 1 / rms, after the per-channel scale; the residual epilogue
 //    with the weighted rows and the sums of squares).
@@ -648,12 +648,13 @@ int w8b_launch(const DirectPlan& p, const void* x, const void* w, const void* sc
 }
 
 // The natural layout at decode sizes: N in 16s, rows of whole 128-byte lines per
-// K slice, 16-byte aligned operands (checked at the launch).
+// K slice. Operands may lie at any address, as for the streaming kernel: plain
+// 16-byte global loads, which need no alignment on this target.
 bool w8n_make_plan(int64_t M, int64_t N, int64_t K, DirectPlan* p) {
   if (M < 1 || M > 16 || N % 16) return false;
   const int64_t nt = N / 16;
   const int rt = nt % 2 == 0 && nt >= 512 ? 2 : 1;
-  const int kw = nt >= 512 ? 4 : 8;
+  const int kw = rt == 2 ? 4 : 8;
   int depth = 4;
   while (depth > 1 && (K % (128 * kw * depth) ||
                        depth * stage_dwords(rt, 2, M <= 8) > kRingDwords))

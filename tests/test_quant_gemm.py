@@ -658,3 +658,38 @@ def test_fused_swiglu_at_prefill_sizes(fmt, m):
     r = rel_err(act, ref)
     print(f"\n[swiglu {fmt} M={m} at prefill size: rel err {r:.3g}]")
     assert r <= 1e-2
+
+
+# the int8 operator at decode sizes: row tiles 1 (odd or few) and 2 per wave, the
+# ring at 4, 2 and 1 stages, the pair form (M <= 8) and the 16-row one, and rows
+# that the direct kernel does not take (K % 1024, M = 17)
+NAT_CASES = [(1, 16, 1024), (7, 48, 2048), (8, 8208, 1024), (9, 8208, 2048), (8, 8192, 512),
+             (16, 8192, 1024), (9, 8224, 2048), (16, 272, 4096), (8, 64, 8192), (5, 32, 640),
+             (16, 64, 128), (17, 64, 1024)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k", NAT_CASES)
+def test_w8_rows_at_decode_sizes_match_float64(m, n, k):
+    from acorninfer_amd.models.qwen3 import WFMT_W8
+    from acorninfer_amd.ops.quant_gemm import Tiling, plan, quant_gemm
+    g = torch.Generator().manual_seed(n + k + m)
+    q = torch.randint(-128, 128, (n, k), generator=g, dtype=torch.int8)
+    q[0, :], q[1, :] = -128, 127
+    s = (0.001 + 0.01 * torch.rand(n, generator=g)).half()
+    x = torch.randn(m, k, generator=g).bfloat16()
+    want = x.double() @ (q.double() * s.double()[:, None]).t()
+    qd, sd, xd = q.cuda(), s.cuda(), x.cuda()
+    t = plan(m, n, k, WFMT_W8)[0]
+    assert (t.rt == -5) == (m <= 16 and k % (128 * (4 if n % 32 == 0 and n >= 8192 else 8)) == 0)
+    xo = torch.empty(m * k + 1, dtype=torch.bfloat16, device="cuda")[1:].view(m, k).copy_(xd)
+    qo = torch.empty(n * k + 1, dtype=torch.int8, device="cuda")[1:].view(n, k).copy_(qd)
+    outs = [quant_gemm(xd, qd, sd, "c", cfg=Tiling()),
+            quant_gemm(xd, qd, sd, "c", cfg=(0, 0, 1)),       # the streaming kernel
+            quant_gemm(xo, qo, sd, "c", cfg=Tiling())]        # operands at odd addresses
+    assert torch.equal(outs[0], outs[2])
+    for out in outs:
+        # the integers are exact; fp32 sums (K roundings of a sum of |x q|) and one to bf16
+        bound = want.abs() * 2.0 ** -8 + k * 2.0 ** -24 * (
+            x.double().abs() @ (q.double().abs() * s.double()[:, None]).t())
+        assert bool(((out.cpu().double() - want).abs() <= bound).all())
