@@ -56,11 +56,11 @@ DENSE_RT = -2
 # dequantised to bf16 into a step workspace (acorn_dequant_w4b) and
 # multiplied by the large-M bf16 kernel (tiling rt == DEQUANT_RT, the other
 # fields the bf16 kernel's). At prefill sizes the MFMA work dominates and that
-# kernel's rate outweighs the extra pass over the weights: on MI355X a W4A16
-# 8B prefill of 512 / 768 tokens takes 15.0 / 19.7 ms this way against
-# 15.9 / 25.4 ms on the int4 kernels; below 512 rows the int4 kernels win
-# (8.5-9.2 vs 12.8 ms at 256 tokens).
-DEQUANT_M_MIN = 512
+# kernel's rate outweighs the extra pass over the weights: on MI355X eight
+# layers of a W4A16 8B prefill take, this way / on the int4 kernels, 3.61 /
+# 3.07 ms at 512 tokens, 4.27 / 3.93 at 640, 4.40 / 4.60 at 768 and 5.00 / 5.28
+# at 1024.
+DEQUANT_M_MIN = 704
 DEQUANT_RT = -4
 # prefill blocks from this many rows run gate|up with the large-M kernel's
 # SwiGLU epilogue (act written directly: no fp32 gate|up output, no silu_mul);
