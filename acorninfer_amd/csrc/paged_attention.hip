@@ -1284,16 +1284,26 @@ int dispatch_d(int64_t D, int64_t rep, const void* q, const void* kp, const void
 
 // One sequence of a prefill launch: its first q row, that row's position and
 // its rows. With no seq_nq every sequence is a window of max_nq rows at row
-// n max_nq and seq_pos0 holds its length, the window included. Rows past q's R
-// rows (or past max_nq) are not served, so bad metadata cannot reach past q / out.
+// n max_nq and seq_pos0 holds its length, the window included (at most `cap`:
+// prefill_cap). Rows past q's R rows (or past max_nq) are not served, so bad
+// metadata cannot reach past q / out.
 struct PrefillSeq {
   int row0, pos0, nq;
 };
+// The window kernels (QW == 1) take a length as at most the tokens its table row
+// has pages for, as K3 does. The others do not: 8192 causal tokens, 32 / 8 heads,
+// take 731 us with the clamp in their kernel and 696 without, where the kernel
+// before the unconditional MFMAs takes 739 and 726 on the same cards.
+template <int QW>
+__host__ __device__ __forceinline__ int prefill_cap(int table_stride, int P) {
+  return QW == 1 ? table_stride * P : 0x7fffffff;
+}
 __device__ __forceinline__ PrefillSeq prefill_seq(const int32_t* row0, const int32_t* pos0,
-                                                  const int32_t* nq, int n, int R, int max_nq) {
+                                                  const int32_t* nq, int n, int R, int max_nq,
+                                                  int cap) {
   PrefillSeq s;
   if (nq == nullptr) {
-    s = {n * max_nq, pos0[n] - max_nq, max_nq};
+    s = {n * max_nq, min(pos0[n], cap) - max_nq, max_nq};
     if (s.pos0 + max_nq <= 0) s.nq = 0;
   } else {
     s = {row0[n], pos0[n], nq[n]};
@@ -1368,7 +1378,8 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
   const int r = lane >> 4, c = lane & 15;
   const int hq = wid % REP, sub = wid / REP;
   const int h = kvh * REP + hq;
-  const PrefillSeq sq = prefill_seq(seq_row0, seq_pos0, seq_nq, n, R, max_nq);
+  const PrefillSeq sq = prefill_seq(seq_row0, seq_pos0, seq_nq, n, R, max_nq,
+                                    prefill_cap<QW>(table_stride, P));
   const int pos0 = sq.pos0, row0 = sq.row0, nq = sq.nq;
   const int tile = SPLIT ? (gridDim.x - 1 - blockIdx.x) / S : gridDim.x - 1 - blockIdx.x;
   const int wg_j0 = tile * WQ;                                  // longest tiles first
@@ -1629,17 +1640,19 @@ template <typename T, int D>
 __global__ __launch_bounds__(kPrefillCombineNT) void paged_prefill_combine_kernel(
     const float* __restrict__ ws, const int32_t* __restrict__ seq_row0,
     const int32_t* __restrict__ seq_pos0, const int32_t* __restrict__ seq_nq, T* __restrict__ out,
-    int R, int H, int max_nq, int S, int cps, int WQ) {
+    int R, int H, int max_nq, int S, int cps, int WQ, int cap) {
   constexpr int LPP = D / 4;
   const int n = blockIdx.y;
   const int pair = (int)(blockIdx.x * (kPrefillCombineNT / LPP)) + threadIdx.x / LPP;
   const int j = pair / H, h = pair % H, d0 = 4 * (threadIdx.x % LPP);
-  const PrefillSeq sq = prefill_seq(seq_row0, seq_pos0, seq_nq, n, R, max_nq);
+  const PrefillSeq sq = prefill_seq(seq_row0, seq_pos0, seq_nq, n, R, max_nq, cap);
   if (j >= sq.nq) return;
   const int L = sq.pos0 + min(j / WQ * WQ + WQ, sq.nq);
   const int total = (L + kPrefillChunk - 1) / kPrefillChunk;
   if (total <= cps) return;
-  const int ns = (total + cps - 1) / cps;        // <= S
+  // (rows placed past their table row's pages have more runs than the S planned
+  // from the table: those past S were not launched and have no partials)
+  const int ns = min((total + cps - 1) / cps, S);
   const size_t slots = (size_t)gridDim.y * max_nq * H;
   const size_t slot = ((size_t)n * max_nq + j) * H + h;
   const float2* ml = (const float2*)(ws + (size_t)S * slots * D) + slot;
@@ -1741,7 +1754,8 @@ int launch_prefill(const PrefillArgs& a) {
     paged_prefill_combine_kernel<T, D>
         <<<dim3((unsigned)((a.max_nq * a.H + pairs - 1) / pairs), (unsigned)a.N),
            dim3(kPrefillCombineNT), 0, a.st>>>(a.ws, a.row0, a.pos0, a.nq, (T*)a.out, (int)a.R,
-                                               (int)a.H, (int)a.max_nq, S, a.plan.cps, WQ);
+                                               (int)a.H, (int)a.max_nq, S, a.plan.cps, WQ,
+                                               prefill_cap<QW>((int)a.table_stride, (int)a.P));
     ACORN_LAUNCH_CHECK();
   }
   return ACORN_OK;

@@ -112,6 +112,26 @@ def test_window_causality_exact(dtype, H, KV, D):
                                            atol=2e-2 if dtype != torch.float32 else 1e-3)
 
 
+def test_length_past_its_table_row_leaves_the_other_sequences():
+    """A sequence length past its table row's pages (bad metadata) counts as the
+    tokens those pages hold, as in K3: the launch plans its key runs and its
+    partials from the table's width. The others' rows are those of a correct batch
+    bit for bit."""
+    from acorninfer_amd.ops.paged_attention import prefill_workspace
+    from acorninfer_amd.ops.paged_verify import paged_verify_attention
+    B, M, H, KV, D, P = 3, 5, 32, 8, 128, 16
+    q, kp, vp, tables, lens = _gpu(*_inputs(B, M, 900, torch.bfloat16, H=H, KV=KV, D=D))
+    ws = prefill_workspace(B, B * M, M, H, KV, D, P, tables.shape[1], "cuda")
+    assert ws is not None, "the case is meant to split"
+    good = paged_verify_attention(q, kp, vp, tables, lens, 4)
+    bad = lens.clone()
+    bad[1] = 8 * tables.shape[1] * P
+    out = paged_verify_attention(q, kp, vp, tables, bad, 4)
+    assert torch.equal(out[[0, 2]], good[[0, 2]])
+    bad[1] = tables.shape[1] * P
+    assert torch.equal(out, paged_verify_attention(q, kp, vp, tables, bad, 4))
+
+
 def test_scatter_verify_bit_exact_and_lengths():
     from acorninfer_amd.cache.pager import BlockAllocator, PagedCacheView, PagedKVCache
     KV, D, P, m = 8, 128, 16, 5
