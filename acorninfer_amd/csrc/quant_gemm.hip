@@ -942,7 +942,8 @@ int dense8_splits(int64_t M, int64_t N, int64_t K) {
 // the larger has left after its full rounds. This predicts the measured times
 // within 10%: 1000 rows, mid / large, qkv 74 / 77 us, o 40 / 56, gate|up 236 /
 // 225, down 112 / 109; gate|up at 700 rows 186 / 218, at 2000 477 / 361; at 4502
-// rows o 213 / 222 and @SPLIT8@ for 4096 of them on the large one.
+// rows o 213 / 222. Dividing the rows there (14 of 18 row tiles of o and down on
+// the large one) took a prefill of those rows, two layers, from 5290 to 4890 us.
 // False: the mid-M kernel. Else *ks splits, *first row tiles on the large one.
 bool dense8_choice(int64_t M, int64_t N, int64_t K, int* ks, int* first) {
   const int mtiles = (int)((M + 255) / 256);
