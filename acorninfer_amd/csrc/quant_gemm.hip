@@ -1064,14 +1064,19 @@ int make_plan(int64_t M, int64_t N, int64_t K, int wfmt, const int* cfg, Tiling*
   if (wfmt == ACORN_WFMT_W8B &&
       (req8 || (no_request && (swiglu ? M >= kDenseLdsM : N % 128 == 0 && M >= kDenseMinM)))) {
     const int mtiles = (int)((M + 255) / 256);
-    int ks = req8 && cfg[3] > 0 ? cfg[3] : 1, first = mtiles;
-    if (req8 && cfg[4] > 0) first = std::min(cfg[4], mtiles);
+    int ks = 1, first = mtiles;
+    bool large = true;
+    if (req8) {
+      // rows divided between the two kernels share one plane: one split
+      if (cfg[4] > 0) first = std::min(cfg[4], mtiles);
+      if (cfg[3] > 0) ks = cfg[3];
+      else if (!swiglu && first == mtiles) ks = dense8_splits(M, N, K);
+    } else if (!swiglu) {
+      large = dense8_choice(M, N, K, &ks, &first);
+    }
     const bool form = !req8 || ((cfg[1] == 0 || cfg[1] == 256) && (cfg[2] == 0 || cfg[2] == 128) &&
                                 (first == mtiles || (ks == 1 && !swiglu && N % 256 == 0 &&
                                                      K % 512 == 0)));
-    bool large = true;
-    if (!swiglu && !(req8 && cfg[3] > 0)) ks = dense8_splits(M, N, K);
-    if (!req8 && !swiglu) large = dense8_choice(M, N, K, &ks, &first);
     if (large && form && dense_gemm8_supported(N, K, ks, swiglu)) {
       const int64_t ntiles = (N + 255) / 256;
       t->kind = 8;

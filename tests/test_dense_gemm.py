@@ -306,3 +306,44 @@ def test_default_tilings_of_the_block_layouts_are_launchable(N, K):
             t, tiles = plan(M, N, K, fmt)
             assert tiles >= 1 and t.ksplit >= 1
             assert plan(M, N, K, fmt, t)[0] == t, (fmt, M, t)
+
+
+@pytest.mark.parametrize("M,N,K", [(512, 4096, 4096), (1100, 1024, 4096), (300, 4096, 12288),
+                                   (1000, 6144, 4096), (257, 1024, 3072), (700, 1040, 512)])
+def test_partial_large_m_int8_requests_resolve_to_launchable_plans(M, N, K):
+    """Requests for the large-M int8 kernel that leave entries to the planner: a
+    division of the rows between the two kernels has one split (they share the
+    output's rows, not its planes), a requested split or division is the one
+    planned, and the resolved plan asked for again is itself (no GPU)."""
+    from acorninfer_amd._lib import WFMT_W8B
+    from acorninfer_amd.ops.quant_gemm import Tiling, plan
+    mtiles = -(-M // 256)
+    for upw in (0, 256):
+        for nw in (0, 128):
+            for ks in (0, 1, 2, 4):
+                for first in (0, 1, 2, mtiles - 1, mtiles, mtiles + 3):
+                    req = Tiling(DENSE_RT, upw, nw, ks, first)
+                    try:
+                        t, _ = plan(M, N, K, WFMT_W8B, req)
+                    except NotImplementedError:
+                        continue
+                    assert t.tpw == (min(first, mtiles) if first else mtiles), (req, t)
+                    assert t.tpw == mtiles or t.ksplit == 1, (req, t)
+                    assert ks == 0 or t.ksplit == ks, (req, t)
+                    assert plan(M, N, K, WFMT_W8B, t)[0] == t, (req, t)
+
+
+@pytest.mark.gpu
+def test_w8b_divided_rows_with_the_split_left_open():
+    """A request that divides the rows and leaves the split to the planner, at a
+    size where the undivided launch would split K: float64 (one bf16 rounding of
+    fp32 sums), and the explicit one-split request bit for bit."""
+    from acorninfer_amd.ops.quant_gemm import Tiling
+    M, N, K = 300, 512, 1024
+    lin, q, scale = _w8b(N, K, 5)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(6)).bfloat16().cuda()
+    assert lin.plan(M, Tiling(DENSE_RT, 0, 0, 0, 0))[0].ksplit > 1
+    want = x.double() @ (q.cuda().double() * scale.cuda().double()[:, None]).t()
+    out = _launch8(lin, x, Tiling(DENSE_RT, 0, 0, 0, 1), False)
+    assert ((out.double() - want).norm() / want.norm()) < 4e-3
+    assert torch.equal(out, _launch8(lin, x, Tiling(DENSE_RT, 0, 0, 1, 1), False))
