@@ -1041,9 +1041,10 @@ int make_plan(int64_t M, int64_t N, int64_t K, int wfmt, const int* cfg, Tiling*
   t->kind = 0;
   const bool no_request = !cfg || (cfg[0] == 0 && cfg[1] == 0 && cfg[2] == 0 && cfg[3] <= 1 &&
                                    cfg[4] == 0);
-  if (wfmt == ACORN_WFMT_W8 && !swiglu && M <= 16 &&
-      (!cfg || cfg[0] == kNatRT ||
-       (!cfg[0] && !cfg[1] && !cfg[2] && !cfg[3] && !cfg[4])) &&
+  // ... and no split either: one split asked for is a request (its caller may
+  // hold no workspace)
+  const bool nothing_set = no_request && (!cfg || cfg[3] == 0);
+  if (wfmt == ACORN_WFMT_W8 && !swiglu && M <= 16 && (nothing_set || cfg[0] == kNatRT) &&
       w8n_make_plan(M, N, K, &t->w8b)) {
     t->kind = 9;
     t->rt = kNatRT;
@@ -1062,7 +1063,8 @@ int make_plan(int64_t M, int64_t N, int64_t K, int wfmt, const int* cfg, Tiling*
   }
   const bool req8 = cfg && cfg[0] == kDenseRT;
   if (wfmt == ACORN_WFMT_W8B &&
-      (req8 || (no_request && (swiglu ? M >= kDenseLdsM : N % 128 == 0 && M >= kDenseMinM)))) {
+      (req8 || (swiglu ? no_request && M >= kDenseLdsM
+                       : nothing_set && N % 128 == 0 && M >= kDenseMinM))) {
     const int mtiles = (int)((M + 255) / 256);
     int ks = 1, first = mtiles;
     bool large = true;
@@ -1101,7 +1103,7 @@ int make_plan(int64_t M, int64_t N, int64_t K, int wfmt, const int* cfg, Tiling*
     }
     if (req8) return ACORN_ERR_UNSUPPORTED;
   }
-  if ((!cfg || (!cfg[0] && !cfg[1] && !cfg[2] && !cfg[3] && !cfg[4])) &&
+  if (nothing_set &&
       (wfmt == ACORN_WFMT_W4B || wfmt == ACORN_WFMT_W8B ||
        (wfmt == ACORN_WFMT_BF16B && M <= 16))) {
     int d[5];
