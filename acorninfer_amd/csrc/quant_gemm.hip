@@ -1128,8 +1128,8 @@ int make_plan(int64_t M, int64_t N, int64_t K, int wfmt, const int* cfg, Tiling*
     // only; wn 128 the direct-to-LDS form, a 4-stage ring)
     const int depth = req && cfg[4] > 0 ? cfg[4] : bm == 256 ? (wn == 128 ? 4 : 2) : 4;
     const int ntile = bm == 256 ? 256 : 4 * wn;    // weight rows per workgroup
-    int ks = req && cfg[3] > 0 ? cfg[3] : 1;
-    if (!(req && cfg[3] > 0) && !swiglu) {
+    int ks = cfg && cfg[3] > 0 ? cfg[3] : 1;
+    if (!(cfg && cfg[3] > 0) && !swiglu) {
       // split K while the launch has fewer workgroups than CUs; the 256 x 256
       // form (one workgroup per CU) stops before a second round of workgroups:
       // at M = 512 / 2048 one round with fewer splits measured faster (qkv

@@ -351,11 +351,14 @@ def test_w8b_divided_rows_with_the_split_left_open():
 
 @pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 4096), (24576, 4096), (4096, 12288),
                                  (1024, 3072), (1152, 4096), (2048, 384)])
-def test_one_split_asked_for_is_one_split_on_int8_blocks(N, K):
+def test_one_split_asked_for_is_one_split_on_the_blocks(N, K):
     """ksplit 1 with all else left open is a request, whose caller may hold no
     workspace: it is planned as one split at every row count (no GPU)."""
-    from acorninfer_amd._lib import WFMT_W8B
+    from acorninfer_amd._lib import WFMT_BF16, WFMT_BF16B, WFMT_W4B, WFMT_W8B
     from acorninfer_amd.ops.quant_gemm import Tiling, plan
-    for M in (1, 8, 16, 17, 64, 255, 256, 300, 512, 1000, 2000, 8192):
-        t, _ = plan(M, N, K, WFMT_W8B, Tiling(0, 0, 0, 1, 0))
-        assert t.ksplit == 1, (M, t)
+    for fmt in (WFMT_W8B, WFMT_W4B, WFMT_BF16B, WFMT_BF16):
+        for M in (1, 8, 16, 17, 64, 255, 256, 300, 512, 1000, 2000, 8192):
+            if (fmt == WFMT_W4B and K % 512) or (fmt == WFMT_BF16 and M <= 16):
+                continue                   # no such blocks; K in pieces that fit the LDS
+            t, _ = plan(M, N, K, fmt, Tiling(0, 0, 0, 1, 0))
+            assert t.ksplit == 1, (fmt, M, t)
