@@ -59,8 +59,11 @@ DENSE_RT = -2
 # kernel's rate outweighs the extra pass over the weights: on MI355X eight
 # layers of a W4A16 8B prefill take, this way / on the int4 kernels, 3.61 /
 # 3.07 ms at 512 tokens, 4.27 / 3.93 at 640, 4.40 / 4.60 at 768 and 5.00 / 5.28
-# at 1024.
+# at 1024. Where there is no int4 form to prefer (weights of another row count
+# than 128s above 64 rows, the fused SwiGLU above 16) it is taken from
+# DEQUANT_M_ODD rows.
 DEQUANT_M_MIN = 704
+DEQUANT_M_ODD = 512
 DEQUANT_RT = -4
 # prefill blocks from this many rows run gate|up with the large-M kernel's
 # SwiGLU epilogue (act written directly: no fp32 gate|up output, no silu_mul);
@@ -204,15 +207,19 @@ class QLinear:
                 n += t.numel() * t.element_size()
         return n
 
+    def dequant_rows(self) -> int:
+        """Rows of x from which int4 weights take the dequantise route by default."""
+        return DEQUANT_M_MIN if self.N % 128 == 0 else DEQUANT_M_ODD
+
     def plan(self, M: int, tiling=None, workspace: bool = False):
         """(Tiling, output tiles) from the library planner. workspace: the
         caller holds a bf16 weight workspace, so int4 weights take the
-        dequantise + bf16 GEMM route by default from DEQUANT_M_MIN rows (a
+        dequantise + bf16 GEMM route by default from dequant_rows() rows (a
         DEQUANT_RT request takes it at any size)."""
         from acorninfer_amd.ops.quant_gemm import Tiling, plan
         if self.fmt == WFMT_W4B and (
                 (tiling is not None and tiling[0] == DEQUANT_RT) or
-                (workspace and (tiling is None or not any(tiling)) and M >= DEQUANT_M_MIN)):
+                (workspace and (tiling is None or not any(tiling)) and M >= self.dequant_rows())):
             rest = tuple(tiling[1:]) if tiling is not None else (0, 0, 0, 0)
             t, tiles = plan(M, self.N, self.K, WFMT_BF16, Tiling(DENSE_RT, *rest))
             return Tiling(DEQUANT_RT, *t[1:]), tiles
@@ -297,11 +304,12 @@ class QLinear:
 
     def swiglu_plan(self, M: int, tiling=None, workspace: bool = False):
         """As plan, for the fused gate|up + SwiGLU launch (int4 at prefill
-        sizes: dequantised onto the bf16 kernel's SwiGLU form)."""
+        sizes, from DEQUANT_M_ODD rows: dequantised onto the bf16 kernel's SwiGLU
+        form, the only one above 16 rows)."""
         from acorninfer_amd.ops.quant_gemm import Tiling, swiglu_plan
         if self.fmt == WFMT_W4B and (
                 (tiling is not None and tiling[0] == DEQUANT_RT) or
-                (workspace and (tiling is None or not any(tiling)) and M >= DEQUANT_M_MIN)):
+                (workspace and (tiling is None or not any(tiling)) and M >= DEQUANT_M_ODD)):
             rest = tuple(tiling[1:]) if tiling is not None else (0, 0, 0, 0)
             t, tiles = swiglu_plan(M, self.N, self.K, WFMT_BF16, Tiling(DENSE_RT, *rest))
             return Tiling(DEQUANT_RT, *t[1:]), tiles
@@ -403,7 +411,7 @@ class Qwen3DecodeModel:
         # the shapes (False: K3 with one row per prompt token)
         self.tiled_prefill = True
         # projections of prefill rows: "own" (bf16 on the library's large-M
-        # kernel; int4 dequantised onto it from DEQUANT_M_MIN rows) or "int4"
+        # kernel; int4 dequantised onto it, QLinear.dequant_rows()) or "int4"
         # (int4 weights on the int4 kernels at every size)
         self.prefill_gemm = "own"
         # prefill blocks whose qkv / o / down run on the large-M kernel in one
@@ -674,13 +682,13 @@ class Qwen3DecodeModel:
 
     def prefill_swiglu(self, rows: int) -> bool:
         """A prefill block of `rows` runs gate|up with the SwiGLU epilogue of
-        the large-M bf16 kernel (bf16 weights from PREFILL_SWIGLU_M rows, int4
-        dequantised onto it from DEQUANT_M_MIN), gate|up in the 16-row
-        interleave."""
+        the large-M kernel (bf16 and int8 weights from PREFILL_SWIGLU_M rows,
+        int4 dequantised onto the bf16 one from dequant_rows()), gate|up in the
+        16-row interleave."""
         gu = self.layers[0].gate_up
         return gu.il16 and rows >= PREFILL_SWIGLU_M and (
             gu.fmt in (WFMT_BF16, WFMT_BF16B, WFMT_W8B) or
-            (gu.fmt == WFMT_W4B and rows >= DEQUANT_M_MIN))
+            (gu.fmt == WFMT_W4B and rows >= gu.dequant_rows()))
 
     def fused_swiglu_possible(self, batch: int) -> bool:
         """The gate|up launch can carry the SwiGLU epilogue (decode sizes,

@@ -362,3 +362,23 @@ def test_one_split_asked_for_is_one_split_on_the_blocks(N, K):
                 continue                   # no such blocks; K in pieces that fit the LDS
             t, _ = plan(M, N, K, fmt, Tiling(0, 0, 0, 1, 0))
             assert t.ksplit == 1, (fmt, M, t)
+
+
+def test_int4_rows_without_an_int4_form_take_the_dequantise_route():
+    """W4B weights of another row count than 128s have no int4 form above 64
+    rows, the fused SwiGLU none above 16: a caller that holds a bf16 workspace gets
+    the dequantise route from 512 rows on (no GPU)."""
+    from acorninfer_amd._lib import WFMT_W4B
+    from acorninfer_amd.models.qwen3 import DEQUANT_M_MIN, DEQUANT_RT, QLinear
+    for N, K in ((1040, 512), (272, 1024), (576, 1024)):
+        lin = QLinear(WFMT_W4B, None, N, K, None)
+        for M in (512, 600, 703, 704, 5000):
+            assert lin.plan(M, workspace=True)[0].rt == DEQUANT_RT
+        with pytest.raises(NotImplementedError):
+            lin.plan(600)
+    for N in (1088, 1152):                            # the fused SwiGLU has no int4 form either
+        for M in (512, 703, 704):
+            lin = QLinear(WFMT_W4B, None, N, 512, None)
+            assert lin.swiglu_plan(M, workspace=True)[0].rt == DEQUANT_RT
+    assert lin.plan(DEQUANT_M_MIN - 1, workspace=True)[0].rt != DEQUANT_RT
+    assert lin.plan(DEQUANT_M_MIN, workspace=True)[0].rt == DEQUANT_RT
