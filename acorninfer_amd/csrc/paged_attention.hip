@@ -1313,6 +1313,17 @@ __device__ __forceinline__ PrefillSeq prefill_seq(const int32_t* row0, const int
   return s;
 }
 
+// Where the fp32 partials of row j of sequence n lie in a run's plane: by packed
+// q row, or by (n, j) where q has many rows that no sequence covers, whichever
+// plane is the smaller.
+__host__ __device__ __forceinline__ int64_t prefill_slots(int64_t N, int64_t R, int64_t max_nq) {
+  return R < N * max_nq ? R : N * max_nq;
+}
+__device__ __forceinline__ int64_t prefill_slot(int64_t N, int64_t R, int64_t max_nq, int n,
+                                                int row0, int j) {
+  return R < N * max_nq ? (int64_t)row0 + j : n * max_nq + j;
+}
+
 // ---------------------------------------------------------------------------
 // Prefill attention: query-tiled flash attention over the paged cache with a
 // causal mask, for a chunked prefill whose new rows' K/V are already in the
@@ -1595,7 +1606,7 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
   if (nvalid == 0) return;
   pv();
   if (SPLIT && total > cps) {                    // one run of several: its fp32 partial
-    const size_t slots = (size_t)gridDim.z * max_nq * H;
+    const size_t slots = (size_t)prefill_slots(gridDim.z, R, max_nq) * H;
     float2* ml = (float2*)(ws + (size_t)S * slots * D);
 #pragma unroll
     for (int qw = 0; qw < QW; ++qw) {
@@ -1603,7 +1614,8 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
       lt += __shfl_xor(lt, 16);
       lt += __shfl_xor(lt, 32);
       if (16 * qw + c < nvalid) {
-        const size_t slot = (size_t)sp * slots + ((size_t)n * max_nq + j0 + 16 * qw + c) * H + h;
+        const size_t slot = (size_t)sp * slots +
+                            (size_t)prefill_slot(gridDim.z, R, max_nq, n, row0, j0 + 16 * qw + c) * H + h;
 #pragma unroll
         for (int jj = 0; jj < DPL; ++jj)
           *(f32x4_t*)(ws + slot * D + 16 * jj + 4 * r) = acc[qw][jj];
@@ -1653,8 +1665,8 @@ __global__ __launch_bounds__(kPrefillCombineNT) void paged_prefill_combine_kerne
   // (rows placed past their table row's pages have more runs than the S planned
   // from the table: those past S were not launched and have no partials)
   const int ns = min((total + cps - 1) / cps, S);
-  const size_t slots = (size_t)gridDim.y * max_nq * H;
-  const size_t slot = ((size_t)n * max_nq + j) * H + h;
+  const size_t slots = (size_t)prefill_slots(gridDim.y, R, max_nq) * H;
+  const size_t slot = (size_t)prefill_slot(gridDim.y, R, max_nq, n, sq.row0, j) * H + h;
   const float2* ml = (const float2*)(ws + (size_t)S * slots * D) + slot;
   const float* src = ws + slot * D + d0;
   float M = -INFINITY;
@@ -1721,7 +1733,9 @@ PrefillPlan prefill_plan(int64_t N, int64_t R, int64_t max_nq, int64_t H, int64_
   if (S <= 1) return p;
   p.cps = (int)((chunks + S - 1) / S);
   p.S = (int)((chunks + p.cps - 1) / p.cps);
-  if (p.S > 1) p.ws_bytes = p.S * N * max_nq * H * (D + 2) * 4;
+  // (S tiles KV stays below 4 / 3 of the target and a tile has at most 256 rows
+  // of heads, so the partials take at most 1024 x 256 x (D + 2) floats, 136 MB)
+  if (p.S > 1) p.ws_bytes = p.S * prefill_slots(N, R, max_nq) * H * (D + 2) * 4;
   return p;
 }
 

@@ -210,6 +210,7 @@ SPLIT_CASES = [
     (64, 8, 64, 16, [(1500, 33), (0, 33)]),
     (8, 2, 128, 16, [(2500, 16)]),
     (4, 4, 64, 16, [(255, 2), (256, 1), (640, 7)]),
+    (16, 2, 128, 16, [(300 + i, 1) for i in range(9)] + [(500, 90)]),
 ]
 
 
@@ -272,3 +273,25 @@ def test_workspace_grows_no_further_than_its_split(max_nq, width):
         assert n.value % run == 0 and (n.value == 0 or 2 <= n.value // run <= 64)
         if N == 300:
             assert n.value == 0
+
+
+def test_workspace_holds_rows_and_not_padding():
+    """Ragged launches (no GPU): the workspace is whole runs of the rows that
+    exist, the packed ones or N x max_nq, whichever is less, and within the
+    planner's bound, however uneven the sequences are."""
+    import ctypes
+    from acorninfer_amd._lib import check, lib
+    n = ctypes.c_int64(-1)
+    split = 0
+    for H, KV, D in ((32, 8, 128), (16, 8, 128), (16, 2, 128), (8, 1, 64), (64, 8, 128)):
+        for N, R, max_nq in ((1, 100000, 16), (64, 963, 900), (32, 1031, 1000), (100, 440, 341),
+                             (16, 512, 497), (60, 1088, 1000), (300, 2300, 2000), (9, 9, 1),
+                             (2, 4096, 4095), (1, 1, 1)):
+            for width in (8, 512, 20000):
+                check(lib().acorn_paged_prefill_workspace(N, R, max_nq, H, KV, D, 16, width,
+                                                          ctypes.byref(n)), "workspace")
+                run = min(R, N * max_nq) * H * (D + 2) * 4
+                assert n.value % run == 0 and (n.value == 0 or 2 <= n.value // run <= 64)
+                assert n.value <= 1024 * 256 * (D + 2) * 4
+                split += n.value > 0
+    assert split > 40
