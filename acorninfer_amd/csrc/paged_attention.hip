@@ -1283,27 +1283,22 @@ int dispatch_d(int64_t D, int64_t rep, const void* q, const void* kp, const void
 }
 
 // One sequence of a prefill launch: its first q row, that row's position and
-// its rows. With no seq_nq every sequence is a window of max_nq rows at row
-// n max_nq and seq_pos0 holds its length, the window included (at most `cap`:
-// prefill_cap). Rows past q's R rows (or past max_nq) are not served, so bad
-// metadata cannot reach past q / out.
+// its rows. WIN (no seq_nq): every sequence is a window of max_nq rows at row
+// n max_nq and seq_pos0 holds its length, the window included, taken as at most
+// `cap`, the tokens its table row has pages for, as K3 takes it. (A template
+// parameter and not a test: one more min in the kernel of the prefill chunks
+// cost 8192 causal tokens 35 of 700 us.) Rows past q's R rows (or past max_nq)
+// are not served, so bad metadata cannot reach past q / out.
 struct PrefillSeq {
   int row0, pos0, nq;
 };
-// The window kernels (QW == 1) take a length as at most the tokens its table row
-// has pages for, as K3 does. The others do not: 8192 causal tokens, 32 / 8 heads,
-// take 731 us with the clamp in their kernel and 696 without, where the kernel
-// before the unconditional MFMAs takes 739 and 726 on the same cards.
-template <int QW>
-__host__ __device__ __forceinline__ int prefill_cap(int table_stride, int P) {
-  return QW == 1 ? table_stride * P : 0x7fffffff;
-}
+template <bool WIN>
 __device__ __forceinline__ PrefillSeq prefill_seq(const int32_t* row0, const int32_t* pos0,
                                                   const int32_t* nq, int n, int R, int max_nq,
                                                   int cap) {
   PrefillSeq s;
-  if (nq == nullptr) {
-    s = {n * max_nq, min(pos0[n], cap) - max_nq, max_nq};
+  if constexpr (WIN) {
+    s = {n * max_nq, min(max(pos0[n], 0), cap) - max_nq, max_nq};
     if (s.pos0 + max_nq <= 0) s.nq = 0;
   } else {
     s = {row0[n], pos0[n], nq[n]};
@@ -1364,14 +1359,15 @@ __device__ __forceinline__ int64_t prefill_slot(int64_t N, int64_t R, int64_t ma
 // divided into runs of `cps` chunks, one workgroup each; a tile of more than
 // one run leaves (acc, m, l) per run in fp32 for paged_prefill_combine_kernel,
 // and a run in which a query sees no key adds nothing (m stays -inf).
-// QW: 16-query blocks per wave; 1 for windows of at most 16 QG rows.
-template <typename T, int D, int REP, int QG, int KC, int QW, bool SPLIT>
+// QW: 16-query blocks per wave; 1 where no sequence has more than 16 QG rows.
+// WIN: windows (prefill_seq).
+template <typename T, int D, int REP, int QG, int KC, int QW, bool SPLIT, bool WIN>
 __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
     const T* __restrict__ q, const T* __restrict__ k_pages, const T* __restrict__ v_pages,
     const int32_t* __restrict__ tables, const int32_t* __restrict__ seq_row0,
     const int32_t* __restrict__ seq_pos0, const int32_t* __restrict__ seq_nq, T* __restrict__ out,
     int R, int H, int KV, int P, int num_blocks, int table_stride, float scale_log2, int max_nq,
-    int S, int cps, float* __restrict__ ws) {
+    int S, int cps, float* __restrict__ ws, int cap) {
   constexpr int NT = REP * QG * kWave;           // threads
   constexpr int KB = D / 32, DPL = D / 16;
   constexpr int KPITCH = 2 * D + 32;             // bytes per staged K row (padded)
@@ -1389,8 +1385,7 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
   const int r = lane >> 4, c = lane & 15;
   const int hq = wid % REP, sub = wid / REP;
   const int h = kvh * REP + hq;
-  const PrefillSeq sq = prefill_seq(seq_row0, seq_pos0, seq_nq, n, R, max_nq,
-                                    prefill_cap<QW>(table_stride, P));
+  const PrefillSeq sq = prefill_seq<WIN>(seq_row0, seq_pos0, seq_nq, n, R, max_nq, cap);
   const int pos0 = sq.pos0, row0 = sq.row0, nq = sq.nq;
   const int tile = SPLIT ? (gridDim.x - 1 - blockIdx.x) / S : gridDim.x - 1 - blockIdx.x;
   const int wg_j0 = tile * WQ;                                  // longest tiles first
@@ -1648,7 +1643,7 @@ constexpr int kPrefillChunk = 64;   // keys staged per barrier (32: 3% slower at
 // Merge of a split tile's partials: one group of D / 4 lanes per (row, head),
 // four dims per lane; tiles of one run were written by the kernel itself.
 constexpr int kPrefillCombineNT = 256;
-template <typename T, int D>
+template <typename T, int D, bool WIN>
 __global__ __launch_bounds__(kPrefillCombineNT) void paged_prefill_combine_kernel(
     const float* __restrict__ ws, const int32_t* __restrict__ seq_row0,
     const int32_t* __restrict__ seq_pos0, const int32_t* __restrict__ seq_nq, T* __restrict__ out,
@@ -1657,7 +1652,7 @@ __global__ __launch_bounds__(kPrefillCombineNT) void paged_prefill_combine_kerne
   const int n = blockIdx.y;
   const int pair = (int)(blockIdx.x * (kPrefillCombineNT / LPP)) + threadIdx.x / LPP;
   const int j = pair / H, h = pair % H, d0 = 4 * (threadIdx.x % LPP);
-  const PrefillSeq sq = prefill_seq(seq_row0, seq_pos0, seq_nq, n, R, max_nq, cap);
+  const PrefillSeq sq = prefill_seq<WIN>(seq_row0, seq_pos0, seq_nq, n, R, max_nq, cap);
   if (j >= sq.nq) return;
   const int L = sq.pos0 + min(j / WQ * WQ + WQ, sq.nq);
   const int total = (L + kPrefillChunk - 1) / kPrefillChunk;
@@ -1750,38 +1745,42 @@ struct PrefillArgs {
   hipStream_t st;
 };
 
-template <typename T, int D, int REP, int QW, bool SPLIT>
+template <typename T, int D, int REP, int QW, bool SPLIT, bool WIN>
 int launch_prefill(const PrefillArgs& a) {
   // four waves per workgroup (eight for 8 q heads per kv head), 16 QW query rows each
   constexpr int QG = REP >= 4 ? 1 : 4 / REP;
   constexpr int WQ = 16 * QW * QG;
   const int64_t tiles = (a.max_nq + WQ - 1) / WQ;
   const int S = SPLIT ? a.plan.S : 1;
-  paged_prefill_kernel<T, D, REP, QG, kPrefillChunk, QW, SPLIT>
+  const int cap = (int)std::min<int64_t>(a.table_stride * a.P, 0x7fffffff);
+  paged_prefill_kernel<T, D, REP, QG, kPrefillChunk, QW, SPLIT, WIN>
       <<<dim3((unsigned)(tiles * S), (unsigned)a.KV, (unsigned)a.N), dim3(REP * QG * kWave), 0,
          a.st>>>((const T*)a.q, (const T*)a.kp, (const T*)a.vp, a.tables, a.row0, a.pos0, a.nq,
                  (T*)a.out, (int)a.R, (int)a.H, (int)a.KV, (int)a.P, (int)a.num_blocks,
-                 (int)a.table_stride, a.scale * kLog2e, (int)a.max_nq, S, a.plan.cps, a.ws);
+                 (int)a.table_stride, a.scale * kLog2e, (int)a.max_nq, S, a.plan.cps, a.ws, cap);
   ACORN_LAUNCH_CHECK();
   if (SPLIT) {
     constexpr int pairs = kPrefillCombineNT / (D / 4);
-    paged_prefill_combine_kernel<T, D>
+    paged_prefill_combine_kernel<T, D, WIN>
         <<<dim3((unsigned)((a.max_nq * a.H + pairs - 1) / pairs), (unsigned)a.N),
            dim3(kPrefillCombineNT), 0, a.st>>>(a.ws, a.row0, a.pos0, a.nq, (T*)a.out, (int)a.R,
-                                               (int)a.H, (int)a.max_nq, S, a.plan.cps, WQ,
-                                               prefill_cap<QW>((int)a.table_stride, (int)a.P));
+                                               (int)a.H, (int)a.max_nq, S, a.plan.cps, WQ, cap);
     ACORN_LAUNCH_CHECK();
   }
   return ACORN_OK;
 }
 
-template <typename T, int D, int REP>
+template <typename T, int D, int REP, bool WIN>
 int prefill_form(const PrefillArgs& a) {
   if (a.plan.S > 1)
-    return a.plan.qw == 1 ? launch_prefill<T, D, REP, 1, true>(a)
-                          : launch_prefill<T, D, REP, 2, true>(a);
-  return a.plan.qw == 1 ? launch_prefill<T, D, REP, 1, false>(a)
-                        : launch_prefill<T, D, REP, 2, false>(a);
+    return a.plan.qw == 1 ? launch_prefill<T, D, REP, 1, true, WIN>(a)
+                          : launch_prefill<T, D, REP, 2, true, WIN>(a);
+  return a.plan.qw == 1 ? launch_prefill<T, D, REP, 1, false, WIN>(a)
+                        : launch_prefill<T, D, REP, 2, false, WIN>(a);
+}
+template <typename T, int D, int REP>
+int prefill_form(const PrefillArgs& a) {
+  return a.nq ? prefill_form<T, D, REP, false>(a) : prefill_form<T, D, REP, true>(a);
 }
 
 template <typename T, int D>

@@ -132,6 +132,25 @@ def test_length_past_its_table_row_leaves_the_other_sequences():
     assert torch.equal(out, paged_verify_attention(q, kp, vp, tables, bad, 4))
 
 
+@pytest.mark.parametrize("hist", [40, 900])          # one run of keys, several
+def test_long_window_length_past_its_table_row(hist):
+    """The same for windows of more rows than one 16-query block per wave, whose
+    launches are another form of the kernel."""
+    from acorninfer_amd.ops.paged_attention import prefill_workspace
+    from acorninfer_amd.ops.paged_verify import paged_verify_attention
+    B, M, H, KV, D, P = 3, 20, 32, 8, 128, 16
+    q, kp, vp, tables, lens = _gpu(*_inputs(B, M, hist, torch.bfloat16, H=H, KV=KV, D=D))
+    W = tables.shape[1]
+    assert (prefill_workspace(B, B * M, M, H, KV, D, P, W, "cuda") is not None) == (hist == 900)
+    good = paged_verify_attention(q, kp, vp, tables, lens, 4)
+    bad = lens.clone()
+    bad[1] = 8 * W * P
+    out = paged_verify_attention(q, kp, vp, tables, bad, 4)
+    assert torch.equal(out[[0, 2]], good[[0, 2]])
+    bad[1] = W * P
+    assert torch.equal(out, paged_verify_attention(q, kp, vp, tables, bad, 4))
+
+
 def test_scatter_verify_bit_exact_and_lengths():
     from acorninfer_amd.cache.pager import BlockAllocator, PagedCacheView, PagedKVCache
     KV, D, P, m = 8, 128, 16, 5
