@@ -1299,7 +1299,6 @@ __device__ __forceinline__ PrefillSeq prefill_seq(const int32_t* row0, const int
   PrefillSeq s;
   if constexpr (WIN) {
     s = {n * max_nq, min(max(pos0[n], 0), cap) - max_nq, max_nq};
-    if (s.pos0 + max_nq <= 0) s.nq = 0;
   } else {
     s = {row0[n], pos0[n], nq[n]};
     if (s.row0 < 0 || s.pos0 < 0) s.nq = 0;
@@ -1398,8 +1397,21 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
   const int sp = SPLIT ? (gridDim.x - 1 - blockIdx.x) % S : 0;
   const int cb = SPLIT ? sp * cps : 0;
   const int nchunks = SPLIT ? min(cb + cps, total) : total;
-  // (uniform over the workgroup; no keys at all: a window longer than its sequence)
-  if (cb >= nchunks) return;
+  if (cb >= nchunks) {                           // uniform over the workgroup
+    // a window's tile before its sequence's first token sees no key: 0 / 0, as K3
+    // gives (a row of a tile that has keys comes to it by itself)
+    if (WIN && total <= 0 && sp == 0) {
+#pragma unroll
+      for (int qw = 0; qw < QW; ++qw)
+        if (16 * qw + c < nvalid) {
+          T* o = out + ((size_t)(row0 + j0 + 16 * qw + c) * H + h) * D + 4 * r;
+#pragma unroll
+          for (int jj = 0; jj < DPL; ++jj)
+            *(u32x2_t*)(o + 16 * jj) = u32x2_t{pack2<T>(NAN, NAN), pack2<T>(NAN, NAN)};
+        }
+    }
+    return;
+  }
   const int32_t* trow = tables + (size_t)n * table_stride;
   const int pshift = __builtin_ctz(P);
   const int tok_stride = KV * D;

@@ -34,8 +34,10 @@ def paged_verify_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torc
     """q [B, m, H, D] (normed + roped, positions len .. len+m-1); k/v_pages
     [NB, P, KV, D] (read only); tables [B, MP] int32; seq_lens [B] int32 =
     len + m. Returns [B, m, H, D] in q.dtype: row j is the window-causal
-    attention output at position len + j. Shape contracts raise
-    AssertionError as the reference's do (paged_verify.py:110-118)."""
+    attention output at position len + j (a row that sees no token is NaN).
+    num_splits applies to the K3 form; the prefill kernel plans its own. Shape
+    contracts raise AssertionError as the reference's do (paged_verify.py:
+    110-118)."""
     require_gpu(q, k_pages, v_pages, tables, seq_lens)
     B, M, H, D = q.shape
     NB, P, KV, _ = k_pages.shape

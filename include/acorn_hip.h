@@ -238,7 +238,8 @@ int acorn_paged_prefill_attention(const void* q, const void* k_pages, const void
  * NULL or too small, nothing is split. seq_row0 and seq_nq both NULL: every
  * sequence is a window of max_nq rows at row n * max_nq (R == N * max_nq), and
  * seq_pos0[n] is its length, the window included (the verify attention of
- * acorninfer/ops/paged_verify.py:96-123; >= max_nq).
+ * acorninfer/ops/paged_verify.py:96-123), taken as at most the tokens its table
+ * row has pages for; a row that sees no token is NaN.
  */
 int acorn_paged_prefill_attention_ws(const void* q, const void* k_pages, const void* v_pages,
                                      const int32_t* tables, const int32_t* seq_row0,

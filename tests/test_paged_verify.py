@@ -151,6 +151,34 @@ def test_long_window_length_past_its_table_row(hist):
     assert torch.equal(out, paged_verify_attention(q, kp, vp, tables, bad, 4))
 
 
+def _k3_rows(q, kp, vp, tables, lens, m):
+    """The window's rows one by one through decode (K3): row (b, j) at its own
+    visible length."""
+    from acorninfer_amd.ops.paged_attention import paged_decode_attention
+    B, _, H, D = q.shape
+    back = torch.arange(m - 1, -1, -1, device=lens.device, dtype=torch.int32)
+    rows = (lens[:, None] - back).reshape(-1).contiguous()
+    return paged_decode_attention(q.reshape(B * m, H, D).contiguous(), kp, vp,
+                                  tables.repeat_interleave(m, 0), rows, 2).view(B, m, H, D)
+
+
+@pytest.mark.parametrize("m,hist", [(5, 40), (5, 900), (20, 40), (20, 900), (70, 900)])
+def test_rows_that_see_no_token_are_nan(m, hist):
+    """Sequences of no token, of fewer than the window (its first rows see none)
+    and whole ones: every row is written, NaN where K3's is (0 / 0), one run of
+    keys and several, one query tile and more."""
+    from acorninfer_amd.ops.paged_verify import paged_verify_attention
+    q, kp, vp, tables, lens = _gpu(*_inputs(4, m, hist, torch.bfloat16, H=32, KV=8, D=128))
+    lens[0], lens[1], lens[2] = 0, 3, m - 1
+    want = _k3_rows(q, kp, vp, tables, lens, m)
+    stale = torch.full_like(q, 7.0)                    # what an unwritten row would show
+    del stale
+    out = paged_verify_attention(q, kp, vp, tables, lens, 2)
+    assert torch.equal(out.isnan(), want.isnan())
+    assert bool(out[0].isnan().all()) and not bool(out[3].isnan().any())
+    torch.testing.assert_close(out.float(), want.float(), equal_nan=True, **TOL_BF16)
+
+
 def test_scatter_verify_bit_exact_and_lengths():
     from acorninfer_amd.cache.pager import BlockAllocator, PagedCacheView, PagedKVCache
     KV, D, P, m = 8, 128, 16, 5
