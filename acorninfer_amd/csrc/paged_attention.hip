@@ -1282,6 +1282,11 @@ int dispatch_d(int64_t D, int64_t rep, const void* q, const void* kp, const void
   return ACORN_ERR_UNSUPPORTED;
 }
 
+// Exponent fields of two values of T in a word: all ones is an infinity or NaN.
+template <typename T> constexpr uint32_t kExpMask = 0;
+template <> constexpr uint32_t kExpMask<__bf16> = 0x7F807F80u;
+template <> constexpr uint32_t kExpMask<_Float16> = 0x7C007C00u;
+
 // One sequence of a prefill launch: its first q row, that row's position and
 // its rows. WIN (no seq_nq): every sequence is a window of max_nq rows at row
 // n max_nq and seq_pos0 holds its length, the window included, taken as at most
@@ -1460,6 +1465,37 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
       *(u32x4_t*)(kvs[b] + KC * KPITCH + poff0 + i * RSTEP * VPITCH) = stage[PH + i];
     }
   };
+  // WIN: a window's rows may hold anything after a query (a drafted token whose
+  // k / v overflowed), and P = 0 times an infinity is NaN: in the V rows behind the
+  // tile's first query (and past the last key) infinities and NaN become 0 once
+  // they are staged, before the barrier; `odd` remembers per wave that there were
+  // some, and the queries that see them add them at the end. Only a tile's last
+  // chunks hold such rows (8 windows of 5 rows over 1024..8192 keys: 38.0 us, 37.3
+  // without).
+  const int t_own = pos0 + wg_j0;                // the tile's first query
+  __shared__ int odd[WIN ? NT / kWave : 1];
+  if (WIN && lane == 0) odd[wid] = 0;
+  auto mend_chunk = [&](int b, int chunk) {
+    if (!WIN || chunk * KC + KC - 1 <= t_own) return;
+    constexpr uint32_t ones = kExpMask<T> & 0xffffu;
+    bool found = false;
+#pragma unroll
+    for (int i = 0; i < PH; ++i) {
+      if (chunk * KC + prow0 + i * RSTEP <= t_own) continue;
+      u32x4_t* at = (u32x4_t*)(kvs[b] + KC * KPITCH + poff0 + i * RSTEP * VPITCH);
+      u32x4_t v = *at;
+      bool here = false;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const bool lo = (v[w] & ones) == ones, hi = (v[w] >> 16 & ones) == ones;
+        here |= lo || hi;
+        v[w] &= (lo ? 0u : 0xffffu) | (hi ? 0u : 0xffff0000u);
+      }
+      if (here) *at = v;
+      found |= here;
+    }
+    if (__any(found) && lane == 0) odd[wid] = 1;
+  };
 
   float m[QW], l[QW], nm[QW];                    // nm: -m (0 while m is -inf)
   f32x4_t acc[QW][DPL];
@@ -1592,6 +1628,7 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
 #pragma unroll
   for (int i = 0; i < PH; ++i) pg_next[i] = page_of(min(cb + 1, nchunks - 1), i);
   store_chunk(0);
+  mend_chunk(0, cb);
   load_chunk(min(cb + 1, nchunks - 1), pg_next);
   __syncthreads();
   for (int ci = cb; ci < nchunks; ++ci) {
@@ -1608,10 +1645,35 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
     store_chunk(b ^ 1);                         // chunk ci + 1 (its buffer was last read in ci - 1)
     __builtin_amdgcn_sched_barrier(0);
     load_chunk(min(ci + 2, nchunks - 1), pg);
+    if (WIN && ci + 1 < nchunks) mend_chunk(b ^ 1, ci + 1);
     __syncthreads();
   }
   if (nvalid == 0) return;
   pv();
+  int any_odd = 0;
+  if (WIN && nchunks * KC - 1 > t_own) {
+#pragma unroll
+    for (int w = 0; w < NT / kWave; ++w) any_odd |= odd[w];
+  }
+  if (WIN && __builtin_expect(any_odd, 0)) {                          // what store_chunk took out, where it is seen
+#pragma unroll
+    for (int qw = 0; qw < QW; ++qw) {
+      const int te = min(pc[qw], nchunks * KC - 1);
+      for (int t = max(t_own + 1, cb * KC); t <= te; ++t) {
+        const unsigned pt = (unsigned)trow[min(t >> pshift, table_stride - 1)];
+        const size_t pg_t = pt < (unsigned)num_blocks ? pt : 0u;
+        const T* vr = v_pages + (pg_t * P + (t & (P - 1))) * tok_stride + (size_t)kvh * D + 4 * r;
+#pragma unroll
+        for (int jj = 0; jj < DPL; ++jj) {
+          T v4[4];
+          __builtin_memcpy(v4, vr + 16 * jj, sizeof(v4));
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (!(fabsf(to_f32(v4[i])) < INFINITY)) acc[qw][jj][i] += to_f32(v4[i]);
+        }
+      }
+    }
+  }
   if (SPLIT && total > cps) {                    // one run of several: its fp32 partial
     const size_t slots = (size_t)prefill_slots(gridDim.z, R, max_nq) * H;
     float2* ml = (float2*)(ws + (size_t)S * slots * D);

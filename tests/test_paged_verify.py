@@ -179,6 +179,43 @@ def test_rows_that_see_no_token_are_nan(m, hist):
     torch.testing.assert_close(out.float(), want.float(), equal_nan=True, **TOL_BF16)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,KV,D,m,hist", [(32, 8, 128, 5, 40), (32, 8, 128, 5, 900),
+                                           (32, 8, 128, 40, 900), (8, 8, 64, 7, 60),
+                                           (64, 8, 128, 20, 300), (16, 8, 64, 70, 35)])
+def test_rows_do_not_see_later_v_whatever_it_holds(H, KV, D, m, hist, dtype):
+    """Infinities and NaN in V of drafted tokens and of the history reach exactly
+    the rows that see them, as K3's rows show; the rows before keep their bits.
+    Windows inside one query tile and over several (of 16 to 64 rows, by the GQA
+    ratio), their keys in one run and in several, across a run's border."""
+    from acorninfer_amd.ops.paged_verify import paged_verify_attention
+    q, kp, vp, tables, lens = _inputs(3, m, hist, dtype, H=H, KV=KV, D=D)
+    mp = tables.shape[1]                               # pages of their own
+    tables = torch.randperm(3 * mp).view(3, mp).to(torch.int32)
+    kp, vp = (torch.cat([t[:mp]] * 3) for t in (kp, vp))
+    q, kp, vp, tables, lens = _gpu(q, kp, vp, tables, lens)
+    clean = paged_verify_attention(q, kp, vp, tables, lens, 2)
+    inf, nan = float("inf"), float("nan")
+
+    def put(b, t, kvh, dim, value):
+        vp[int(tables[b, t // 16]), t % 16, kvh, dim] = value
+    n0, n1, n2 = (int(n) for n in lens)
+    put(0, n0 - 1, 0, 3, inf)                          # the last drafted token
+    put(0, n0 - 2, KV - 1, slice(None), nan)
+    put(1, n1 - m + 1, 0, 17, -inf)                    # the second one
+    put(1, n1 - 1, 0, 17, inf)                         # both signs: NaN from there
+    put(1, n1 - m // 2, 1, 40, nan)
+    put(2, n2 - m, 0, 0, inf)                          # the window's first: every row
+    put(2, hist // 2, 1, 5, nan)                       # history: every row
+    want = _k3_rows(q, kp, vp, tables, lens, m)
+    out = paged_verify_attention(q, kp, vp, tables, lens, 2)
+    ok = want.isfinite()
+    assert torch.equal(out.isfinite(), ok) and bool((~ok).any())
+    assert torch.equal(out[ok], clean[ok])
+    assert torch.equal(out[0, :m - 2], clean[0, :m - 2])
+    assert torch.equal(out == inf, want == inf) and torch.equal(out == -inf, want == -inf)
+
+
 def test_scatter_verify_bit_exact_and_lengths():
     from acorninfer_amd.cache.pager import BlockAllocator, PagedCacheView, PagedKVCache
     KV, D, P, m = 8, 128, 16, 5
