@@ -525,7 +525,9 @@ __global__ __launch_bounds__(NW * 64, 1) void dense_dl_kernel(const __bf16* __re
 //    refilled for both halves of the next pair after its own last use;
 //  * 8 bytes become an operand in 14 VALU instructions (xor, signed byte
 //    conversions, packs) beside the 4 MFMAs it feeds.
-template <typename OUT, bool SWIGLU>
+// DMA false: x or weights off 16-byte alignment, which the loads into LDS are not
+// specified for: the same bytes by way of registers, waited for at once.
+template <typename OUT, bool SWIGLU, bool DMA>
 __global__ __launch_bounds__(512, 1) void dense_dl8_kernel(const __bf16* __restrict__ x,
                                                            const uint8_t* __restrict__ w,
                                                            const _Float16* __restrict__ scale,
@@ -575,11 +577,17 @@ __global__ __launch_bounds__(512, 1) void dense_dl8_kernel(const __bf16* __restr
 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)(&lds[0][0]);
   auto dma = [&](const uint8_t* src, uint32_t dst) {
+    if constexpr (DMA) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                 :: "v"(src), "s"(dst) : "memory", "m0");
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                   :: "v"(src), "s"(dst) : "memory", "m0");
 #pragma clang diagnostic pop
+    } else {
+      u32x4 v;
+      __builtin_memcpy(&v, src, sizeof(v));
+      *(u32x4*)(&lds[0][0] + (dst - lds0) + 16 * lane) = v;
+    }
   };
   const int pairs = steps / 2;
   auto issue_one = [&](int d, int i) {         // load i of pair d: weights, then x
@@ -815,12 +823,18 @@ int dense_gemm8_launch(const void* x, const void* w, const void* scale, void* ou
   const __bf16* xp = (const __bf16*)x;
   const uint8_t* wp = (const uint8_t*)w;
   const _Float16* sp = (const _Float16*)scale;
+  auto launch = [&](auto kernel, auto* out) {
+    kernel<<<grid, block, 0, st>>>(xp, wp, sp, out, (int)M, (int)N, (int)K, tn, tm, steps);
+  };
+  const bool dma = ((uintptr_t)x | (uintptr_t)w) % 16 == 0;   // (rows are whole 128-byte lines)
   if (out_f32)
-    dense_dl8_kernel<float, false><<<grid, block, 0, st>>>(xp, wp, sp, out_f32, (int)M, (int)N, (int)K, tn, tm, steps);
+    launch(dma ? dense_dl8_kernel<float, false, true> : dense_dl8_kernel<float, false, false>, out_f32);
   else if (swiglu)
-    dense_dl8_kernel<__bf16, true><<<grid, block, 0, st>>>(xp, wp, sp, (__bf16*)out_bf16, (int)M, (int)N, (int)K, tn, tm, steps);
+    launch(dma ? dense_dl8_kernel<__bf16, true, true> : dense_dl8_kernel<__bf16, true, false>,
+           (__bf16*)out_bf16);
   else
-    dense_dl8_kernel<__bf16, false><<<grid, block, 0, st>>>(xp, wp, sp, (__bf16*)out_bf16, (int)M, (int)N, (int)K, tn, tm, steps);
+    launch(dma ? dense_dl8_kernel<__bf16, false, true> : dense_dl8_kernel<__bf16, false, false>,
+           (__bf16*)out_bf16);
   return ACORN_OK;
 }
 

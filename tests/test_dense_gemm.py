@@ -382,3 +382,32 @@ def test_int4_rows_without_an_int4_form_take_the_dequantise_route():
             assert lin.swiglu_plan(M, workspace=True)[0].rt == DEQUANT_RT
     assert lin.plan(DEQUANT_M_MIN - 1, workspace=True)[0].rt != DEQUANT_RT
     assert lin.plan(DEQUANT_M_MIN, workspace=True)[0].rt == DEQUANT_RT
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,swiglu", [(513, 272, 256, False), (300, 512, 1024, False),
+                                          (600, 1056, 512, True)])
+def test_w8b_large_m_operands_at_any_address(M, N, K, swiglu):
+    """x one element and the weights one byte off their alignment, each and both
+    (loads straight into LDS need 16 bytes): bit for bit the aligned launch, in
+    bf16 and fp32, in one split and several."""
+    from acorninfer_amd._lib import stream_ptr
+    from acorninfer_amd.ops.quant_gemm import Tiling
+    lin, _, _ = _w8b(N, K, 3 * N)
+    lin.il16 = swiglu
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(9)).bfloat16().cuda()
+    xo = torch.empty(M * K + 1, dtype=x.dtype, device="cuda")[1:].view(M, K).copy_(x)
+    w, wo = lin.w, torch.empty(N * K + 1, dtype=lin.w.dtype, device="cuda")[1:].view(lin.w.shape)
+    wo.copy_(w)
+
+    def outs(xs, ws):
+        lin.w = ws
+        if swiglu:
+            act = torch.empty(M, N // 2, dtype=torch.bfloat16, device="cuda")
+            lin.launch_swiglu(xs, M, lin.swiglu_plan(M)[0], act, stream_ptr())
+            return [act]
+        return [_launch8(lin, xs, Tiling(DENSE_RT, 0, 0, ks, 0), ks == 2) for ks in (1, 2)]
+    want = outs(x, w)
+    for xs, ws in ((xo, w), (x, wo), (xo, wo)):
+        for a, b in zip(outs(xs, ws), want):
+            assert torch.equal(a, b)
