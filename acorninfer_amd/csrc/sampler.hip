@@ -517,6 +517,8 @@ constexpr int kSplitCap = kNT;       // listed elements per row (one per thread 
 // shorter rows: one workgroup reads them in less than four launches take
 constexpr int64_t kSplitMinV = 16384;
 constexpr int64_t kSplitMaxRows = 4096;  // bounds the workspace (34 KB per row)
+// masses of at most 2^40 each add up in 64 bits
+constexpr int64_t kSplitMaxV = (int64_t)1 << 23;
 
 enum { kRowDrawn = 0, kRowBad = 1, kRowGreedy = 2, kRowWhole = 3 };
 enum { kModeTopK = 0, kModeTopP = 1, kModeAll = 2 };
@@ -1188,7 +1190,7 @@ void launch_split(const SplitArgs& a, int64_t rows, hipStream_t st) {
 
 extern "C" int acorn_sample_workspace(int64_t rows, int64_t vocab, int64_t* bytes) {
   if (rows < 0 || vocab <= 0 || !bytes) return ACORN_ERR_VALUE;
-  *bytes = vocab >= kSplitMinV && vocab <= ((int64_t)1 << 31) && rows <= kSplitMaxRows
+  *bytes = vocab >= kSplitMinV && vocab <= kSplitMaxV && rows <= kSplitMaxRows
                ? rows * (int64_t)sizeof(SplitRow)
                : 0;
   return ACORN_OK;

@@ -439,7 +439,8 @@ int acorn_sample(const void* logits, int64_t rows, int64_t vocab, int dtype,
  * rounding of a boundary). ws is 64-byte aligned device memory of at least the
  * bytes acorn_sample_workspace reports for (rows, vocab); its contents need not
  * be set, and calls that overlap need workspaces of their own. Where it reports
- * 0 (short rows), or with ws NULL or too small, the call is acorn_sample.
+ * 0 (short rows; rows of more than 2^23 elements, whose masses could pass 64
+ * bits), or with ws NULL or too small, the call is acorn_sample.
  */
 int acorn_sample_split(const void* logits, int64_t rows, int64_t vocab, int dtype,
                        const float* temperature, const int32_t* top_k, const float* top_p,

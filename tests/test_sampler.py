@@ -230,3 +230,17 @@ def test_split_rows_equal_one_workgroup_rows(dtype, V):
     for _ in range(2):
         tok2, lp2, _ = sample_batch(rows, t, k, p, u)
         assert torch.equal(tok2, tok) and torch.equal(lp2.view(torch.int32), lp.view(torch.int32))
+
+
+def test_split_rows_are_those_whose_masses_add_up_in_64_bits():
+    """The split form's sums (no GPU): a row of V equal logits has mass V x 2^40,
+    which passes 2^64 from 2^24 elements; longer rows have no workspace and run
+    on the one-workgroup form, whose draw adds in fp32."""
+    import ctypes
+    from acorninfer_amd._lib import check, lib
+    n = ctypes.c_int64(-1)
+    for V, split in ((16383, False), (16384, True), (151936, True), (1 << 23, True),
+                     ((1 << 24) + 8, False), (1 << 31, False)):
+        check(lib().acorn_sample_workspace(3, V, ctypes.byref(n)), "workspace")
+        assert (n.value > 0) == split, V
+        assert not split or V * 2 ** 40 < 2 ** 64
