@@ -1,7 +1,7 @@
 // Token sampler: temperature -> top-k -> top-p -> draw. Long rows (a language
 // model's vocabulary) are split over kSplitG workgroups in four launches
-// (sample_*_kernel below); short rows, calls without a workspace and the few
-// rows the split form hands over run as one workgroup per row (sample_row).
+// (sample_*_kernel below); short and very long rows, calls without a workspace and
+// rows whose maximum / T overflows run as one workgroup per row (sample_row).
 //
 // Semantics follow acorninfer/sampler.py:38-68 (HF warper order):
 //   x = logits / T                                   (fp32)
@@ -505,8 +505,8 @@ __device__ void sample_row(
 // The selection is sample_row's, bit for bit: the same keys and the same
 // integer masses relative to the row's maximum. A bin is a monotone function
 // of x, so bins respect the key order. The draw adds integer masses instead of
-// fp32 ones. Rows whose boundary holds more elements than the lists (a large
-// top-k, many ties) or whose maximum overflows are left to sample_row.
+// fp32 ones. Where the boundary holds more elements than the lists (a large top-k,
+// many ties, a flat row) pick goes down the keys instead (split_descend).
 // Four launches of a few microseconds each, bound by their latency.
 constexpr int kSplitG = 32;          // workgroups (chunks) per row
 constexpr int kSplitNT = 1024;       // their threads
@@ -593,42 +593,41 @@ __device__ __forceinline__ void load8(const T* row, int64_t i, int64_t end, bool
   }
 }
 
-// Elements [c0, c1) of a row in groups of eight, kOct of a thread's groups
-// requested together. Rows whose groups are whole and 16-byte aligned (V % 8 ==
-// 0) are read as vectors, clamped to the last one so that every load is
-// unconditional; others element by element.
-constexpr int kOct = 1;
-template <typename T, int NT>
+// Elements [c0, c1) of a row in groups of eight, U of a thread's groups requested
+// together. Rows whose groups are whole and 16-byte aligned (V % 8 == 0) are read
+// as vectors, clamped to the last one so that every load is unconditional; others
+// element by element.
+template <typename T, int U = 1>
 struct Octets {
   static constexpr int E = 16 / sizeof(T), Q = 8 / E;
   const T* row;
   int64_t c0, c1, n;                    // the range and its groups
   bool fast;
-  u32x4v w[kOct][Q];
+  u32x4v w[U][Q];
   __device__ Octets(const T* row_, int64_t V, int64_t c0_, int64_t c1_)
       : row(row_), c0(c0_), c1(c1_), n((c1_ - c0_ + 7) / 8),
         fast(((uintptr_t)row_ % 16) == 0 && V % 8 == 0) {}
-  // request groups j0, j0 + stride, ... (kOct of them)
+  // request groups j0, j0 + stride, ... (U of them)
   __device__ __forceinline__ void load(int64_t j0, int64_t stride) {
     if (!fast || n == 0) return;
 #pragma unroll
-    for (int u = 0; u < kOct; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int q = 0; q < Q; ++q)
         w[u][q] = ((const u32x4v*)(row + c0 + min(j0 + u * stride, n - 1) * 8))[q];
 #pragma unroll
-    for (int u = 0; u < kOct; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int q = 0; q < Q; ++q) asm volatile("" ::"v"(w[u][q]));
   }
-  // f(index, value) of the groups j0, j0 + stride, ... < end; the first kOct
-  // have been requested by load(j0, stride)
+  // f(index, value) of the groups j0, j0 + stride, ... < end; the first U have
+  // been requested by load(j0, stride)
   template <typename F>
   __device__ __forceinline__ void each(int64_t j0, int64_t stride, int64_t end, F f) {
-    for (int64_t j = j0; j < end; j += kOct * stride) {
+    for (int64_t j = j0; j < end; j += U * stride) {
       if (j != j0) load(j, stride);
 #pragma unroll
-      for (int u = 0; u < kOct; ++u) {
+      for (int u = 0; u < U; ++u) {
         const int64_t ju = j + u * stride;
         if (ju >= end) continue;
         const int64_t i = c0 + ju * 8;
@@ -645,10 +644,6 @@ struct Octets {
           if (i + e < c1) f(i + e, v[e]);
       }
     }
-  }
-  template <typename F>
-  __device__ __forceinline__ void each(int64_t j0, int64_t stride, F f) {
-    each(j0, stride, n, f);
   }
 };
 
@@ -732,7 +727,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
   if (!(Tm > 0.f) && c != 0) return;
   const T* row = (const T*)a.logits + r * a.V;
   const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
-  Octets<T, kSplitNT> o(row, a.V, c0, c1);
+  Octets<T> o(row, a.V, c0, c1);
   // consecutive elements per thread: thread order is vocabulary order
   const int64_t seg = (o.n + kSplitNT - 1) / kSplitNT, end = min((tid + 1) * seg, o.n);
   o.load(tid * seg, 1);                  // in flight with the chunk maxima
@@ -799,11 +794,11 @@ __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
   __syncthreads();
   const int bin = sh_bin;
   uint32_t mine_n = 0, listed;
-  if (seg > kOct) o.load(tid * seg, 1);
+  if (seg > 1) o.load(tid * seg, 1);
   o.each(tid * seg, 1, end, [&](int64_t, float l) { mine_n += split_bin(l / Tm, M) <= bin; });
   uint32_t pos = block_scan<uint32_t, kSplitNT>(mine_n, upart, listed);
   if (mine_n && pos < (uint32_t)kSplitCapC) {
-    if (seg > kOct) o.load(tid * seg, 1);
+    if (seg > 1) o.load(tid * seg, 1);
     o.each(tid * seg, 1, end, [&](int64_t i, float l) {
       const float x = l / Tm;
       if (split_bin(x, M) <= bin) {
@@ -840,6 +835,194 @@ __device__ __forceinline__ void split_boundary(const unsigned long long (&h)[PER
   }
 }
 
+// The mass that top-p keeps at least, of the mass it chooses from.
+__device__ __forceinline__ unsigned long long split_goal(float p, unsigned long long z) {
+  return max(1ull, (unsigned long long)(fmax((double)p, 0.0) * (double)z));
+}
+
+// The lowest float that `ok`, a property of all floats from some one up to top, holds for.
+template <typename F>
+__device__ __forceinline__ float lowest_float(float top, F ok) {
+  uint32_t lo = okey(-3.402823466e38f), hi = okey(top);   // ok(hi)
+  while (lo < hi) {                                       // 64 candidates at a time
+    const uint32_t step = (hi - lo) / kWave + 1;
+    const uint64_t at = (uint64_t)lo + (threadIdx.x % kWave) * (uint64_t)step;
+    const uint32_t mine = at < hi ? (uint32_t)at : hi;
+    const uint64_t yes = __ballot(ok(key_float(mine)));
+    const int first = __ffsll((unsigned long long)yes) - 1;
+    if (first < 0) {
+      lo = __shfl(mine, kWave - 1) + 1;
+    } else {
+      hi = __shfl(mine, first);
+      if (first > 0) lo = __shfl(mine, first - 1) + 1;
+      else lo = hi;
+    }
+  }
+  return key_float(hi);
+}
+
+// A row whose boundary holds more elements than the lists: the kept set by radix
+// descent over the keys (11, 11 and 10 bits), as in sample_row, but from the
+// boundary bin the histogram has found: the elements outside it are told by one
+// comparison of the logit, rows are read as vectors, several in flight, and equal
+// neighbours (ties) are added once per wave. Returns (lowest kept key, first kept
+// index among its ties) and leaves the chunks' kept masses in cm, which holds
+// those above the bin (top-p) or 0. Bound by the VALU work per element of one CU per
+// row: 8 bf16 rows of 151936 with a spread of 2 around 8 (top-p 0.9 then ends in one
+// value of 1460 tokens) 179 us, on sample_row 612; top-k 5000 142, there 377.
+template <typename T>
+__device__ unsigned long long split_descend(const T* row, int64_t V, int64_t chunk, float Tm,
+                                            float M, float lmax, int mode, unsigned long long kk,
+                                            float pp, int bin, unsigned long long above,
+                                            unsigned long long zk, unsigned long long* part,
+                                            unsigned long long* cm) {
+  __shared__ unsigned long long hsum[kSplitNB], sh_above;
+  __shared__ uint32_t hcnt[kSplitNB], ties[kSplitG], sh_d, sh_tie0;
+  static_assert(kSplitNB == 2 * kNT, "two digits per thread");
+  const int tid = threadIdx.x, lane = tid % kWave, wid = tid / kWave;
+  Octets<T, 4> o(row, V, 0, V);
+  uint32_t key = 0, cnt = 0;                          // of the boundary
+  unsigned long long below = 0;                       // count or mass above it
+  // the key at which the running count (top-k) or mass from the highest key down
+  // passes `goal`, of logits in [lo, hi) with keys from kmin; `start` lies above them
+  auto descend = [&](float lo, float hi, uint32_t kmin, bool by_mass, unsigned long long goal,
+                     unsigned long long start) {
+    uint32_t prefix = 0, pmask = 0;
+    below = start;
+#pragma unroll 1
+    for (int shift = 21; shift >= 0; shift = shift == 21 ? 10 : shift - 10) {
+      const uint32_t digits = shift ? 2047u : 1023u;
+      for (int q = tid; q < kSplitNB; q += kNT) {
+        hsum[q] = 0;
+        hcnt[q] = 0;
+      }
+      if (tid == 0) sh_d = 0;
+      __syncthreads();
+      o.load(tid, kNT);
+      o.each(tid, kNT, o.n, [&](int64_t, float l) {
+        if (!(l >= lo && l < hi)) return;
+        const float x = l / Tm;
+        const uint32_t k = okey(x);
+        if (k < kmin || (k & pmask) != prefix) return;
+        const unsigned long long m = by_mass ? mass_fix(x, M) : 1ull;
+        const uint32_t k0 = __builtin_amdgcn_readfirstlane(k);
+        const uint64_t same = __ballot(k == k0);
+        const int d = (int)((k >> shift) & digits);
+        if (k != k0 || lane == __ffsll((unsigned long long)same) - 1) {
+          const uint32_t c = k == k0 ? (uint32_t)__popcll(same) : 1u;
+          atomicAdd(&hsum[d], c * m);
+          atomicAdd(&hcnt[d], c);
+        }
+      });
+      __syncthreads();
+      const int d1 = kSplitNB - 1 - 2 * tid;          // this thread's digits, highest first
+      const unsigned long long v1 = hsum[d1], v0 = hsum[d1 - 1];
+      unsigned long long total;
+      const unsigned long long run =
+          below + block_scan<unsigned long long, kNT>(v1 + v0, part, total);
+      if (run < goal && goal <= run + v1 + v0) {
+        sh_d = goal <= run + v1 ? d1 : d1 - 1;
+        sh_above = goal <= run + v1 ? run : run + v1;
+      }
+      __syncthreads();
+      prefix |= sh_d << shift;
+      pmask |= digits << shift;
+      below = sh_above;
+      cnt = hcnt[sh_d];
+      __syncthreads();
+    }
+    key = prefix;
+  };
+  auto in_bin = [&](int b) {
+    return lowest_float(lmax, [&](float l) { return split_bin(l / Tm, M) <= b; });
+  };
+  float lo = in_bin(bin), hi = bin > 0 ? in_bin(bin - 1) : INFINITY;
+  uint32_t keep = 0xffffffffu;                        // ties kept
+  unsigned long long goal = 0;
+  if (mode == kModeTopK) {
+    descend(lo, hi, 0u, false, kk, above);
+    const uint32_t kkey = key;
+    lo = lowest_float(lmax, [&](float l) { return okey(l / Tm) >= kkey; });
+    hi = INFINITY;
+    if (pp < 1.0f) {
+      unsigned long long sum = 0;
+      o.load(tid, kNT);
+      o.each(tid, kNT, o.n, [&](int64_t, float l) {
+        if (l >= lo && okey(l / Tm) >= kkey) sum += mass_fix(l / Tm, M);
+      });
+      block_scan<unsigned long long, kNT>(sum, part, zk);
+      goal = split_goal(pp, zk);
+      descend(lo, hi, kkey, true, goal, 0);
+    }
+  } else {
+    goal = split_goal(pp, zk);
+    descend(lo, hi, 0u, true, goal, above);
+  }
+  const unsigned long long m = mass_fix(key_float(key), M);
+  if (goal > 0 && m > 0) {
+    const double need = ceil(((double)goal - (double)below) / (double)m);
+    keep = (uint32_t)fmax(1.0, fmin(need, (double)cnt));
+  }
+  // per chunk, a wave each: its ties and the mass above them
+  for (int c = wid; c < kSplitG; c += kNT / kWave) {
+    const int64_t c0 = min(c * chunk, V), c1 = min(c0 + chunk, V);
+    Octets<T, 4> oc(row, V, c0, c1);
+    unsigned long long sum = 0;
+    uint32_t n = 0;
+    oc.load(lane, kWave);
+    oc.each(lane, kWave, oc.n, [&](int64_t, float l) {
+      if (!(l >= lo && l < hi)) return;
+      const float x = l / Tm;
+      const uint32_t k = okey(x);
+      if (k > key) sum += mass_fix(x, M);
+      n += k == key;
+    });
+    sum = wave_scan(sum);
+    n = wave_scan(n);
+    if (lane == kWave - 1) {
+      cm[c] += sum;
+      ties[c] = n;
+    }
+  }
+  if (tid == 0) sh_tie0 = 0;
+  __syncthreads();
+  // ties are kept from the highest index down: `drop` of them are not, the last of
+  // these in chunk `cut`
+  const uint32_t mine = lane < kSplitG ? ties[lane] : 0u, upto = wave_scan(mine);
+  const uint32_t all = __shfl(upto, kWave - 1), drop = keep < all ? all - keep : 0u;
+  const int cut = drop ? __ffsll((unsigned long long)__ballot(upto > drop)) - 1 : -1;
+  const uint32_t before = upto - mine;
+  if (tid < kSplitG) {
+    const uint32_t lost = drop > before ? min(drop - before, mine) : 0u;
+    cm[lane] += (mine - lost) * m;
+  }
+  if (cut >= 0) {                                     // the first kept tie's index
+    const uint32_t rank = drop - __shfl(before, cut);
+    const int64_t c0 = min(cut * chunk, V), c1 = min(c0 + chunk, V);
+    const bool aligned = ((uintptr_t)row % 16) == 0 && V % 8 == 0;
+    uint32_t base = 0;
+    for (int64_t t0 = c0; t0 < c1 && base <= rank; t0 += kNT * 8) {
+      const int64_t i = t0 + tid * 8;
+      float x[8];
+      uint32_t n = 0, tot;
+      if (i < c1) {
+        load8(row, i, c1, aligned, x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) n += i + e < c1 && okey(x[e] / Tm) == key;
+      }
+      uint32_t at = base + block_scan<uint32_t, kNT>(n, (uint32_t*)part, tot);
+      if (n && at <= rank && rank < at + n) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (i + e < c1 && okey(x[e] / Tm) == key && at++ == rank) sh_tie0 = (uint32_t)(i + e);
+      }
+      base += tot;
+    }
+  }
+  __syncthreads();
+  return (unsigned long long)key << 32 | sh_tie0;
+}
+
 template <typename T>
 __global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
   __shared__ unsigned long long part[kSplitNT / kWave];
@@ -857,7 +1040,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
   // holds consecutive elements, so that thread order is vocabulary order
   const T* row = (const T*)a.logits + r * a.V;
   const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
-  Octets<T, kSplitNT> o(row, a.V, c0, c1);
+  Octets<T> o(row, a.V, c0, c1);
   const int64_t seg = (o.n + kSplitNT - 1) / kSplitNT;
   o.load(tid * seg, 1);
   constexpr int kPer = kSplitNB / kSplitNT;
@@ -876,9 +1059,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
   for (int q = 0; q < kPer; ++q) mine += h[q];
   const unsigned long long run = block_scan<unsigned long long, kSplitNT>(mine, part, total);
   const unsigned long long goal =
-      mode == kModeTopK
-          ? (unsigned long long)a.top_k[r]
-          : max(1ull, (unsigned long long)(fmax((double)a.top_p[r], 0.0) * (double)total));
+      mode == kModeTopK ? (unsigned long long)a.top_k[r] : split_goal(a.top_p[r], total);
   split_boundary<kSplitNT, kPer>(h, run, mine, goal, &sh_bin, &sh_above);
   __syncthreads();
   const int bin = sh_bin;
@@ -1008,70 +1189,87 @@ __global__ __launch_bounds__(kNT) void sample_pick_kernel(SplitArgs a) {
     if (lane == kSplitG - 1) sh_over = over || incl > (uint32_t)kSplitCap;
   }
   __syncthreads();
-  if (whole || sh_over) {                             // (uniform over the workgroup)
+  if (whole) {                                        // (uniform over the workgroup)
     if (tid == 0) w.state = kRowWhole;
     sample_row<T>(r, (const T*)a.logits, a.V, a.temperature, a.top_k, a.top_p, a.uniform,
                   a.token, a.logprob, a.processed, a.status);
     return;
   }
-  const int n = (int)off[kSplitG];
+  const bool longer = sh_over;
+  if (longer) {
+    unsigned long long zk = 0;
+    if (mode == kModeTopP) {                          // the boundary bin, as in `gather`
+      unsigned long long mine = 0;
 #pragma unroll
-  for (int u = 0; u < kSlots; ++u) {
-    const int c = u * (kNT / kWave) + tid / kWave;
-    if (sel[u] >> lane & 1) {
-      const uint32_t at = off[c] + __popcll(sel[u] & (((uint64_t)1 << lane) - 1));
-      skey[at] = lk[u];
-      sidx[at] = li[u];
+      for (int q = 0; q < kPer; ++q) mine += h[q];
+      const unsigned long long run = block_scan<unsigned long long, kNT>(mine, part, zk);
+      split_boundary<kNT, kPer>(h, run, mine, split_goal(pp, zk), &sh_bin, &sh_above);
+      __syncthreads();
+      bin = sh_bin;
     }
-  }
-  __syncthreads();
-  uint32_t key = 0, idx = 0;
-  unsigned long long m = 0;
-  if (tid < n) {
-    key = skey[tid];
-    idx = sidx[tid];
-    m = mass_fix(key_float(key), M);
-    sw[tid] = m;
-  }
-  __syncthreads();
-  // rank by counting: elements above mine, their mass, ties and those after me
-  uint32_t higher = 0, ties = 0, after = 0;
-  unsigned long long above = 0;
-  if ((tid & ~(kWave - 1)) < n) {
-    for (int j = 0; j < n; ++j) {
-      const uint32_t kj = skey[j];
-      const unsigned long long mj = sw[j];
-      if (kj > key) {
-        ++higher;
-        above += mj;
-      }
-      if (kj == key) {
-        ++ties;
-        after += j > tid;
+    const unsigned long long low = split_descend<T>(
+        (const T*)a.logits + r * a.V, a.V, chunk, Tm, M, lmax, mode, (unsigned long long)kk, pp,
+        bin, sh_above, zk, part, cm);
+    if (tid == 0) sh_low = low;
+  } else {
+    const int n = (int)off[kSplitG];
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+      const int c = u * (kNT / kWave) + tid / kWave;
+      if (sel[u] >> lane & 1) {
+        const uint32_t at = off[c] + __popcll(sel[u] & (((uint64_t)1 << lane) - 1));
+        skey[at] = lk[u];
+        sidx[at] = li[u];
       }
     }
-  }
-  bool keep = tid < n && (mode != kModeTopK || (int64_t)higher < kk);
-  if (mode == kModeTopK && keep) atomicAdd(&sh_zk, m);
-  __syncthreads();
-  if (pp < 1.0f && mode != kModeAll) {
-    const unsigned long long zk = mode == kModeTopK ? sh_zk : w.zk;
-    if (mode == kModeTopP) above += w.above;
-    const unsigned long long target =
-        max(1ull, (unsigned long long)(fmax((double)pp, 0.0) * (double)zk));
-    // a group of equal values is kept while the mass above it is below the
-    // target; of the last one, as many as reach it, from the highest index down
-    keep = keep && above < target;
-    if (keep && m > 0) {
-      const double need = ceil(((double)target - (double)above) / (double)m);
-      keep = (double)after < fmax(1.0, fmin(need, (double)ties));
+    __syncthreads();
+    uint32_t key = 0, idx = 0;
+    unsigned long long m = 0;
+    if (tid < n) {
+      key = skey[tid];
+      idx = sidx[tid];
+      m = mass_fix(key_float(key), M);
+      sw[tid] = m;
     }
+    __syncthreads();
+    // rank by counting: elements above mine, their mass, ties and those after me
+    uint32_t higher = 0, ties = 0, after = 0;
+    unsigned long long above = 0;
+    if ((tid & ~(kWave - 1)) < n) {
+      for (int j = 0; j < n; ++j) {
+        const uint32_t kj = skey[j];
+        const unsigned long long mj = sw[j];
+        if (kj > key) {
+          ++higher;
+          above += mj;
+        }
+        if (kj == key) {
+          ++ties;
+          after += j > tid;
+        }
+      }
+    }
+    bool keep = tid < n && (mode != kModeTopK || (int64_t)higher < kk);
+    if (mode == kModeTopK && keep) atomicAdd(&sh_zk, m);
+    __syncthreads();
+    if (pp < 1.0f && mode != kModeAll) {
+      const unsigned long long zk = mode == kModeTopK ? sh_zk : w.zk;
+      if (mode == kModeTopP) above += w.above;
+      const unsigned long long target = split_goal(pp, zk);
+      // a group of equal values is kept while the mass above it is below the
+      // target; of the last one, as many as reach it, from the highest index down
+      keep = keep && above < target;
+      if (keep && m > 0) {
+        const double need = ceil(((double)target - (double)above) / (double)m);
+        keep = (double)after < fmax(1.0, fmin(need, (double)ties));
+      }
+    }
+    if (keep) {
+      atomicAdd(&cm[idx / (uint32_t)chunk], m);
+      atomicMin(&sh_low, ((unsigned long long)key << 32) | idx);
+    }
+    if (tid < n) sw[tid] = keep ? m : 0;
   }
-  if (keep) {
-    atomicAdd(&cm[idx / (uint32_t)chunk], m);
-    atomicMin(&sh_low, ((unsigned long long)key << 32) | idx);
-  }
-  if (tid < n) sw[tid] = keep ? m : 0;
   __syncthreads();
   const uint32_t pkey = mode == kModeAll ? 0u : (uint32_t)(sh_low >> 32);
   const uint32_t tie0 = mode == kModeAll ? 0u : (uint32_t)sh_low;
@@ -1101,7 +1299,7 @@ __global__ __launch_bounds__(kNT) void sample_pick_kernel(SplitArgs a) {
     a.logprob[r] = (x - M) - logf((float)((double)sh_z / kFix));
     a.status[r] = 0;
   };
-  if (mode == kModeTopK) {                            // inside the chunk's list
+  if (mode == kModeTopK && !longer) {                 // inside the chunk's list
     if (tid >= kWave) return;
     const int j = (int)off[c] + lane;
     const unsigned long long mj = j < (int)off[c + 1] ? sw[j] : 0;

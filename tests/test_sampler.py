@@ -232,6 +232,60 @@ def test_split_rows_equal_one_workgroup_rows(dtype, V):
         assert torch.equal(tok2, tok) and torch.equal(lp2.view(torch.int32), lp.view(torch.int32))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [16384, 16640 + 9, 151936])
+def test_split_rows_with_long_boundaries_equal_one_workgroup_rows(dtype, V):
+    """Rows whose boundary holds more elements than the split form's lists (64 per
+    chunk, 1024 per row), against the one-workgroup form as above: the kept set and
+    its values bit for bit, the draw by the 64-bit distribution. Rows: logits of
+    high magnitude (in bf16 one value is a tie group of more than 1024), flat ones,
+    a spread within one bin, around 0 with both signs, two values, all equal but
+    one, and ties only in the first and the last chunk. Options: top-p alone, high
+    and low, a large top-k alone and with top-p, both at a T that widens or narrows
+    the bins."""
+    from acorninfer_amd._lib import check, dtype_code, lib, ptr, stream_ptr
+    from acorninfer_amd.sampler import sample_batch
+    g = torch.Generator().manual_seed(V + 1)
+    x = torch.randn(8, V, generator=g)
+    x[0] = x[0] * 2 + 8
+    x[1] *= 0.1
+    x[2] = 3 + x[2] * 1e-3
+    x[3] *= 1e-5
+    x[4] = torch.randint(0, 2, (V,), generator=g).float()
+    x[5] = -4.0
+    x[5, V // 3] = -1.0
+    x[6] = -5 + 0.01 * x[6]
+    x[6, :70] = 6.0
+    x[6, V - 75:] = 6.0
+    options = [(1.0, 0, 0.9), (0.3, 0, 0.5), (1.7, 0, 0.999), (1.0, 5000, 1.0), (0.8, 5000, 0.8),
+               (1.3, V - 1, 0.3), (1.0, 100, 0.95), (1.0, 120, 0.4), (1.0, 0, 1e-6)]
+    rows = x.repeat_interleave(len(options), 0).to(dtype).cuda()
+    opts = options * x.shape[0]
+    B = rows.shape[0]
+    t = torch.tensor([o[0] for o in opts], device="cuda")
+    k = torch.tensor([o[1] for o in opts], dtype=torch.int32, device="cuda")
+    p = torch.tensor([o[2] for o in opts], device="cuda")
+    u = torch.rand(B, generator=g).cuda()
+    got_p, want_p = (torch.full((B, V), 7.0, device="cuda") for _ in range(2))
+    tok, lp, st = sample_batch(rows, t, k, p, u, processed=got_p)
+    wtok, wlp, wst = torch.empty_like(tok), torch.empty_like(lp), torch.empty_like(st)
+    check(lib().acorn_sample(ptr(rows), B, V, dtype_code(rows), ptr(t), ptr(k), ptr(p), ptr(u),
+                             ptr(wtok), ptr(wlp), ptr(want_p), ptr(wst), stream_ptr()), "sample")
+    assert int(st.sum()) == 0 and int(wst.sum()) == 0
+    assert torch.equal(got_p, want_p)
+    # the drawn token's interval of the distribution holds the uniform (bounds as above)
+    prob = torch.softmax(want_p.double(), 1)
+    cum = prob.cumsum(1).gather(1, tok[:, None])[:, 0]
+    lo = cum - prob.gather(1, tok[:, None])[:, 0]
+    assert (prob.gather(1, tok[:, None]) > 0).all()
+    assert ((lo - 4e-6 <= u) & (u <= cum + 4e-6)).all()
+    same = tok == wtok
+    torch.testing.assert_close(lp[same], wlp[same], rtol=1e-5, atol=1e-5)
+    tok2, lp2, _ = sample_batch(rows, t, k, p, u)
+    assert torch.equal(tok2, tok) and torch.equal(lp2, lp)
+
+
 def test_split_rows_are_those_whose_masses_add_up_in_64_bits():
     """The split form's sums (no GPU): a row of V equal logits has mass V x 2^40,
     which passes 2^64 from 2^24 elements; longer rows have no workspace and run
