@@ -516,6 +516,16 @@ constexpr int kSplitCapC = 64;       // listed elements per chunk (one wave)
 constexpr int kSplitCap = kNT;       // listed elements per row (one per thread of `pick`)
 // shorter rows: one workgroup reads them in less than four launches take
 constexpr int64_t kSplitMinV = 16384;
+// More rows: the stats of several chunks per workgroup, so that they stay one round
+// of workgroups (two per CU), and chunks of `hist` and `gather` on 256 threads, whose
+// dispatch is a quarter of the time (rows with nothing left to do, the greedy ones,
+// cost no more than that). us at 64 rows of 151936, 1024 threads and a chunk each /
+// this, one workgroup per row: greedy 36 / 15.6, 11.0; T 1 68 / 39, 170; top-p 0.9
+// 160 / 114, 555; top-k 20 + top-p 93 / 57, 579. At 8 rows greedy takes 11.5, 10.7 on
+// one workgroup; 64 greedy rows of 16384 14.4, 7.9 there, sampled 26 to 67, 30 to 138.
+constexpr int64_t kSplitWGs = 512;
+constexpr int64_t kSplitWideRows = 8;
+constexpr int kSplitFewNT = 256;
 constexpr int64_t kSplitMaxRows = 4096;  // bounds the workspace (34 KB per row)
 // masses of at most 2^40 each add up in 64 bits
 constexpr int64_t kSplitMaxV = (int64_t)1 << 23;
@@ -676,21 +686,24 @@ __device__ __forceinline__ V block_scan(V v, V* part, V& total) {
   return before + incl - v;
 }
 
-template <typename T>
-__global__ __launch_bounds__(kSplitNT) void sample_stats_kernel(SplitArgs a) {
+// `span` chunks per workgroup (U == 1: one): their maximum stands at the first.
+template <typename T, int U>
+__global__ __launch_bounds__(kSplitNT) void sample_stats_kernel(SplitArgs a, int span_) {
   __shared__ float red_f[kSplitNT / kWave];
   __shared__ int64_t red_i[kSplitNT / kWave];
   __shared__ int red_b[kSplitNT / kWave];
-  const int64_t r = blockIdx.x / kSplitG;
-  const int c = blockIdx.x % kSplitG, tid = threadIdx.x;
+  const int span = U == 1 ? 1 : span_, per = kSplitG / span;
+  const int64_t r = blockIdx.x / per;
+  const int c = blockIdx.x % per * span, tid = threadIdx.x;
   SplitRow& w = a.ws[r];
   constexpr int kShare = kSplitNB / kSplitG;
-  if (tid < kShare) w.hist[c * kShare + tid] = 0;
-  const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
+  for (int q = tid; q < span * kShare; q += kSplitNT) w.hist[c * kShare + q] = 0;
+  const int64_t c0 = min(c * split_chunk(a.V), a.V);
+  const int64_t c1 = min(c0 + span * split_chunk(a.V), a.V);
   float bv;
   int64_t bi;
   bool bad;
-  scan_max<T, kSplitNT, 1>((const T*)a.logits + r * a.V + c0, c1 - c0, bv, bi, bad);
+  scan_max<T, kSplitNT, U>((const T*)a.logits + r * a.V + c0, c1 - c0, bv, bi, bad);
   if (bi != INT64_MAX) bi += c0;
   wave_first_max(bv, bi);
   bad = __any(bad);
@@ -711,14 +724,19 @@ __global__ __launch_bounds__(kSplitNT) void sample_stats_kernel(SplitArgs a) {
     w.cmax[c] = bv;
     w.cimax[c] = bi == INT64_MAX ? 0xffffffffu : (uint32_t)bi;
     w.cbad[c] = bad;
+    for (int q = 1; q < span; ++q) {
+      w.cmax[c + q] = -INFINITY;
+      w.cimax[c + q] = 0xffffffffu;
+      w.cbad[c + q] = 0;
+    }
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void sample_hist_kernel(SplitArgs a) {
   __shared__ unsigned long long lhist[kSplitNB];
-  __shared__ unsigned long long part[kSplitNT / kWave];
-  __shared__ uint32_t upart[kSplitNT / kWave];
+  __shared__ unsigned long long part[NT / kWave];
+  __shared__ uint32_t upart[NT / kWave];
   __shared__ int sh_bin;
   const int64_t r = blockIdx.x / kSplitG;
   const int c = blockIdx.x % kSplitG, tid = threadIdx.x;
@@ -729,7 +747,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
   const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
   Octets<T> o(row, a.V, c0, c1);
   // consecutive elements per thread: thread order is vocabulary order
-  const int64_t seg = (o.n + kSplitNT - 1) / kSplitNT, end = min((tid + 1) * seg, o.n);
+  const int64_t seg = (o.n + NT - 1) / NT, end = min((tid + 1) * seg, o.n);
   o.load(tid * seg, 1);                  // in flight with the chunk maxima
   float lmax;
   int64_t imax;
@@ -751,7 +769,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
     return;
   }
   const int mode = split_mode(a, r);
-  for (int b = tid; b < kSplitNB; b += kSplitNT) lhist[b] = 0;
+  for (int b = tid; b < kSplitNB; b += NT) lhist[b] = 0;
   __syncthreads();
   unsigned long long sum = 0;
   o.each(tid * seg, 1, end, [&](int64_t, float l) {
@@ -765,14 +783,14 @@ __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
   });
   if (mode == kModeAll) {
     unsigned long long total;
-    block_scan<unsigned long long, kSplitNT>(sum, part, total);
+    block_scan<unsigned long long, NT>(sum, part, total);
     if (tid == 0) w.hard[c] = total;
     return;
   }
   __syncthreads();
-  constexpr int kPer = kSplitNB / kSplitNT;
+  constexpr int kPer = kSplitNB / NT;
   if (mode == kModeTopP) {
-    for (int q = tid; q < kSplitNB; q += kSplitNT)
+    for (int q = tid; q < kSplitNB; q += NT)
       if (lhist[q]) atomicAdd(&w.hist[q], lhist[q]);
     return;
   }
@@ -780,7 +798,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
   // row's first k: neither those bins nor those elements are passed on
   unsigned long long mine = 0, total;
   for (int q = 0; q < kPer; ++q) mine += lhist[tid * kPer + q];
-  unsigned long long run = block_scan<unsigned long long, kSplitNT>(mine, part, total);
+  unsigned long long run = block_scan<unsigned long long, NT>(mine, part, total);
   const unsigned long long kk = (unsigned long long)a.top_k[r];
   if (tid == 0 && total < kk) sh_bin = kSplitNB - 1;
   for (int q = 0; q < kPer; ++q) {
@@ -796,7 +814,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_hist_kernel(SplitArgs a) {
   uint32_t mine_n = 0, listed;
   if (seg > 1) o.load(tid * seg, 1);
   o.each(tid * seg, 1, end, [&](int64_t, float l) { mine_n += split_bin(l / Tm, M) <= bin; });
-  uint32_t pos = block_scan<uint32_t, kSplitNT>(mine_n, upart, listed);
+  uint32_t pos = block_scan<uint32_t, NT>(mine_n, upart, listed);
   if (mine_n && pos < (uint32_t)kSplitCapC) {
     if (seg > 1) o.load(tid * seg, 1);
     o.each(tid * seg, 1, end, [&](int64_t i, float l) {
@@ -1023,10 +1041,10 @@ __device__ unsigned long long split_descend(const T* row, int64_t V, int64_t chu
   return (unsigned long long)key << 32 | sh_tie0;
 }
 
-template <typename T>
-__global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
-  __shared__ unsigned long long part[kSplitNT / kWave];
-  __shared__ uint32_t upart[kSplitNT / kWave];
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void sample_gather_kernel(SplitArgs a) {
+  __shared__ unsigned long long part[NT / kWave];
+  __shared__ uint32_t upart[NT / kWave];
   __shared__ int sh_bin;
   __shared__ unsigned long long sh_above;
   const int64_t r = blockIdx.x / kSplitG;
@@ -1041,9 +1059,9 @@ __global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
   const T* row = (const T*)a.logits + r * a.V;
   const int64_t c0 = min(c * split_chunk(a.V), a.V), c1 = min(c0 + split_chunk(a.V), a.V);
   Octets<T> o(row, a.V, c0, c1);
-  const int64_t seg = (o.n + kSplitNT - 1) / kSplitNT;
+  const int64_t seg = (o.n + NT - 1) / NT;
   o.load(tid * seg, 1);
-  constexpr int kPer = kSplitNB / kSplitNT;
+  constexpr int kPer = kSplitNB / NT;
   unsigned long long h[kPer], mine = 0, total;
 #pragma unroll
   for (int q = 0; q < kPer; ++q) h[q] = w.hist[tid * kPer + q];
@@ -1057,10 +1075,10 @@ __global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
 
 #pragma unroll
   for (int q = 0; q < kPer; ++q) mine += h[q];
-  const unsigned long long run = block_scan<unsigned long long, kSplitNT>(mine, part, total);
+  const unsigned long long run = block_scan<unsigned long long, NT>(mine, part, total);
   const unsigned long long goal =
       mode == kModeTopK ? (unsigned long long)a.top_k[r] : split_goal(a.top_p[r], total);
-  split_boundary<kSplitNT, kPer>(h, run, mine, goal, &sh_bin, &sh_above);
+  split_boundary<NT, kPer>(h, run, mine, goal, &sh_bin, &sh_above);
   __syncthreads();
   const int bin = sh_bin;
 
@@ -1075,7 +1093,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
     else if (b < bin)
       hard += mass_fix(x, M);
   });
-  uint32_t pos = block_scan<uint32_t, kSplitNT>(mine_n, upart, listed);
+  uint32_t pos = block_scan<uint32_t, NT>(mine_n, upart, listed);
   if (mine_n && pos < (uint32_t)kSplitCapC) {    // (few threads: the chunk is read again)
     o.load(tid * seg, 1);
     o.each(tid * seg, 1, end, [&](int64_t i, float l) {
@@ -1091,7 +1109,7 @@ __global__ __launch_bounds__(kSplitNT) void sample_gather_kernel(SplitArgs a) {
     });
   }
   unsigned long long hsum;
-  block_scan<unsigned long long, kSplitNT>(hard, part, hsum);
+  block_scan<unsigned long long, NT>(hard, part, hsum);
   if (tid == 0) {
     w.hard[c] = hsum;
     w.ccnt[c] = listed;
@@ -1374,12 +1392,26 @@ __global__ __launch_bounds__(kNT) void sample_kernel(
                 processed, status);
 }
 
+template <typename T, int NT>
+void launch_split_chunks(const SplitArgs& a, int64_t rows, hipStream_t st) {
+  const dim3 grid((unsigned)(rows * kSplitG));
+  sample_hist_kernel<T, NT><<<grid, NT, 0, st>>>(a);
+  sample_gather_kernel<T, NT><<<grid, NT, 0, st>>>(a);
+}
 template <typename T>
 void launch_split(const SplitArgs& a, int64_t rows, hipStream_t st) {
   const dim3 grid((unsigned)(rows * kSplitG));
-  sample_stats_kernel<T><<<grid, kSplitNT, 0, st>>>(a);
-  sample_hist_kernel<T><<<grid, kSplitNT, 0, st>>>(a);
-  sample_gather_kernel<T><<<grid, kSplitNT, 0, st>>>(a);
+  int span = 1;
+  while (span < kSplitG && rows * kSplitG / span > kSplitWGs) span *= 2;
+  const dim3 stats((unsigned)(rows * (kSplitG / span)));
+  if (span == 1)
+    sample_stats_kernel<T, 1><<<stats, kSplitNT, 0, st>>>(a, span);
+  else
+    sample_stats_kernel<T, 4><<<stats, kSplitNT, 0, st>>>(a, span);
+  if (rows <= kSplitWideRows)
+    launch_split_chunks<T, kSplitNT>(a, rows, st);
+  else
+    launch_split_chunks<T, kSplitFewNT>(a, rows, st);
   sample_pick_kernel<T><<<(unsigned)rows, kNT, 0, st>>>(a);
   if (a.processed) sample_processed_kernel<T><<<grid, kSplitNT, 0, st>>>(a);
 }

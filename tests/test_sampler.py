@@ -286,6 +286,39 @@ def test_split_rows_with_long_boundaries_equal_one_workgroup_rows(dtype, V):
     assert torch.equal(tok2, tok) and torch.equal(lp2, lp)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [16384, 20003])
+@pytest.mark.parametrize("B", [9, 16, 17, 40, 130, 600])
+def test_split_forms_of_few_and_of_many_rows_agree(B, V):
+    """Batches past 8 rows run their chunks on smaller workgroups and, past 16, the
+    maxima of 2 to 32 chunks on one: every row's token, logprob and processed row are
+    those it has in a batch of 8, bit for bit. Every option, a greedy and a
+    non-finite row among them."""
+    from acorninfer_amd.sampler import sample_batch
+    g = torch.Generator().manual_seed(B)
+    x = torch.randn(B, V, generator=g) * 3
+    x[::5] *= 0.1
+    x[3, V // 2] = float("inf")
+    x[6, V - 1] = 40.0
+    rows = x.bfloat16().cuda()
+    options = [(0.7, 20, 0.95), (1.0, 0, 0.9), (0.6, 50, 1.0), (1.0, 0, 1.0), (0.9, 5000, 0.8),
+               (0.0, 0, 1.0), (1.0, 1, 1.0)]
+    opts = [options[i % len(options)] for i in range(B)]
+    t = torch.tensor([o[0] for o in opts], device="cuda")
+    k = torch.tensor([o[1] for o in opts], dtype=torch.int32, device="cuda")
+    p = torch.tensor([o[2] for o in opts], device="cuda")
+    u = torch.rand(B, generator=g).cuda()
+
+    def run(s):
+        proc = torch.full((s.stop - s.start, V), 7.0, device="cuda")
+        return (*sample_batch(rows[s], t[s], k[s], p[s], u[s], processed=proc), proc)
+    whole = run(slice(0, B))
+    for a in range(0, B, 8):
+        s = slice(a, min(a + 8, B))
+        for got, want in zip(whole, run(s)):
+            assert torch.equal(got[s].nan_to_num(99.0), want.nan_to_num(99.0)), s
+
+
 def test_split_rows_are_those_whose_masses_add_up_in_64_bits():
     """The split form's sums (no GPU): a row of V equal logits has mass V x 2^40,
     which passes 2^64 from 2^24 elements; longer rows have no workspace and run
