@@ -1808,11 +1808,23 @@ PrefillPlan prefill_plan(int64_t N, int64_t R, int64_t max_nq, int64_t H, int64_
   const int64_t S = std::min(std::min((target + base / 2) / base, (chunks + min_run - 1) / min_run),
                              kPrefillMaxRuns);
   if (S <= 1) return p;
-  p.cps = (int)((chunks + S - 1) / S);
-  p.S = (int)((chunks + p.cps - 1) / p.cps);
+  const int64_t cps = (chunks + S - 1) / S, runs = (chunks + cps - 1) / cps;
+  // ... and only where that is faster: rounds of resident workgroups times their
+  // chunks, after and before, in chunks' time (1.8 us), of which the merge launch
+  // takes 3 and 10 MB of partials, written and read, one. Of 1706 launches swept
+  // (1..8 sequences of 5..1150 rows over 0..8000 tokens, four head counts), 251 were
+  // slower split than not without this (5 x 520 rows over 1500, 16 / 8 heads, 94 us
+  // against 77; 3 x 800 over 700, 32 / 8, 64 against 44), 19 with it.
+  const int64_t slots = rep >= 8 ? kCUs : 2 * kCUs;    // eight-wave workgroups: one per CU
+  const int64_t before = chunks * ((base + slots - 1) / slots);
+  const int64_t after = cps * ((runs * base + slots - 1) / slots) + 3 +
+                        runs * prefill_slots(N, R, max_nq) * H * (D + 2) * 8 / 10000000;
+  if (runs <= 1 || after > before) return p;
+  p.cps = (int)cps;
+  p.S = (int)runs;
   // (S tiles KV stays below 4 / 3 of the target and a tile has at most 256 rows
   // of heads, so the partials take at most 1024 x 256 x (D + 2) floats, 136 MB)
-  if (p.S > 1) p.ws_bytes = p.S * prefill_slots(N, R, max_nq) * H * (D + 2) * 4;
+  p.ws_bytes = p.S * prefill_slots(N, R, max_nq) * H * (D + 2) * 4;
   return p;
 }
 
