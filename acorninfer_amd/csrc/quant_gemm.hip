@@ -980,8 +980,10 @@ bool dense8_choice(int64_t M, int64_t N, int64_t K, int* ks, int* first) {
 // slices. us at 8 rows, splitting K to 768 waves / this rule (8B): int4 qkv
 // 7.9 / 6.1, o 8.5 / 5.3, gate|up 13.2 / 13.0, down 11.1 / 10.2; int8 9.1 / 7.1,
 // 9.3 / 5.8, 19.5 / 19.1, 13.5 / 12.1; bf16 11.8 / 11.2, 9.9 / 7.5, 33.8 / 32.4,
-// 21.1 / 18.3. (int4 and int8 down at 16 rows are 6-10% slower than split, and
-// gain more than that back as the folded norm.)
+// 21.1 / 18.3. (int8 down at 16 rows is 15% slower than split, and gains more than
+// that back as the folded norm.) Not for int4 weights of 8 MB and more past 8 rows:
+// a step of eight 8B layers at 16 rows takes 733 us with one split and 700 with the
+// kernel's own, whose many waves keep more of the cold weights in flight.
 // Above, int4 up to 24 rows stages x once (11.0 against 11.6 us for qkv); the
 // rest runs on the mid-M kernels with 256-row workgroups and as many splits as
 // stay within one round of the CUs: int4 at 64 rows, tiled / mid-M, 21 / 15, 20
@@ -996,6 +998,7 @@ bool default_request(int64_t M, int64_t N, int64_t K, int wfmt, bool swiglu, int
     const int rt = nt >= 384 && nt % 2 == 0 ? 2 : 1;
     if (swiglu && rt != 2) return false;
     if (wfmt == ACORN_WFMT_W4B) {
+      if (M > 8 && N * K >= ((int64_t)16 << 20)) return false;
       const int kw = many ? 2 : 4;
       const int64_t st = K / 128 / (2 * kw);          // stages of two groups per slice
       const int depth = M <= 8 && rt == 1 && st % 4 == 0 ? 4 : st % 2 == 0 ? 2 : 1;

@@ -13,6 +13,7 @@ use it.
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -84,14 +85,19 @@ def prefill_supported(dtype: torch.dtype, head_dim: int, page_size: int, num_hea
             and num_heads % kv_heads == 0 and num_heads // kv_heads in (1, 2, 4, 8))
 
 
+@functools.lru_cache(maxsize=1024)
+def _prefill_workspace_bytes(*sizes: int) -> int:
+    n = ctypes.c_int64(0)
+    check(lib().acorn_paged_prefill_workspace(*sizes, ctypes.byref(n)), "paged_prefill_workspace")
+    return n.value
+
+
 def prefill_workspace(N: int, R: int, max_nq: int, H: int, KV: int, D: int, P: int,
                       table_width: int, device) -> torch.Tensor | None:
     """The workspace a prefill launch of these sizes splits its keys over, or
     None where it does not."""
-    n = ctypes.c_int64(0)
-    check(lib().acorn_paged_prefill_workspace(N, R, max_nq, H, KV, D, P, table_width,
-                                              ctypes.byref(n)), "paged_prefill_workspace")
-    return torch.empty(n.value, dtype=torch.uint8, device=device) if n.value else None
+    n = _prefill_workspace_bytes(N, R, max_nq, H, KV, D, P, table_width)
+    return torch.empty(n, dtype=torch.uint8, device=device) if n else None
 
 
 def paged_prefill_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor,
@@ -121,7 +127,8 @@ def paged_prefill_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: tor
     q2 = q.contiguous()
     if out is None:
         out = torch.empty_like(q2)
-    _check_out(out, (R, H, D), q)
+    else:
+        _check_out(out, (R, H, D), q)
     W = max(1, tables.shape[1])
     ws = prefill_workspace(N, R, int(max_nq), H, KV, D, P, W, q.device)
     rc = lib().acorn_paged_prefill_attention_ws(

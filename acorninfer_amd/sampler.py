@@ -17,6 +17,7 @@ graph-capturable batched form for the decode step: it never synchronises.
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass
 
 import torch
@@ -31,12 +32,18 @@ class SamplingParams:
     top_k: int = 0  # 0 = disabled
 
 
+@functools.lru_cache(maxsize=256)
+def _sample_workspace_bytes(rows: int, vocab: int) -> int:
+    n = ctypes.c_int64(0)
+    check(lib().acorn_sample_workspace(rows, vocab, ctypes.byref(n)), "sample_workspace")
+    return n.value
+
+
 def sample_workspace(rows: int, vocab: int, device) -> torch.Tensor | None:
     """The workspace acorn_sample_split takes for (rows, vocab), or None where
     it uses none."""
-    n = ctypes.c_int64(0)
-    check(lib().acorn_sample_workspace(rows, vocab, ctypes.byref(n)), "sample_workspace")
-    return torch.empty(n.value, dtype=torch.uint8, device=device) if n.value else None
+    n = _sample_workspace_bytes(rows, vocab)
+    return torch.empty(n, dtype=torch.uint8, device=device) if n else None
 
 
 def sample_batch(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
