@@ -1470,8 +1470,7 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
   // tile's first query (and past the last key) infinities and NaN become 0 once
   // they are staged, before the barrier; `odd` remembers per wave that there were
   // some, and the queries that see them add them at the end. Only a tile's last
-  // chunks hold such rows (8 windows of 5 rows over 1024..8192 keys: 38.0 us, 37.3
-  // without).
+  // chunks hold such rows (0.7 of 38 us for 8 windows of 5 rows over 1024..8192 keys).
   const int t_own = pos0 + wg_j0;                // the tile's first query
   __shared__ int odd[WIN ? NT / kWave : 1];
   if (WIN && lane == 0) odd[wid] = 0;
@@ -1526,17 +1525,32 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
   // due) and the scores go k-block by k-block over their 2 QW independent
   // sums, so no MFMA waits for the one before it: 8192 causal tokens, 32 / 8
   // heads, 718 -> 687 us; 8 windows of 5 rows over 1024..8192 keys 41.7 -> 39.4.
-  u32x4_t va[DPL], pb[QW];
+  // TWO: in bf16 windows P goes through the MFMAs as two terms, P cut to bf16 and the
+  // rest (never 0 where P is not: a visible infinity in V stays one), so that a
+  // row is no further from 64 bits than K3's, whose many splits hold their own
+  // largest P as exactly 1 (relative error, one sequence, 2 rows over 400 tokens:
+  // one term 0.0023, K3 0.0019, two terms 0.0016; 8 windows of 5 rows over
+  // 1024..8192 keys 38.4 -> 40.8 us).
+  constexpr bool TWO = WIN && std::is_same<T, __bf16>::value;
+  u32x4_t va[DPL], pb[QW], pr[TWO ? QW : 1];
 #pragma unroll
   for (int jj = 0; jj < DPL; ++jj) va[jj] = u32x4_t{0u, 0u, 0u, 0u};
 #pragma unroll
   for (int qw = 0; qw < QW; ++qw) pb[qw] = u32x4_t{0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int qw = 0; qw < (TWO ? QW : 1); ++qw) pr[qw] = u32x4_t{0u, 0u, 0u, 0u};
   const int tlast = pos0 + j0 + min(16 * QW, nvalid) - 1;   // the wave's last query
   auto pv = [&]() {
 #pragma unroll
     for (int jj = 0; jj < DPL; ++jj)
 #pragma unroll
       for (int qw = 0; qw < QW; ++qw) acc[qw][jj] = mfma16x16x32<T>(va[jj], pb[qw], acc[qw][jj]);
+    if constexpr (TWO) {
+#pragma unroll
+      for (int jj = 0; jj < DPL; ++jj)
+#pragma unroll
+        for (int qw = 0; qw < QW; ++qw) acc[qw][jj] = mfma16x16x32<T>(va[jj], pr[qw], acc[qw][jj]);
+    }
   };
   auto step = [&](int b, int sub, int t0) {
     // keys after every query, as all that follow: the step due stays due, and
@@ -1572,6 +1586,7 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
       // P V MFMAs run unconditionally
       if (!live[qw]) {
         pb[qw] = u32x4_t{0u, 0u, 0u, 0u};
+        if (TWO) pr[qw] = u32x4_t{0u, 0u, 0u, 0u};
         continue;
       }
       float sv[8];                               // raw scores; scaled inside the exp2
@@ -1590,11 +1605,9 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
 #pragma unroll
       for (int i = 1; i < 8; ++i) mx = fmaxf(mx, sv[i]);
       mx *= scale_log2;                          // scale_log2 > 0: the max of the scaled scores
-      // (windows follow the maximum at once: the P of the largest score is then 1,
-      // which T holds exactly, as in each of K3's splits. With the slack a window's
-      // rows were up to 16% further from 64 bits than K3's, now nearer, but for two
-      // rows over at most 72 tokens (1.05 x); 8 windows of 5 rows 38.3 -> 39.3 us)
-      if (__builtin_amdgcn_ballot_w64(mx > m[qw] + (WIN ? 0.f : kMaxSlack)) != 0) {
+      // (fp16 windows follow the maximum at once: the P of the largest score is then
+      // 1, which fp16 holds exactly, as in each of K3's splits)
+      if (__builtin_amdgcn_ballot_w64(mx > m[qw] + (WIN && !TWO ? 0.f : kMaxSlack)) != 0) {
         mx = fmaxf(mx, __shfl_xor(mx, 16));
         mx = fmaxf(mx, __shfl_xor(mx, 32));
         const float mn = fmaxf(m[qw], mx);
@@ -1607,10 +1620,19 @@ __global__ __launch_bounds__(REP * QG * kWave, 2) void paged_prefill_kernel(
         for (int jj = 0; jj < DPL; ++jj) acc[qw][jj] *= alpha;
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        pb[qw][i] = pack_dot<T>(__builtin_amdgcn_exp2f(__builtin_fmaf(sv[2 * i], scale_log2, nm[qw])),
-                                __builtin_amdgcn_exp2f(__builtin_fmaf(sv[2 * i + 1], scale_log2, nm[qw])),
-                                l[qw]);
+      for (int i = 0; i < 4; ++i) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[2 * i], scale_log2, nm[qw]));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[2 * i + 1], scale_log2, nm[qw]));
+        if constexpr (TWO) {
+          const float h0 = __uint_as_float(__float_as_uint(p0) & 0xffff0000u);
+          const float h1 = __uint_as_float(__float_as_uint(p1) & 0xffff0000u);
+          pb[qw][i] = __float_as_uint(p0) >> 16 | __float_as_uint(h1);
+          pr[qw][i] = pack_bf16x2(fmaxf(p0 - h0, p0 * 0x1p-30f), fmaxf(p1 - h1, p1 * 0x1p-30f));
+          l[qw] += p0 + p1;
+        } else {
+          pb[qw][i] = pack_dot<T>(p0, p1, l[qw]);
+        }
+      }
     }
     typedef __attribute__((address_space(3))) s16x4_t lds_s16x4;
     const __attribute__((address_space(3))) uint8_t* vl =

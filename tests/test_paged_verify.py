@@ -218,14 +218,14 @@ def test_rows_do_not_see_later_v_whatever_it_holds(H, KV, D, m, hist, dtype):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H,hist", [(32, 40), (32, 130), (16, 400), (32, 1600)])
-def test_window_rows_are_as_near_to_float64_as_decode_rows(H, hist, dtype):
+def test_window_rows_are_as_near_to_float64_as_decode_rows(H, hist, dtype, B=8):
     """Eight windows of five rows against attention in float64, and the same rows
     through K3 with its own split rule: rounding P to the activation dtype costs a
-    window no more (both sides hold some 10^5 outputs, so that the two error norms
-    are known to within a percent)."""
+    window no more (both sides hold 2 x 10^4 outputs and more, so that the two error
+    norms are known to within a percent)."""
     from acorninfer_amd.ops.paged_attention import paged_decode_attention, plan_splits
     from acorninfer_amd.ops.paged_verify import paged_verify_attention
-    B, m, KV, D = 8, 5, 8, 128
+    m, KV, D = 5, 8, 128
     q, kp, vp, tables, lens = _gpu(*_inputs(B, m, hist, dtype, H=H, KV=KV, D=D, seed=hist))
     exact = torch.empty(B, m, H, D, dtype=torch.float64, device="cuda")
     for b in range(B):
@@ -240,12 +240,18 @@ def test_window_rows_are_as_near_to_float64_as_decode_rows(H, hist, dtype):
     k3 = paged_decode_attention(
         q.reshape(B * m, H, D), kp, vp, tables.repeat_interleave(m, 0),
         (lens[:, None] - back).reshape(-1).contiguous(),
-        plan_splits(B * m, KV, tables.shape[1])).view(B, m, H, D)
+        plan_splits(B, KV, tables.shape[1])).view(B, m, H, D)
     out = paged_verify_attention(q, kp, vp, tables, lens, 4)
 
     def err(x):
         return float((x.double() - exact).norm() / exact.norm())
     assert err(out) <= err(k3) * 1.01
+
+
+def test_one_short_window_is_as_near_to_float64_as_decode_rows():
+    """The same where K3 splits its keys by the page (few sequences), which is where
+    its rows are nearest: each split holds its largest P exactly."""
+    test_window_rows_are_as_near_to_float64_as_decode_rows(32, 400, torch.bfloat16, B=1)
 
 
 def test_scatter_verify_bit_exact_and_lengths():
