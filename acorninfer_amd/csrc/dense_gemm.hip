@@ -28,7 +28,7 @@
 // follow, both operands in LDS and two waves per SIMD: one stages through
 // registers (1.0-1.06 PFLOP/s at M = 2048-8192), the other loads straight
 // into LDS (global_load_lds) in whole 128-byte rows through two pair-of-stage
-// buffers, the planner's default from 512 rows (1.11-1.33 PFLOP/s at
+// buffers, the planner's default from 256 rows (1.11-1.33 PFLOP/s at
 // M = 8192; hipBLASLt: 1.3-1.5).
 #include <hip/hip_runtime.h>
 

@@ -1347,10 +1347,11 @@ __device__ __forceinline__ int64_t prefill_slot(int64_t N, int64_t R, int64_t ma
 //    (the scores of the two 16-key halves are its B operand as they lie;
 //    16x16x16 runs at half the rate on gfx950; the V^T operand comes from
 //    LDS through ds_read_b64_tr_b16, no register transposes); blocks whose
-//    queries all precede the keys skip the scores and add P = 0; keys past a
-//    query's position are masked where a chunk crosses the diagonal, and the
-//    first chunk holds key 0, so every column's max is finite from the
-//    start; rows past the last key re-read it (finite, masked);
+//    queries all precede the keys add P = 0, and a step past the wave's last
+//    query is left out; keys past a query's position are masked where a chunk
+//    crosses the diagonal; rows past the last key re-read it (masked). Without
+//    SPLIT and WIN the first chunk holds key 0, so every column's max is finite
+//    from there on;
 //  * the longest query tiles (the last ones) are dispatched first.
 // A workgroup reads its keys once for REP x QG x 32 query rows: O(L^2 / 32)
 // K / V bytes per prompt of L tokens and kv head, against O(L^2) for one
@@ -1359,7 +1360,7 @@ __device__ __forceinline__ int64_t prefill_slot(int64_t N, int64_t R, int64_t ma
 // Few query rows over long contexts (a late chunk of a chunked prefill, a
 // follow-up turn, a verify window) give tiles x KV x N workgroups that leave
 // CUs idle while each walks its whole prefix alone: three sequences of 40..300
-// rows over 2000..8000 tokens took 155 us. With SPLIT the keys of a tile are
+// rows over 2000..8000 tokens took 155 us (58.6 now). With SPLIT the keys of a tile are
 // divided into runs of `cps` chunks, one workgroup each; a tile of more than
 // one run leaves (acc, m, l) per run in fp32 for paged_prefill_combine_kernel,
 // and a run in which a query sees no key adds nothing (m stays -inf).
@@ -1811,10 +1812,9 @@ struct PrefillPlan {
 // run costs its rows' fp32 partials, written and read: small next to a window's
 // keys, about five chunks' time for a full tile, so runs keep kWindowMinRun
 // chunks, kPrefillMinRun, or kPrefillBusyRun once half the CUs have a tile.
-// Measured, one split / this rule (us): 8 windows of 5 rows over 1024..8192
-// tokens 162 / 48, 3 prompts' 40..300 rows over 2000..8000 tokens 153 / 64,
-// 100 rows over 8000 219 / 48, 512 over 8000 232 / 112, 1000 over 8000
-// 250 / 197; 1000 rows with no prefix 39.5 unsplit, 43.7 in two runs.
+// Measured, one split / this rule (us), 32 / 8 heads: 5 rows over 8000 tokens
+// 157 / 27, 64 rows 213 / 39, 150 rows 216 / 63, 520 rows 227 / 150, 800 rows
+// 236 / 193.
 constexpr int64_t kWindowMinRun = 4, kPrefillMinRun = 6, kPrefillBusyRun = 16;
 constexpr int64_t kPrefillMaxRuns = 64;
 PrefillPlan prefill_plan(int64_t N, int64_t R, int64_t max_nq, int64_t H, int64_t KV, int64_t D,

@@ -486,7 +486,7 @@ __device__ void sample_row(
 //
 // One workgroup per row leaves all but `rows` CUs idle and walks the row about
 // ten times, an IEEE division and often an LDS atomic per element each time:
-// 444 us for 8 rows of 151936 (2.4 MB) at T 0.6, top-k 20, top-p 0.95. Here a
+// 464 us for 8 rows of 151936 (2.4 MB) at T 0.6, top-k 20, top-p 0.95. Here a
 // row is kSplitG chunks of consecutive elements and each launch reads a chunk
 // once:
 //   stats   chunk maxima and finiteness; clears the row's histogram
@@ -507,7 +507,7 @@ __device__ void sample_row(
 // of x, so bins respect the key order. The draw adds integer masses instead of
 // fp32 ones. Where the boundary holds more elements than the lists (a large top-k,
 // many ties, a flat row) pick goes down the keys instead (split_descend).
-// Four launches of a few microseconds each, bound by their latency.
+// Four launches of a few microseconds each, bound by their latency: 27.3 us.
 constexpr int kSplitG = 32;          // workgroups (chunks) per row
 constexpr int kSplitNT = 1024;       // their threads
 constexpr int kSplitNB = 2048;       // histogram bins: 32 in x, the last takes the rest

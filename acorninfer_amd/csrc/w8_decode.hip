@@ -325,8 +325,8 @@ int by_upw(const DirectPlan& p, const W8dArgs& a, hipStream_t st) {
   return ACORN_ERR_UNSUPPORTED;
 }
 
-// The natural-layout form: one row tile (few row tiles) or two per wave, two
-// blocks per stage, four stages in flight where K allows, four K slices.
+// The natural-layout form: one row tile (few row tiles) and eight K slices, or two
+// row tiles and four; two blocks per stage, four stages in flight where K allows.
 template <int RT, int DEPTH, int KW>
 int launch_nat(const DirectPlan& p, const W8dArgs& a, hipStream_t st) {
   const dim3 grid((unsigned)p.groups), block(KW * kWave);

@@ -10,9 +10,10 @@ the pages (`PagedKVCache.scatter_verify`).
 A window is a short prefill whose prefix is in the cache: it runs on the
 query-tiled prefill kernel (`acorn_paged_prefill_attention_ws`), which reads a
 sequence's K/V once for the whole window and divides a long context over
-several workgroups. As one K3 row per window token, the form below, eight
-windows of five over 1024..8192 tokens took 110 us, each row reading the
-context for itself; shapes the prefill kernel is not built for (fp32, head
+several workgroups. Rows stay independent as in K3: what a later token's V
+holds, infinities and NaN included, reaches no earlier row. Eight windows of
+five over 1024..8192 tokens take 41 us; as one K3 row per window token, the form
+below, 109, each row reading the context for itself. Shapes the prefill kernel is not built for (fp32, head
 sizes other than 64 / 128, pages under 16 tokens) and one-token windows, which
 are decode, keep it: the window is flattened to B*m query rows and the
 split/combine kernels of decode run over them.

@@ -85,8 +85,8 @@ class Tiling(NamedTuple):
     above), ksplit, and tpw = stages in flight per wave.
     int8 decode kernel (WFMT_W8B, M <= 16): rt row tiles per wave, upw 64-k
     blocks per stage, nw the wave layout (1, 4, 22, 44), ksplit,
-    tpw = stages in flight; above 16 rows W8B runs on the tiled kernel or the
-    int8 mid-M kernel.
+    tpw = stages in flight; above 16 rows W8B runs on the tiled, the int8 mid-M
+    or, from 256 rows, the large-M kernel.
     bf16 decode kernel (WFMT_BF16B, M <= 16): rt row tiles per wave, upw
     32-k blocks per stage, nw the wave layout (1, 4, 22, 44), ksplit, tpw =
     stages in flight; above 16 rows BF16B runs on the tiled kernel and from

@@ -283,7 +283,12 @@ int acorn_paged_attention_qkv_supported(int64_t H, int64_t KV, int64_t D, int64_
  *                         model's bf16 weights)
  *   wfmt ACORN_WFMT_F32 : w fp32 [N,K], x fp32 [M,K]; fp32 result in part
  * cfg: NULL or int[6] {rt, upw, nw, ksplit, tpw, -}; 0 entries are chosen by
- * the planner (acorn_gemm_plan). With the chosen ksplit:
+ * the planner (acorn_gemm_plan; a requested ksplit of 1 is one split). rt also
+ * names a kernel: -2 the large-M one (bf16; W8B, where upw 256, nw 128 and tpw is
+ * the number of 256-row tiles of x it takes, the rows past them, in one split,
+ * running on the mid-M kernel), -3 the mid-M one (W4B, W8B), -5 the direct one on
+ * natural W8 rows (M <= 16). x, w and scale may lie at any address, but for the
+ * bf16 large-M kernel, whose x and w are 16-byte aligned. With the chosen ksplit:
  *   out_bf16 != NULL, ksplit == 1: writes bf16 [M,N];
  *   out_bf16 != NULL, ksplit > 1 : part is an fp32 workspace [ksplit,M,N]; a
  *       second launch sums the partials in split order into out_bf16
@@ -354,7 +359,7 @@ int acorn_gemm_swiglu_plan(int64_t M, int64_t N, int64_t K, int wfmt, int* cfg);
  * dequantisation the reference's large-M quantised GEMM applies in-kernel
  * before its bf16 dot (acorninfer/ops/quant_gemm.py:175-183: int -> fp32 x
  * scale -> bf16). With acorn_quant_gemm on ACORN_WFMT_BF16 it forms the
- * int4 GEMM at prefill sizes (from about 512 rows), where the bf16 MFMA kernel
+ * int4 GEMM at prefill sizes (from about 700 rows), where the bf16 MFMA kernel
  * outruns any in-kernel unpacking. N % 16 == 0, K % 512 == 0; out holds
  * N * K bf16 (the caller's workspace).
  */
