@@ -838,13 +838,19 @@ int make_tile_plan(int64_t M, int64_t N, int64_t K, int wfmt, int req_bm, int re
   // layer, 64-row tiles towards two workgroups per CU 34 / 25 / 70 / 40 us, this
   // rule 21 / 19 / 44 / 30; 160 rows 41 / 31 / 100 / 55 and 38 / 27 / 97 / 54.
   // The weights of a 0.6B layer at 17 and 64 rows are 5-20% faster in 64-row tiles.
+  // A split of 128-row x tiles keeps 256 k (2048 x 1024 at 255 rows, 8 splits 17.5
+  // us, 4 14.2), and a vocabulary's rows stay in 64-row tiles up to 48 rows (151936 x
+  // 4096 at 17 / 33 rows 252 / 272 us in 128-row tiles, 242 / 263).
   if ((wfmt == ACORN_WFMT_BF16 || wfmt == ACORN_WFMT_BF16B) && !req_bm && !req_bn && !req_ks &&
-      M > 16 && N % 128 == 0 && K % 64 == 0 && (M > 64 || N * K >= ((int64_t)8 << 20))) {
+      M > 16 && N % 128 == 0 && K % 64 == 0 && (M > 64 || N * K >= ((int64_t)8 << 20)) &&
+      (M > 48 || N / 128 <= 4 * kCUs)) {
     int64_t bm = M <= 32 ? 32 : M <= 128 ? 64 : 128;
     if (bm == 64 && N / 128 * ((M + 63) / 64) > kCUs) bm = 128;
     const int64_t tiles = N / 128 * ((M + bm - 1) / bm);
     int ks = 1;
-    while (tiles * ks * 2 <= kCUs && ks < 8 && K % (128 * ks) == 0) ks *= 2;
+    while (tiles * ks * 2 <= kCUs && ks < 8 && K % (128 * ks) == 0 &&
+           (bm < 128 || K >= 512 * (int64_t)ks))
+      ks *= 2;
     return make_tile_plan(M, N, K, wfmt, (int)bm, 128, ks, t);
   }
   const int bn = (req_bn == 64 || req_bn == 128) ? req_bn : M <= 64 ? 64 : 128;
