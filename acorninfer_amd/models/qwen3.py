@@ -59,10 +59,11 @@ DENSE_RT = -2
 # kernel's rate outweighs the extra pass over the weights: on MI355X eight
 # layers of a W4A16 8B prefill take, this way / on the int4 kernels, 3.61 /
 # 3.07 ms at 512 tokens, 4.27 / 3.93 at 640, 4.40 / 4.60 at 768 and 5.00 / 5.28
-# at 1024. Where there is no int4 form to prefer (weights of another row count
+# at 1024 (two layers at 690: 1.34 / 1.39; the mid-M kernel's tiles are 64 rows).
+# Where there is no int4 form to prefer (weights of another row count
 # than 128s above 64 rows, the fused SwiGLU above 16) it is taken from
 # DEQUANT_M_ODD rows.
-DEQUANT_M_MIN = 704
+DEQUANT_M_MIN = 641
 DEQUANT_M_ODD = 512
 DEQUANT_RT = -4
 # prefill blocks from this many rows run gate|up with the large-M kernel's
