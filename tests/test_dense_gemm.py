@@ -411,3 +411,20 @@ def test_w8b_large_m_operands_at_any_address(M, N, K, swiglu):
     for xs, ws in ((xo, w), (x, wo), (xo, wo)):
         for a, b in zip(outs(xs, ws), want):
             assert torch.equal(a, b)
+
+
+def test_default_tilings_where_one_split_or_eight_lose():
+    """Sizes at which the general default loses, measured (no GPU): large int4
+    weights past 8 rows keep several splits, small ones and fewer rows one; a bf16
+    split of 128-row x tiles keeps 256 k."""
+    from acorninfer_amd._lib import WFMT_BF16, WFMT_W4B
+    from acorninfer_amd.ops.quant_gemm import plan
+    for N, K in ((6144, 4096), (4096, 4096), (4096, 12288)):
+        assert plan(8, N, K, WFMT_W4B)[0].ksplit == 1
+        assert all(plan(M, N, K, WFMT_W4B)[0].ksplit > 1 for M in (9, 16))
+    assert plan(16, 4096, 1024, WFMT_W4B)[0].ksplit == 1
+    for N, K, M in ((2048, 1024, 255), (1024, 1024, 200), (4096, 2048, 160)):
+        t = plan(M, N, K, WFMT_BF16)[0]
+        assert t.upw == 128 and K // t.ksplit >= 256, t
+    assert plan(17, 151936, 4096, WFMT_BF16)[0].nw == 64
+    assert plan(64, 151936, 4096, WFMT_BF16)[0].nw == 128

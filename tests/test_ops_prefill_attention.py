@@ -295,3 +295,23 @@ def test_workspace_holds_rows_and_not_padding():
                 assert n.value <= 1024 * 256 * (D + 2) * 4
                 split += n.value > 0
     assert split > 40
+
+
+def test_keys_are_divided_only_where_the_launch_gets_faster():
+    """The planner's choice (no GPU) at sizes measured both ways: launches whose
+    runs would not fit one round of workgroups, or whose partials cost more than
+    they save, stay whole; long prefixes under few rows are divided."""
+    import ctypes
+    from acorninfer_amd._lib import check, lib
+    n = ctypes.c_int64(-1)
+
+    def split(N, R, max_nq, H, KV, width):
+        check(lib().acorn_paged_prefill_workspace(N, R, max_nq, H, KV, 128, 16, width,
+                                                  ctypes.byref(n)), "workspace")
+        return n.value > 0
+    for whole in ((5, 2635, 528, 16, 8, 115), (3, 3500, 1268, 16, 8, 177), (2, 1600, 800, 32, 8, 94),
+                  (3, 1560, 520, 32, 8, 77), (1, 1150, 1150, 32, 8, 116), (1, 8192, 8192, 32, 8, 512)):
+        assert not split(*whole), whole
+    for divided in ((1, 5, 5, 32, 8, 501), (1, 64, 64, 32, 8, 504), (1, 520, 520, 32, 8, 533),
+                    (8, 40, 5, 32, 8, 512), (3, 500, 300, 32, 8, 500)):
+        assert split(*divided), divided
